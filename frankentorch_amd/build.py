@@ -25,6 +25,7 @@ HIP_SOURCES = [
     "indexops.hip",
     "gemm.hip",
     "sdpa.hip",
+    "sdpa_decode.hip",
     "backward.hip",
     "sdpa_bwd.hip",
     "lossops.hip",

@@ -27,6 +27,10 @@ hipStream_t resolve_stream(fth_stream s);
 // Number of compute units of device 0 (cached).
 int compute_units();
 
+// Scratch memory of the stream: valid until the next call for the same stream, so for kernels launched on it right away (their
+// successors on the stream run after them). Kept and grown, never given back; safe with several threads and streams.
+int32_t stream_workspace(hipStream_t st, size_t bytes, void **ws);
+
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Softmax over contiguous rows too long or too ragged for the 128-bit row kernels (any length up to 65 536 floats /

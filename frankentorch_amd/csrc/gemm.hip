@@ -1637,6 +1637,7 @@ template <typename T> int32_t launch_trans_a(GemmArgs<T> &p, const fth_gemm_desc
 }  // namespace
 
 namespace fth {
+int32_t stream_workspace(hipStream_t st, size_t bytes, void **ws) { return get_workspace(st, bytes, ws, 0); }
 int64_t gemm_rowmax_groups(int64_t n) { return fth::ceil_div(n, 128) * 2; }
 bool gemm_f32_nt_rowmax(int64_t m, int64_t n, int64_t k, const float *a, const float *b, float *c, float *rowmax, hipStream_t st,
                         int32_t *rc) {

@@ -1,0 +1,18 @@
+// Few-query attention against a long K/V cache (csrc/sdpa_decode.hip), used by csrc/sdpa.hip.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "ft_kernel_hip.h"
+
+namespace fth {
+
+// True when the key-split kernel covers the problem: seq_q <= 8, no causal flag, d_k == d_v in {32, 64, 128}. Operands are
+// 16-byte aligned with strides that are multiples of four (the caller checks).
+bool sdpa_decode_applies(const fth_sdpa_desc &d);
+int32_t sdpa_decode_f32(const fth_sdpa_desc &d, float scale, const float *q, const float *k, const float *v, const float *mask,
+                        int64_t mask_bh_stride, float *out, hipStream_t st);
+
+}  // namespace fth

@@ -1,0 +1,51 @@
+"""Attention of a few new tokens against a K/V cache (the key-split kernel): edges of the 32-key tiles and of the shares, row
+counts around the 16- and 32-row tiles, grouped heads, masks of every alignment. Against the CPU checker, fp32 <= 2e-5."""
+import math
+
+import numpy as np
+import pytest
+
+from conftest import TOL_GEMM_F32, rel_err
+from frankentorch_amd import synth
+from frankentorch_amd.device import DeviceBuffer
+
+pytestmark = pytest.mark.gpu
+
+# (batch, h_q, h_kv, seq_q, seq_k, d)
+SHAPES = [(1, 1, 1, 1, 1, 64), (2, 4, 4, 1, 31, 32), (1, 8, 2, 4, 32, 64), (1, 8, 2, 4, 33, 128), (2, 17, 1, 1, 64, 32), (1, 8, 1, 4, 65, 64),
+          (1, 6, 2, 8, 130, 128), (1, 33, 1, 1, 97, 64), (3, 32, 8, 1, 397, 128), (1, 4, 1, 8, 1027, 64), (1, 8, 8, 2, 4099, 128), (1, 9, 1, 8, 200, 32)]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("mask_kind", ["none", "shared", "per_head"])
+def test_few_queries_against_a_cache(hip, oracle, shape, mask_kind):
+    batch, hq, hkv, sq, sk, d = shape
+    q, k, v = (synth.normal(51, t, s) for t, s in (("q", (batch, hq, sq, d)), ("k", (batch, hkv, sk, d)), ("v", (batch, hkv, sk, d))))
+    scale = np.float32(1.0 / math.sqrt(d))
+    mask = np.zeros((sq, sk), np.float32)
+    if mask_kind != "none":
+        mshape = (sq, sk) if mask_kind == "shared" else (batch * hq, sq, sk)
+        mask = synth.normal(51, "mask", mshape, 0.0, 0.5)
+        mask[synth.uniform(51, "hide", mshape) < 0.3] = -np.inf
+        mask[..., : sk // 2] = -np.inf  # whole shares without a visible key
+        mask[..., sk - 1] = 0.25
+        if sk > 40:
+            mask[..., 0, :] = -np.inf   # a row with nothing visible is NaN
+
+    def run(kk, vv, heads_kv):
+        bufs = [DeviceBuffer.from_host(t) for t in (q, kk, vv, mask)]
+        out = DeviceBuffer.from_host(np.full(q.shape, 7.0, np.float32))
+        desc = hip.sdpa_desc_gqa(batch, hq, heads_kv, sq, sk, d, d, False)
+        if mask_kind == "none":
+            hip.sdpa_forward(desc, scale, bufs[0], bufs[1], bufs[2], out)
+        else:
+            hip.sdpa_forward_masked(desc, scale, bufs[0], bufs[1], bufs[2], bufs[3], 0 if mask.ndim == 2 else sq * sk, out)
+        return out.to_host()
+
+    got, ref = run(k, v, hkv), oracle.sdpa_forward_masked_gqa(q, k, v, scale, mask)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    ok = ~np.isnan(ref)
+    if ok.any():
+        assert rel_err(got[ok], ref[ok]) <= TOL_GEMM_F32
+    expanded = run(np.repeat(k, hq // hkv, axis=1), np.repeat(v, hq // hkv, axis=1), hq)
+    assert np.array_equal(got.view(np.uint32), expanded.view(np.uint32))
