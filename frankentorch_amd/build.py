@@ -24,6 +24,7 @@ HIP_SOURCES = [
     "rowops.hip",
     "indexops.hip",
     "gemm.hip",
+    "gemm_split.hip",
     "sdpa.hip",
     "sdpa_decode.hip",
     "backward.hip",

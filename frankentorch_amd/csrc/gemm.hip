@@ -47,6 +47,7 @@
 
 #include "common.hpp"
 #include "devmath.hpp"
+#include "gemm_split.hpp"
 #include "pool.hpp"
 
 namespace {
@@ -1260,7 +1261,7 @@ struct StreamWorkspace {
     void *partials = nullptr;
     size_t partial_bytes = 0;
 };
-// slot 0: split-tile accumulators; slot 1: transposed copy of a [k, m] A operand.
+// slot 0: split-tile accumulators; slot 1: transposed copy of a [k, m] A operand; slot 2: planes of the split product.
 //
 // A block that a larger request outgrows is retired, never handed back to the shared pool: kernels
 // queued on the stream may still be using it, the pool serves every stream and thread (so "ordered
@@ -1553,6 +1554,19 @@ int32_t gemm_entry(const fth_gemm_desc *d, T alpha, const T *a, const T *b, T *c
         FTH_CHECK_LAUNCH("gemm_k0");
         return FTH_OK;
     }
+    if constexpr (std::is_same<T, float>::value) {
+        // Large single products: exact three-way bf16 split (gemm_split.hip). FT_HIP_GEMM_SPLIT=0 is a tuning knob.
+        static const bool split_off = [] {
+            const char *e = std::getenv("FT_HIP_GEMM_SPLIT");
+            return e && std::atoi(e) == 0;
+        }();
+        if (!split_off && d->batch == 1 && fth::split_gemm_pays(d->m, d->n, d->k)) {
+            fth::SplitGemm g{a, b, d->trans_a ? 1 : d->lda, d->trans_a ? d->lda : 1, d->trans_b ? d->ldb : 1, d->trans_b ? 1 : d->ldb,
+                             c, bias, residual, nullptr, d->m, d->n, d->k, d->ldc, alpha, d->epilogue};
+            int32_t rc = FTH_OK;
+            if (fth::split_gemm(g, st, &rc)) return rc;
+        }
+    }
     if (d->trans_a) return launch_trans_a<T>(p, d, st);
     constexpr int EPV = Mfma<T>::EPV;
     auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15u) == 0; };
@@ -1588,6 +1602,10 @@ bool launch_nt_rowmax(int64_t m, int64_t n, int64_t k, const float *a, const flo
     }();
     if (direct_off || m <= 0 || n <= 0 || k <= 0 || k % 32 != 0 || !al(a) || !al(b) || k > lim || n > lim || big_tiles < cus || forced_tile() > 0)
         return false;
+    if (fth::split_gemm_pays(m, n, k)) {
+        fth::SplitGemm g{a, b, k, 1, k, 1, c, nullptr, nullptr, rowmax, m, n, k, n, 1.f, 0};
+        if (fth::split_gemm(g, st, rc)) return true;
+    }
     GemmArgs<float> p;
     p.a = a; p.b = b; p.c = c; p.bias = nullptr; p.residual = nullptr;
     p.m = m; p.n = n; p.k = k;
@@ -1638,6 +1656,7 @@ template <typename T> int32_t launch_trans_a(GemmArgs<T> &p, const fth_gemm_desc
 
 namespace fth {
 int32_t stream_workspace(hipStream_t st, size_t bytes, void **ws) { return get_workspace(st, bytes, ws, 0); }
+int32_t stream_split_workspace(hipStream_t st, size_t bytes, void **ws) { return get_workspace(st, bytes, ws, 2); }
 int64_t gemm_rowmax_groups(int64_t n) { return fth::ceil_div(n, 128) * 2; }
 bool gemm_f32_nt_rowmax(int64_t m, int64_t n, int64_t k, const float *a, const float *b, float *c, float *rowmax, hipStream_t st,
                         int32_t *rc) {

@@ -1,0 +1,586 @@
+// fp32 matrix products on the bf16 matrix units.
+//
+// A float has 24 significant bits; three bf16 values hold 8 each. Rounding to nearest three times, x = x0 + x1 + x2 EXACTLY
+// (x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1, which has at most 8 significant bits left), so nothing of an operand
+// is given up. Of the nine products of two such sums six are formed, x0 y0, x0 y1, x1 y0, x1 y1, x0 y2, x2 y0, each exact in
+// the matrix unit and summed in fp32; the three left out are below 2^-24 |x y| together and of either sign (root mean square
+// 2^-26 |x y|). Six bf16 MFMAs of 32 k cost 96 cycles where the fp32 MFMAs cost 256. The sum is rounded 6 times per 32 k
+// instead of 8 times or more, which is why the result is closer to the exact one than the fp32 MFMA kernel's: relative
+// 2-norm error against 64-bit sums, normal operands, K 768 / 3072 / 4096: 4.2e-7 / 8.6e-7 / 1.00e-6 here, 4.95e-7 / 9.9e-7 /
+// 1.15e-6 there.
+//
+// Two passes. split_rows_kernel / split_cols_kernel write an operand's three planes once, in the order in which the product
+// reads them; the product then moves planes to LDS with direct loads and has no vector arithmetic in its loop. Splitting
+// inside the product was tried and costs more: vector instructions and MFMAs share issue cycles, every element would be
+// split again by each tile that reads it, and the loop stayed at 190-230 TFLOP/s (of fp32 products) where this one reaches
+// 240-263.
+//
+// What the split cannot represent is found in the results. An infinity, a NaN or a float that rounds up to a bf16 infinity
+// leaves a non-finite sum; magnitudes whose lowest bits fall below the bf16 subnormals (operands under 2^-109) can only
+// matter in a result under 2^-100. A wavefront that holds a non-finite sum or a non-zero one under 2^-100 computes its part
+// of the tile again from the fp32 operands on fp32 MFMAs.
+//
+// replaces gemm::sgemm / sgemm_bt / sgemm_tb (crates/ft-kernel-cpu/src/lib.rs:1310-1338, 1430-1524) for large products.
+
+#include <cfloat>
+#include <mutex>
+
+#include "common.hpp"
+#include "devmath.hpp"
+#include "gemm_split.hpp"
+
+namespace {
+
+constexpr int kWave = 64;
+constexpr int kXcds = 8;
+constexpr int kGroupM = 8;
+constexpr int kBK = 32;       // k of a K-tile: one 16 x 16 x 32 MFMA
+constexpr int kPlanes = 3;
+constexpr int kBlock = 1024;  // bytes of one plane of 16 rows x 32 k
+constexpr float kTiny = 0x1p-100f;
+
+using bf16x8 = __attribute__((ext_vector_type(8))) __bf16;
+using bf16x2 = __attribute__((ext_vector_type(2))) __bf16;
+using f32x2 = __attribute__((ext_vector_type(2))) float;
+using f32x4 = __attribute__((ext_vector_type(4))) float;
+using u32x4 = __attribute__((ext_vector_type(4))) uint32_t;
+typedef f32x4 f32x4_any __attribute__((aligned(4)));  // 128-bit access at any float
+
+__device__ __forceinline__ uint32_t pack_bf16(float x, float y) {
+    const f32x2 v = {x, y};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));  // v_cvt_pk_bf16_f32: to nearest even
+}
+__device__ __forceinline__ float lo_f32(uint32_t p) { return __builtin_bit_cast(float, p << 16); }
+__device__ __forceinline__ float hi_f32(uint32_t p) { return __builtin_bit_cast(float, p & 0xffff0000u); }
+
+// The three parts of two floats, one dword each.
+__device__ __forceinline__ void split2(float x, float y, uint32_t &p0, uint32_t &p1, uint32_t &p2) {
+    p0 = pack_bf16(x, y);
+    x -= lo_f32(p0);
+    y -= hi_f32(p0);
+    p1 = pack_bf16(x, y);
+    x -= lo_f32(p1);
+    y -= hi_f32(p1);
+    p2 = pack_bf16(x, y);
+}
+
+// Planes of an operand: [K-tile][plane][16-row block][16 rows][4 chunks of 8 k], a 16-byte chunk at slot chunk ^ swz(row) of
+// its row. The LDS holds the same image, and a wavefront's 128-bit operand read (16 rows at the same chunk, in the lane
+// groups the LDS serves together) touches every bank once: 0 conflict cycles by counter; chunk ^ (row / 4) has 2 a read.
+__device__ __forceinline__ int swz(int row) {
+    const int t = row >> 2;
+    return (((t ^ (t >> 1)) & 1) << 1) | ((t >> 1) & 1);
+}
+
+__device__ __forceinline__ void store_chunk(const float (&v)[8], unsigned char *planes, int64_t kt, int blocks, int64_t row, int chunk) {
+    u32x4 w[kPlanes];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        uint32_t p0, p1, p2;
+        split2(v[2 * e], v[2 * e + 1], p0, p1, p2);
+        w[0][e] = p0;
+        w[1][e] = p1;
+        w[2][e] = p2;
+    }
+#pragma unroll
+    for (int s = 0; s < kPlanes; ++s)
+        *reinterpret_cast<u32x4 *>(planes + (kt * kPlanes + s) * blocks * kBlock + row * 64 + ((chunk ^ swz((int)(row & 15))) << 4)) = w[s];
+}
+
+// Operand stored [rows][k]. A wavefront takes one 16-row block and one K-tile: whole 128-byte lines in, three whole 1 KB
+// blocks out. Rows and k beyond the operand are zero. Bound by memory (4 bytes in, 6 out per element).
+__global__ __launch_bounds__(256) void split_rows_kernel(const float *x, unsigned char *planes, int64_t rows, int64_t k, int64_t ld, int blocks,
+                                                         int ktiles) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t kt = (int64_t)blockIdx.x * 4 + wave;
+    if (kt >= ktiles) return;
+    const int64_t row = (int64_t)blockIdx.y * 16 + (lane >> 2);
+    const int chunk = lane & 3;
+    const int64_t k0 = kt * kBK + chunk * 8;
+    float v[8];
+    if (row < rows && k0 + 8 <= k) {
+        const float *src = x + row * ld + k0;
+        const f32x4 lo = *reinterpret_cast<const f32x4_any *>(src), hi = *reinterpret_cast<const f32x4_any *>(src + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] = lo[e];
+            v[4 + e] = hi[e];
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = row < rows && k0 + e < k ? x[row * ld + k0 + e] : 0.f;
+    }
+    store_chunk(v, planes, kt, blocks, row, chunk);
+}
+
+// Operand stored [k][rows]. A workgroup takes 64 rows and one K-tile, a wavefront one 8-k chunk of it: 256-byte runs in.
+__global__ __launch_bounds__(256) void split_cols_kernel(const float *x, unsigned char *planes, int64_t rows, int64_t k, int64_t ld, int blocks) {
+    const int lane = threadIdx.x & 63, chunk = threadIdx.x >> 6;
+    const int64_t kt = blockIdx.y, row = (int64_t)blockIdx.x * 64 + lane, k0 = kt * kBK + chunk * 8;
+    if (row >= (int64_t)blocks * 16) return;
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = row < rows && k0 + e < k ? x[(k0 + e) * ld + row] : 0.f;
+    store_chunk(v, planes, kt, blocks, row, chunk);
+}
+
+struct PlaneArgs {
+    fth::SplitGemm g;
+    const unsigned char *a, *b;
+    int a_blocks, b_blocks;  // 16-row blocks of the planes
+    int ktiles;              // of the whole product
+    int splits, kt_per;      // the K-tiles are cut into `splits` runs of kt_per (the last one shorter)
+    int tiles_m, tiles_n;
+    int64_t tiles;
+    float *partial;          // splits > 1: [splits][m][n] sums without epilogue
+    int order;               // tile order inside a group of tile rows, as in the fp32 kernel: 1 walks along the rows of C
+    int64_t rowmax_groups;
+};
+
+__device__ __forceinline__ void tile_of_id(int64_t id, int tiles_m, int tiles_n, int order, int &tm, int &tn) {
+    const int64_t group = (int64_t)kGroupM * tiles_n;
+    const int64_t g = id / group;
+    const int first_m = (int)(g * kGroupM);
+    const int gm = (tiles_m - first_m) < kGroupM ? (tiles_m - first_m) : kGroupM;
+    const int in_g = (int)(id - g * group);
+    tm = first_m + (order ? in_g / tiles_n : in_g % gm);
+    tn = order ? in_g % tiles_n : in_g / gm;
+}
+
+// Hardware workgroup id -> virtual id such that each XCD owns one contiguous run of virtual ids.
+__device__ __forceinline__ int xcd_contiguous_id(int pid, int grid) {
+    const int per = grid / kXcds, rem = grid % kXcds, xcd = pid % kXcds, q = pid / kXcds;
+    return q + xcd * per + (xcd < rem ? xcd : rem);
+}
+
+__device__ __forceinline__ const unsigned char *uniform_ptr(const unsigned char *ptr) {
+    const uint64_t v = reinterpret_cast<uint64_t>(ptr);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return reinterpret_cast<const unsigned char *>(((uint64_t)hi << 32) | lo);
+}
+
+// 1 KB from a uniform base plus per-lane offsets to LDS. In assembly so that the compiler does not wait for it at the next LDS
+// read; the kernel waits for vmcnt(0) itself before each barrier. Writes no register.
+__device__ __forceinline__ void load_to_lds_16(const unsigned char *base, unsigned lane_bytes, unsigned lds_chunk) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_bytes), "s"(base), "s"(lds_chunk) : "memory", "m0");
+}
+
+__device__ __forceinline__ float nan_max(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+__device__ __forceinline__ float gelu_tanh(float x) {
+    const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
+    return x / (1.0f + __builtin_amdgcn_exp2f(u * -2.8853900817779268f));
+}
+
+// Four k of one operand row for the fp32 MFMAs, zero beyond the operand's k.
+__device__ __forceinline__ f32x4 four_k(const float *row, int64_t ks, int64_t k0, int64_t k_end) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (ks == 1 && k0 + 4 <= k_end) return *reinterpret_cast<const f32x4_any *>(row + k0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (k0 + e < k_end) v[e] = row[(k0 + e) * ks];
+    return v;
+}
+
+// The product. WM x WN wavefronts share a BM x BN tile; a wavefront's operands of one K-tile are 3 (TM + TN) 128-bit LDS reads
+// for 6 TM TN MFMAs. Two LDS buffers of a K-tile's planes, one barrier a K-tile: behind it the loads of the K-tile after
+// next are issued into the buffer that was just read out, and the operands of the next K-tile are read while this one's
+// MFMAs run, plane by plane as a plane's last MFMA has been issued (x2 y0 and x0 y2 first, x0 y0 last; only plane 0 needs
+// two register sets). The operands are passed (B, A): a lane then holds four neighbouring columns of one row of C, stored
+// as one vector. Persistent: workgroups walk the tiles `grid` apart, loads run ahead across tile borders.
+// Bound by the matrix units and the power they draw: 4096^3 263 TFLOP/s of fp32 products, 1.58 PFLOP/s of bf16 ones
+// (fp32 MFMA kernel: 146).
+template <int BM, int BN, int WM, int WN, bool ROWMAX>
+__global__ __launch_bounds__(WM *WN *kWave, 2) void plane_gemm_kernel(const PlaneArgs p) {
+    constexpr int NW = WM * WN;
+    constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 16, TN = WTN / 16;
+    constexpr int BUF = kPlanes * (BM + BN) * 64;                          // bytes: A planes [3][BM][64], then B planes [3][BN][64]
+    constexpr int A_CH = kPlanes * BM / 16, B_CH = kPlanes * BN / 16;      // 1 KB blocks of a K-tile
+    constexpr int LA = (A_CH + NW - 1) / NW, LB = (B_CH + NW - 1) / NW;
+    static_assert(!ROWMAX || WTN == 64, "row maxima are kept per 64 columns");
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm0 = (wave / WN) * WTM, wn0 = (wave % WN) * WTN;
+    const int l16 = lane & 15, lq = lane >> 4;
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)reinterpret_cast<uintptr_t>(smem));
+    const int grid = (int)gridDim.x;
+    const int vb = xcd_contiguous_id((int)blockIdx.x, grid);
+    const int64_t items = p.tiles * p.splits;
+    if (vb >= items) return;
+
+    auto run_of = [&](int64_t item, int &first) __attribute__((always_inline)) {
+        const int s = (int)(item / p.tiles);
+        first = s * p.kt_per;
+        const int rest = p.ktiles - first;
+        return rest < p.kt_per ? rest : p.kt_per;
+    };
+    // ---- loader: one K-tile ahead of the operand reads ----
+    int64_t ld_item = vb;
+    int ld_left = 0;  // K-tiles of ld_item still to request
+    const unsigned char *ak = nullptr, *bk = nullptr;
+    unsigned a_off[LA], b_off[LB];
+    const int64_t a_step = (int64_t)p.a_blocks * kPlanes * kBlock, b_step = (int64_t)p.b_blocks * kPlanes * kBlock;
+    auto setup = [&]() __attribute__((always_inline)) {
+        int tm, tn, first;
+        ld_left = __builtin_amdgcn_readfirstlane(run_of(ld_item, first));
+        tile_of_id(ld_item % p.tiles, p.tiles_m, p.tiles_n, p.order, tm, tn);
+        ak = uniform_ptr(p.a + first * a_step);
+        bk = uniform_ptr(p.b + first * b_step);
+#pragma unroll
+        for (int i = 0; i < LA; ++i) {
+            const int c = i * NW + wave;
+            int blk = tm * (BM / 16) + c % (BM / 16);
+            blk = blk < p.a_blocks ? blk : p.a_blocks - 1;
+            a_off[i] = (unsigned)(c / (BM / 16) * p.a_blocks + blk) * (unsigned)kBlock + lane * 16u;
+        }
+#pragma unroll
+        for (int i = 0; i < LB; ++i) {
+            const int c = i * NW + wave;
+            int blk = tn * (BN / 16) + c % (BN / 16);
+            blk = blk < p.b_blocks ? blk : p.b_blocks - 1;
+            b_off[i] = (unsigned)(c / (BN / 16) * p.b_blocks + blk) * (unsigned)kBlock + lane * 16u;
+        }
+    };
+    const unsigned wdst = lds0 + (unsigned)wave * kBlock;
+    auto issue = [&](int buf) __attribute__((always_inline)) {
+        if (ld_left == 0) return;  // past the last K-tile of this workgroup
+#pragma unroll
+        for (int i = 0; i < LA; ++i)
+            if (A_CH % NW == 0 || i + 1 < LA || i * NW + wave < A_CH) load_to_lds_16(ak, a_off[i], wdst + buf * BUF + i * NW * kBlock);
+#pragma unroll
+        for (int i = 0; i < LB; ++i)
+            if (B_CH % NW == 0 || i + 1 < LB || i * NW + wave < B_CH) load_to_lds_16(bk, b_off[i], wdst + buf * BUF + (A_CH + i * NW) * kBlock);
+        ak += a_step;
+        bk += b_step;
+        if (--ld_left == 0) {
+            ld_item += grid;
+            if (ld_item < items) setup();
+        }
+    };
+
+    struct Frag { bf16x8 a[TM], b[TN]; };
+    const int a_rd = (wm0 + l16) * 64 + ((lq ^ swz(l16)) << 4), b_rd = A_CH * kBlock + (wn0 + l16) * 64 + ((lq ^ swz(l16)) << 4);
+    auto fetch = [&](Frag &f, int buf, int s) __attribute__((always_inline)) {
+        const unsigned char *s0 = smem + buf * BUF;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) f.a[i] = *reinterpret_cast<const bf16x8 *>(s0 + s * BM * 64 + a_rd + i * kBlock);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) f.b[j] = *reinterpret_cast<const bf16x8 *>(s0 + s * BN * 64 + b_rd + j * kBlock);
+    };
+    f32x4 acc[TM][TN];
+    auto mul = [&](const Frag &fa, const Frag &fb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb.b[j], fa.a[i], acc[i][j], 0, 0, 0);
+    };
+    auto zero = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    };
+
+    // This wavefront's part of a tile again, from the fp32 operands.
+    auto again = [&](int64_t m0, int64_t n0, int first, int nk) __attribute__((always_inline)) {
+        zero();
+        const fth::SplitGemm &g = p.g;
+        const int64_t k_end = (int64_t)(first + nk) * kBK < g.k ? (int64_t)(first + nk) * kBK : g.k;
+        for (int64_t k0 = (int64_t)first * kBK; k0 < k_end; k0 += 16) {
+            f32x4 av[TM];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                int64_t row = m0 + i * 16 + l16;
+                row = row < g.m ? row : g.m - 1;
+                av[i] = four_k(g.a + row * g.a_rs, g.a_ks, k0 + lq * 4, k_end);
+            }
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                int64_t col = n0 + j * 16 + l16;
+                col = col < g.n ? col : g.n - 1;
+                const f32x4 bv = four_k(g.b + col * g.b_rs, g.b_ks, k0 + lq * 4, k_end);
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[e], av[i][e], acc[i][j], 0, 0, 0);
+            }
+        }
+    };
+
+    auto finish = [&](int64_t item, int first, int nk) __attribute__((always_inline)) {
+        int tm, tn;
+        tile_of_id(item % p.tiles, p.tiles_m, p.tiles_n, p.order, tm, tn);
+        const int64_t m0 = (int64_t)tm * BM + wm0, n0 = (int64_t)tn * BN + wn0;
+        float big = 0.f, small = FLT_MAX;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    big = nan_max(big, __builtin_fabsf(acc[i][j][e]));
+                    small = __builtin_fminf(small, __builtin_fabsf(acc[i][j][e]));
+                }
+        if (__builtin_amdgcn_ballot_w64(!(big <= FLT_MAX) || small < kTiny)) {  // rare: look closer (an exact zero is nothing to worry about)
+            bool doubt = !(big <= FLT_MAX);
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) doubt = doubt || (acc[i][j][e] != 0.f && __builtin_fabsf(acc[i][j][e]) < kTiny);
+            if (__builtin_amdgcn_ballot_w64(doubt)) again(m0, n0, first, nk);
+        }
+        const int64_t m = p.g.m, n = p.g.n;
+        const bool parts = p.splits > 1;
+        float *c = parts ? p.partial + (item / p.tiles) * m * n : p.g.c;
+        const int64_t ldc = parts ? n : p.g.ldc;
+        if (!parts) {
+            if (p.g.alpha != 1.f) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) acc[i][j] *= p.g.alpha;
+            }
+            if (p.g.epilogue & FTH_EPI_BIAS) {
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int64_t col = n0 + j * 16 + lq * 4 + e;
+                        const float b = col < n ? p.g.bias[col] : 0.f;
+#pragma unroll
+                        for (int i = 0; i < TM; ++i) acc[i][j][e] += b;
+                    }
+            }
+            if (p.g.epilogue & FTH_EPI_GELU) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc[i][j][e] = fth::gelu_erf(acc[i][j][e]);
+            } else if (p.g.epilogue & FTH_EPI_GELU_TANH) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc[i][j][e] = gelu_tanh(acc[i][j][e]);
+            }
+        }
+        const float *res = !parts && (p.g.epilogue & FTH_EPI_RESIDUAL) ? p.g.residual : nullptr;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const int64_t row = m0 + i * 16 + l16;
+            float top = -__builtin_inff();
+            if (row < m) {
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    const int64_t col = n0 + j * 16 + lq * 4;
+                    float *dst = c + row * ldc + col;
+                    if (col + 4 <= n) {
+                        if (res) acc[i][j] += *reinterpret_cast<const f32x4_any *>(res + row * ldc + col);
+                        *reinterpret_cast<f32x4_any *>(dst) = acc[i][j];
+                        if constexpr (ROWMAX)
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) top = nan_max(top, acc[i][j][e]);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            if (col + e < n) {
+                                const float v = res ? acc[i][j][e] + res[row * ldc + col + e] : acc[i][j][e];
+                                dst[e] = v;
+                                if constexpr (ROWMAX) top = nan_max(top, v);
+                            }
+                    }
+                }
+            }
+            if constexpr (ROWMAX) {
+                top = nan_max(top, __shfl_xor(top, 16));
+                top = nan_max(top, __shfl_xor(top, 32));
+                const int64_t group = n0 / 64;
+                if (lq == 0 && row < m && group < p.rowmax_groups) p.g.rowmax[group * m + row] = top;
+            }
+        }
+    };
+
+    Frag f0, f1, g1, g2;
+    int64_t item = vb;
+    int first = 0, nk = __builtin_amdgcn_readfirstlane(run_of(item, first)), kt = 0;
+    zero();
+    setup();
+    issue(0);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): own part landed
+    __syncthreads();
+    issue(1);
+    fetch(f0, 0, 0);
+    fetch(g1, 0, 1);
+    fetch(g2, 0, 2);
+    // One K-tile; false when it was the last one. The next K-tile's own loads have landed behind the wait, everyone's behind the
+    // barrier, and everyone has this K-tile's operands in registers. After the last K-tile the reads fetch what is left there.
+    auto step = [&](int buf, const Frag &cur, Frag &nxt) __attribute__((always_inline)) {
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+        __syncthreads();
+        issue(buf);
+        mul(cur, g2);
+        mul(g2, cur);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(g2, buf ^ 1, 2);
+        fetch(nxt, buf ^ 1, 0);
+        mul(g1, g1);
+        mul(g1, cur);
+        mul(cur, g1);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(g1, buf ^ 1, 1);
+        mul(cur, cur);
+        __builtin_amdgcn_sched_barrier(0);
+        if (++kt < nk) return true;
+        finish(item, first, nk);
+        item += grid;
+        if (item >= items) return false;
+        nk = __builtin_amdgcn_readfirstlane(run_of(item, first));
+        kt = 0;
+        zero();
+        fetch(nxt, buf ^ 1, 0);  // again: nothing of the next tile is held in registers across the output
+        fetch(g1, buf ^ 1, 1);
+        fetch(g2, buf ^ 1, 2);
+        return true;
+    };
+    while (step(0, f0, f1) && step(1, f1, f0)) {
+    }
+}
+
+// Sum of the split runs in K order, then the epilogue.
+__global__ __launch_bounds__(256) void plane_reduce_kernel(const PlaneArgs p) {
+    const int64_t n = p.g.n, total = p.g.m * n;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= total) return;
+    float v = p.partial[i];
+    for (int s = 1; s < p.splits; ++s) v += p.partial[s * total + i];
+    const int64_t row = i / n, col = i - row * n;
+    if (p.g.alpha != 1.f) v *= p.g.alpha;
+    if (p.g.epilogue & FTH_EPI_BIAS) v += p.g.bias[col];
+    if (p.g.epilogue & FTH_EPI_GELU) v = fth::gelu_erf(v);
+    if (p.g.epilogue & FTH_EPI_GELU_TANH) v = gelu_tanh(v);
+    if (p.g.epilogue & FTH_EPI_RESIDUAL) v += p.g.residual[row * p.g.ldc + col];
+    p.g.c[row * p.g.ldc + col] = v;
+}
+
+// ---- which tile, how many runs of K ----
+
+struct Tile { int bm, bn, per_cu; double rate; };  // rate: TFLOP/s of fp32 products with every workgroup busy
+constexpr Tile kTiles[] = {{128, 256, 1, 250.}, {128, 192, 1, 238.}, {64, 128, 2, 200.}};
+
+struct Choice { int tile = -1, splits = 1, kt_per = 0; double us = 0; };
+
+// Time of the product alone: rounds of tiles over the compute units, and for split K the partial sums' way through memory
+// (written and read at 4 TB/s, 4 us for the second launch).
+Choice choose(int64_t m, int64_t n, int64_t k, bool rowmax) {
+    const int cus = fth::compute_units() > 0 ? fth::compute_units() : 256;
+    const int64_t ktiles = fth::ceil_div(k, kBK);
+    Choice best;
+    for (int t = 0; t < (rowmax ? 1 : 3); ++t) {
+        const Tile &c = kTiles[t];
+        const int64_t tiles = fth::ceil_div(m, c.bm) * fth::ceil_div(n, c.bn);
+        for (int s = 1; s <= (rowmax ? 1 : 16); ++s) {
+            const int64_t per = fth::ceil_div(ktiles, s);
+            if (s > 1 && (per < 8 || (int64_t)(s - 1) * per >= ktiles)) break;
+            const int64_t rounds = fth::ceil_div(tiles * s, (int64_t)cus * c.per_cu);
+            double us = rounds * (2.0 * c.bm * c.bn * kBK * per * c.per_cu * cus / c.rate * 1e-6 + 3.0) + 2.0;
+            if (s > 1) us += (s + 1.0) * m * n * 4 / 4e6 + 4.0;
+            if (best.tile < 0 || us < best.us) best = {t, s, (int)per, us};
+        }
+    }
+    return best;
+}
+
+size_t plane_bytes(int64_t rows, int64_t k) { return (size_t)(fth::ceil_div(k, kBK) * kPlanes * fth::ceil_div(rows, 16)) * kBlock; }
+
+constexpr size_t kScratchBound = (size_t)1 << 30;  // planes and partial sums of one product
+
+template <int BM, int BN, int WM, int WN, bool ROWMAX> int32_t launch_planes(PlaneArgs &p, int per_cu, hipStream_t st) {
+    constexpr int smem = 2 * kPlanes * (BM + BN) * 64;
+    auto kern = plane_gemm_kernel<BM, BN, WM, WN, ROWMAX>;
+    static const hipError_t ready = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    FTH_HIP(ready);
+    p.tiles_m = (int)fth::ceil_div(p.g.m, BM);
+    p.tiles_n = (int)fth::ceil_div(p.g.n, BN);
+    p.tiles = (int64_t)p.tiles_m * p.tiles_n;
+    p.order = p.tiles_n > p.tiles_m ? 1 : 0;
+    const int64_t slots = (int64_t)(fth::compute_units() > 0 ? fth::compute_units() : 256) * per_cu, items = p.tiles * p.splits;
+    kern<<<dim3((unsigned)(items < slots ? items : slots)), dim3(WM * WN * kWave), smem, st>>>(p);
+    FTH_CHECK_LAUNCH("gemm_planes");
+    return FTH_OK;
+}
+
+int32_t launch_split(const float *x, unsigned char *planes, int64_t rows, int64_t k, int64_t rs, int64_t ks, hipStream_t st) {
+    const int blocks = (int)fth::ceil_div(rows, 16), ktiles = (int)fth::ceil_div(k, kBK);
+    if (ks == 1)
+        split_rows_kernel<<<dim3((unsigned)fth::ceil_div(ktiles, 4), (unsigned)blocks), dim3(256), 0, st>>>(x, planes, rows, k, rs, blocks, ktiles);
+    else
+        split_cols_kernel<<<dim3((unsigned)fth::ceil_div(blocks, 4), (unsigned)ktiles), dim3(256), 0, st>>>(x, planes, rows, k, ks, blocks);
+    FTH_CHECK_LAUNCH("gemm_split");
+    return FTH_OK;
+}
+
+int32_t run_split(const fth::SplitGemm &g, const Choice &ch, unsigned char *scratch, hipStream_t st) {
+    PlaneArgs p{};
+    p.g = g;
+    p.ktiles = (int)fth::ceil_div(g.k, kBK);
+    p.a_blocks = (int)fth::ceil_div(g.m, 16);
+    p.b_blocks = (int)fth::ceil_div(g.n, 16);
+    p.splits = ch.splits;
+    p.kt_per = ch.kt_per;
+    p.rowmax_groups = fth::gemm_rowmax_groups(g.n);
+    unsigned char *pa = scratch, *pb = pa + plane_bytes(g.m, g.k);
+    p.a = pa;
+    p.b = pb;
+    p.partial = reinterpret_cast<float *>(pb + plane_bytes(g.n, g.k));
+    if (int32_t rc = launch_split(g.a, pa, g.m, g.k, g.a_rs, g.a_ks, st)) return rc;
+    if (int32_t rc = launch_split(g.b, pb, g.n, g.k, g.b_rs, g.b_ks, st)) return rc;
+    int32_t rc = FTH_OK;
+    switch (ch.tile) {
+        case 0:
+            rc = g.rowmax ? launch_planes<128, 256, 2, 4, true>(p, kTiles[0].per_cu, st) : launch_planes<128, 256, 2, 4, false>(p, kTiles[0].per_cu, st);
+            break;
+        case 1: rc = launch_planes<128, 192, 2, 4, false>(p, kTiles[1].per_cu, st); break;
+        default: rc = launch_planes<64, 128, 2, 2, false>(p, kTiles[2].per_cu, st); break;
+    }
+    if (rc || ch.splits == 1) return rc;
+    plane_reduce_kernel<<<dim3((unsigned)fth::ceil_div(g.m * g.n, 256)), dim3(256), 0, st>>>(p);
+    FTH_CHECK_LAUNCH("gemm_planes_reduce");
+    return FTH_OK;
+}
+
+size_t scratch_bytes(int64_t m, int64_t n, int64_t k, const Choice &ch) {
+    return plane_bytes(m, k) + plane_bytes(n, k) + (ch.splits > 1 ? (size_t)ch.splits * m * n * sizeof(float) : 0);
+}
+
+}  // namespace
+
+namespace fth {
+
+bool split_gemm_pays(int64_t m, int64_t n, int64_t k) {
+    if (m < 64 || n < 64 || k < 128 || m > (1 << 20) || n > (1 << 20) || k > (1 << 20) || m * n > ((int64_t)1 << 31)) return false;
+    const Choice ch = choose(m, n, k, false);
+    if (scratch_bytes(m, n, k, ch) > kScratchBound) return false;
+    // The planes: 10 bytes an element at 3.5 TB/s and two launches; the fp32 kernel: 130 TFLOP/s.
+    const double us = ch.us + 10.0 * k * (m + n) / 3.5e6 + 5.0;
+    return us < 0.95 * 2.0 * m * n * k / 130e6;
+}
+
+bool split_gemm(const SplitGemm &g, hipStream_t st, int32_t *rc) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return false;
+    const Choice ch = choose(g.m, g.n, g.k, g.rowmax != nullptr);
+    // The scratch belongs to the stream; the lock keeps another thread's product on the same stream from being queued between
+    // the planes and their reader.
+    static std::mutex *mu = new std::mutex();
+    std::lock_guard<std::mutex> lock(*mu);
+    void *scratch = nullptr;
+    if (stream_split_workspace(st, scratch_bytes(g.m, g.n, g.k, ch), &scratch)) return false;
+    *rc = run_split(g, ch, static_cast<unsigned char *>(scratch), st);
+    return true;
+}
+
+}  // namespace fth

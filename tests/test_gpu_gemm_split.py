@@ -1,0 +1,97 @@
+"""Large fp32 products (operands split into three bf16 parts, six matrix products) against 64-bit sums.
+
+Bound on the error: each result is a sum rounded to fp32 6 K / 32 times, each rounding at most 2^-24 of a partial sum that
+grows as sqrt(k): relative 2-norm error about 2^-25 sqrt(6 K / 32 / 2), with a factor of 4 for the matrix unit's own rounding."""
+import numpy as np
+import pytest
+
+from frankentorch_amd.device import EPI_BIAS, EPI_GELU, EPI_GELU_TANH, EPI_RESIDUAL, DeviceBuffer
+
+pytestmark = pytest.mark.gpu
+
+# ragged tiles in both directions with K no multiple of 32; whole tiles; few tiles and a deep K (the K range is split);
+# tall and narrow; K shorter than a run of the split
+SHAPES = [(4097, 3077, 1001), (4096, 3072, 768), (1030, 770, 20003), (20011, 1000, 520), (2048, 2304, 3072)]
+
+
+def _gemm(hip, m, n, k, a, b, trans_a=False, trans_b=False, **kw):
+    dc = DeviceBuffer((m, n), np.float32)
+    bias, res = kw.pop("bias", None), kw.pop("residual", None)
+    up = lambda x: None if x is None else DeviceBuffer.from_host(x)
+    hip.gemm(hip.gemm_desc(m, n, k, trans_a=trans_a, trans_b=trans_b, epilogue=kw.pop("epilogue", 0)), up(a), up(b), dc, up(bias), up(res),
+             kw.pop("alpha", 1.0))
+    return dc.to_host()
+
+
+def _rel(got, ref):
+    return np.linalg.norm(got.astype(np.float64) - ref) / np.linalg.norm(ref)
+
+
+def _bound(k):
+    return 4 * 2.0 ** -25 * np.sqrt(6 * k / 32 / 2)
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("form", ["nt", "nn", "tn"])
+def test_split_product_forms(hip, m, n, k, form):
+    rng = np.random.default_rng(m + n + k)
+    a, b = rng.standard_normal((m, k), np.float32), rng.standard_normal((n, k), np.float32)
+    rows = np.unique(np.r_[np.arange(0, m, 97), m - 17 : m])
+    ref = a[rows].astype(np.float64) @ b.T.astype(np.float64)
+    got = _gemm(hip, m, n, k, np.ascontiguousarray(a.T) if form == "tn" else a, b if form == "nt" else np.ascontiguousarray(b.T),
+                trans_a=form == "tn", trans_b=form == "nt")
+    assert _rel(got[rows], ref) <= _bound(k)
+
+
+@pytest.mark.parametrize("m,n,k", [(4097, 3077, 1001), (1030, 770, 20003)])
+@pytest.mark.parametrize("epilogue,alpha", [(EPI_BIAS, 1.0), (EPI_BIAS | EPI_GELU, 1.0), (EPI_BIAS | EPI_GELU_TANH, 1.0), (EPI_BIAS | EPI_RESIDUAL, -0.5)])
+def test_split_product_epilogues(hip, m, n, k, epilogue, alpha):
+    rng = np.random.default_rng(7)
+    a, b = rng.standard_normal((m, k), np.float32), rng.standard_normal((n, k), np.float32) * np.float32(k ** -0.5)
+    bias, res = rng.standard_normal(n, np.float32), rng.standard_normal((m, n), np.float32)
+    plain = _gemm(hip, m, n, k, a, b, trans_b=True).astype(np.float64) * alpha + bias
+    got = _gemm(hip, m, n, k, a, b, trans_b=True, epilogue=epilogue, alpha=alpha, bias=bias, residual=res if epilogue & EPI_RESIDUAL else None)
+    if epilogue & EPI_GELU:
+        from scipy.special import erf
+        plain = plain * 0.5 * (1 + erf(plain / np.sqrt(2)))
+    if epilogue & EPI_GELU_TANH:
+        plain = 0.5 * plain * (1 + np.tanh(np.sqrt(2 / np.pi) * (plain + 0.044715 * plain ** 3)))
+    if epilogue & EPI_RESIDUAL:
+        plain = plain + res
+    assert np.abs(got - plain).max() <= 4e-6  # a few roundings of values up to 8
+
+
+def test_split_product_values_the_parts_cannot_hold(hip):
+    """Infinities, NaN, floats that round up to a bf16 infinity, overflowing products and magnitudes whose low bits lie below
+    the bf16 subnormals: what fp32 arithmetic gives."""
+    m, n, k = 4096, 3072, 768
+    rng = np.random.default_rng(3)
+    a, b = rng.standard_normal((m, k), np.float32), rng.standard_normal((n, k), np.float32)
+    a[5, 7], a[6, 8], a[700, 9], b[40, 11], b[41, 12] = np.inf, -np.inf, np.nan, np.inf, np.nan
+    a[1000], b[1500] = 0, 0
+    a[1000, 3], b[1500, 3] = np.finfo(np.float32).max, np.float32(0.5)
+    a[1001] = a[1002] * np.float32(1e-36)
+    a[1003] *= np.float32(1e30)
+    b[1600] *= np.float32(1e30)
+    got = _gemm(hip, m, n, k, a, b, trans_b=True)
+    with np.errstate(all="ignore"):
+        for r in (5, 6, 700, 1000, 1001, 1003, 1004):
+            ref = (a[r].astype(np.float64) * b.astype(np.float64)).sum(1)
+            want = ref.astype(np.float32)
+            assert np.array_equal(np.isnan(got[r]), np.isnan(want)), r
+            fine = np.isfinite(want)
+            assert np.array_equal(got[r][~fine & ~np.isnan(want)], want[~fine & ~np.isnan(want)]), r
+            scale = np.abs(a[r].astype(np.float64)) @ np.abs(b.astype(np.float64)).T
+            # 2^-24 per rounding of a running sum, 192 of them at most, and the subnormal spacing
+            ok = np.abs(got[r].astype(np.float64) - ref)[fine] <= (192 * 2.0 ** -24 * scale[fine] + k * 2.0 ** -149)
+            assert ok.all(), (r, int((~ok).sum()))
+    assert got[1000, 1500] == np.float32(np.finfo(np.float32).max) * np.float32(0.5)
+
+
+def test_split_product_is_repeatable_and_padding_is_not_read_into_it(hip):
+    m, n, k = 4097, 3077, 1001
+    rng = np.random.default_rng(4)
+    a, b = rng.standard_normal((m, k), np.float32), rng.standard_normal((n, k), np.float32)
+    first = _gemm(hip, m, n, k, a, b, trans_b=True)
+    _gemm(hip, m + 64, n, k, np.full((m + 64, k), np.nan, np.float32), b, trans_b=True)  # leaves NaN in the scratch memory
+    assert np.array_equal(first, _gemm(hip, m, n, k, a, b, trans_b=True))
