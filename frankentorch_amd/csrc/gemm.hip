@@ -1560,7 +1560,9 @@ int32_t gemm_entry(const fth_gemm_desc *d, T alpha, const T *a, const T *b, T *c
             const char *e = std::getenv("FT_HIP_GEMM_SPLIT");
             return e && std::atoi(e) == 0;
         }();
-        if (!split_off && d->batch == 1 && fth::split_gemm_pays(d->m, d->n, d->k)) {
+        const bool direct = d->k % 32 == 0 && d->lda % 4 == 0 && d->ldb % 4 == 0 && (d->trans_b || d->n % 4 == 0) && (!d->trans_a || d->m % 4 == 0) &&
+                            ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15u) == 0;
+        if (!split_off && d->batch == 1 && fth::split_gemm_pays(d->m, d->n, d->k, direct)) {
             fth::SplitGemm g{a, b, d->trans_a ? 1 : d->lda, d->trans_a ? d->lda : 1, d->trans_b ? d->ldb : 1, d->trans_b ? 1 : d->ldb,
                              c, bias, residual, nullptr, d->m, d->n, d->k, d->ldc, alpha, d->epilogue};
             int32_t rc = FTH_OK;
@@ -1602,7 +1604,7 @@ bool launch_nt_rowmax(int64_t m, int64_t n, int64_t k, const float *a, const flo
     }();
     if (direct_off || m <= 0 || n <= 0 || k <= 0 || k % 32 != 0 || !al(a) || !al(b) || k > lim || n > lim || big_tiles < cus || forced_tile() > 0)
         return false;
-    if (fth::split_gemm_pays(m, n, k)) {
+    if (fth::split_gemm_pays(m, n, k, true)) {
         fth::SplitGemm g{a, b, k, 1, k, 1, c, nullptr, nullptr, rowmax, m, n, k, n, 1.f, 0};
         if (fth::split_gemm(g, st, rc)) return true;
     }
@@ -1656,7 +1658,17 @@ template <typename T> int32_t launch_trans_a(GemmArgs<T> &p, const fth_gemm_desc
 
 namespace fth {
 int32_t stream_workspace(hipStream_t st, size_t bytes, void **ws) { return get_workspace(st, bytes, ws, 0); }
-int32_t stream_split_workspace(hipStream_t st, size_t bytes, void **ws) { return get_workspace(st, bytes, ws, 2); }
+bool stream_split_workspace(hipStream_t st, size_t bytes, void **ws) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &capture) != hipSuccess) return false;
+    if (capture != hipStreamCaptureStatusNone) {  // no allocation inside a capture
+        WorkspaceTable &t = workspace_table();
+        std::lock_guard<std::mutex> lock(t.mu);
+        auto it = t.table.find(std::make_pair(st, 2));
+        if (it == t.table.end() || it->second.partial_bytes < bytes) return false;
+    }
+    return get_workspace(st, bytes, ws, 2) == FTH_OK;
+}
 int64_t gemm_rowmax_groups(int64_t n) { return fth::ceil_div(n, 128) * 2; }
 bool gemm_f32_nt_rowmax(int64_t m, int64_t n, int64_t k, const float *a, const float *b, float *c, float *rowmax, hipStream_t st,
                         int32_t *rc) {

@@ -9,7 +9,7 @@
 // 2-norm error against 64-bit sums, normal operands, K 768 / 3072 / 4096: 4.2e-7 / 8.6e-7 / 1.00e-6 here, 4.95e-7 / 9.9e-7 /
 // 1.15e-6 there.
 //
-// Two passes. split_rows_kernel / split_cols_kernel write an operand's three planes once, in the order in which the product
+// Two passes. split_kernel writes an operand's three planes once, in the order in which the product
 // reads them; the product then moves planes to LDS with direct loads and has no vector arithmetic in its loop. Splitting
 // inside the product was tried and costs more: vector instructions and MFMAs share issue cycles, every element would be
 // split again by each tile that reads it, and the loop stayed at 190-230 TFLOP/s (of fp32 products) where this one reaches
@@ -87,41 +87,52 @@ __device__ __forceinline__ void store_chunk(const float (&v)[8], unsigned char *
         *reinterpret_cast<u32x4 *>(planes + (kt * kPlanes + s) * blocks * kBlock + row * 64 + ((chunk ^ swz((int)(row & 15))) << 4)) = w[s];
 }
 
-// Operand stored [rows][k]. A wavefront takes one 16-row block and one K-tile: whole 128-byte lines in, three whole 1 KB
-// blocks out. Rows and k beyond the operand are zero. Bound by memory (4 bytes in, 6 out per element).
-__global__ __launch_bounds__(256) void split_rows_kernel(const float *x, unsigned char *planes, int64_t rows, int64_t k, int64_t ld, int blocks,
-                                                         int ktiles) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t kt = (int64_t)blockIdx.x * 4 + wave;
-    if (kt >= ktiles) return;
-    const int64_t row = (int64_t)blockIdx.y * 16 + (lane >> 2);
-    const int chunk = lane & 3;
-    const int64_t k0 = kt * kBK + chunk * 8;
-    float v[8];
-    if (row < rows && k0 + 8 <= k) {
-        const float *src = x + row * ld + k0;
-        const f32x4 lo = *reinterpret_cast<const f32x4_any *>(src), hi = *reinterpret_cast<const f32x4_any *>(src + 4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[e] = lo[e];
-            v[4 + e] = hi[e];
-        }
-    } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = row < rows && k0 + e < k ? x[row * ld + k0 + e] : 0.f;
-    }
-    store_chunk(v, planes, kt, blocks, row, chunk);
-}
+// One operand to split: [rows][k] (by_k) with row pitch ld, or [k][rows] with row pitch ld.
+struct SplitArgs {
+    const float *x;
+    unsigned char *planes;
+    int64_t rows, k, ld;
+    int blocks, ktiles;  // 16-row blocks, K-tiles
+    bool by_k;
+    int64_t groups;      // workgroups
+};
 
-// Operand stored [k][rows]. A workgroup takes 64 rows and one K-tile, a wavefront one 8-k chunk of it: 256-byte runs in.
-__global__ __launch_bounds__(256) void split_cols_kernel(const float *x, unsigned char *planes, int64_t rows, int64_t k, int64_t ld, int blocks) {
-    const int lane = threadIdx.x & 63, chunk = threadIdx.x >> 6;
-    const int64_t kt = blockIdx.y, row = (int64_t)blockIdx.x * 64 + lane, k0 = kt * kBK + chunk * 8;
-    if (row >= (int64_t)blocks * 16) return;
+// Both operands of a product in one launch. Stored [rows][k]: a wavefront takes one 16-row block and one K-tile, whole 128-byte
+// lines in, three whole 1 KB blocks out. Stored [k][rows]: a workgroup takes 64 rows and one K-tile, a wavefront one 8-k chunk
+// of it, 256-byte runs in. Rows and k beyond the operand are zero. Bound by memory: 4 bytes in, 6 out per element; 103 M
+// elements (2048 x 50257) in 200 us, 5.1 TB/s.
+__global__ __launch_bounds__(256) void split_kernel(const SplitArgs first, const SplitArgs second) {
+    const bool is_first = blockIdx.x < first.groups;
+    const SplitArgs &o = is_first ? first : second;
+    const int64_t id = is_first ? blockIdx.x : blockIdx.x - first.groups;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     float v[8];
+    if (o.by_k) {
+        const int64_t quads = (o.ktiles + 3) / 4, blk = id / quads, kt = (id - blk * quads) * 4 + wave;
+        if (kt >= o.ktiles) return;
+        const int64_t row = blk * 16 + (lane >> 2);
+        const int chunk = lane & 3;
+        const int64_t k0 = kt * kBK + chunk * 8;
+        if (row < o.rows && k0 + 8 <= o.k) {
+            const float *src = o.x + row * o.ld + k0;
+            const f32x4 lo = *reinterpret_cast<const f32x4_any *>(src), hi = *reinterpret_cast<const f32x4_any *>(src + 4);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = row < rows && k0 + e < k ? x[(k0 + e) * ld + row] : 0.f;
-    store_chunk(v, planes, kt, blocks, row, chunk);
+            for (int e = 0; e < 4; ++e) {
+                v[e] = lo[e];
+                v[4 + e] = hi[e];
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = row < o.rows && k0 + e < o.k ? o.x[row * o.ld + k0 + e] : 0.f;
+        }
+        store_chunk(v, o.planes, kt, o.blocks, row, chunk);
+    } else {
+        const int64_t across = (o.blocks + 3) / 4, kt = id / across, row = (id - kt * across) * 64 + lane, k0 = kt * kBK + wave * 8;
+        if (row >= (int64_t)o.blocks * 16) return;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = row < o.rows && k0 + e < o.k ? o.x[(k0 + e) * o.ld + row] : 0.f;
+        store_chunk(v, o.planes, kt, o.blocks, row, wave);
+    }
 }
 
 struct PlaneArgs {
@@ -468,13 +479,17 @@ __global__ __launch_bounds__(256) void plane_reduce_kernel(const PlaneArgs p) {
 
 // ---- which tile, how many runs of K ----
 
-struct Tile { int bm, bn, per_cu; double rate; };  // rate: TFLOP/s of fp32 products with every workgroup busy
-constexpr Tile kTiles[] = {{128, 256, 1, 250.}, {128, 192, 1, 238.}, {64, 128, 2, 200.}};
+// One workgroup of 128 x 256 or 128 x 192 a compute unit, or two of 64 x 128. Rates are TFLOP/s of fp32 products with every
+// compute unit busy, measured on 4096^3, 8192 x 768 x 3072 and 2331 x 768 x 768; the small tile's with one and with two
+// workgroups on a compute unit.
+struct Tile { int bm, bn; double rate[2]; };
+constexpr Tile kTiles[] = {{128, 256, {250., 250.}}, {128, 192, {238., 238.}}, {64, 128, {145., 200.}}};
+constexpr int kResident[] = {1, 1, 2};
 
 struct Choice { int tile = -1, splits = 1, kt_per = 0; double us = 0; };
 
-// Time of the product alone: rounds of tiles over the compute units, and for split K the partial sums' way through memory
-// (written and read at 4 TB/s, 4 us for the second launch).
+// Time of the product alone: the tiles that the busiest compute unit works through, and for split K the partial sums' way
+// through memory (written and read at 4 TB/s, 4 us for the second launch).
 Choice choose(int64_t m, int64_t n, int64_t k, bool rowmax) {
     const int cus = fth::compute_units() > 0 ? fth::compute_units() : 256;
     const int64_t ktiles = fth::ceil_div(k, kBK);
@@ -484,9 +499,11 @@ Choice choose(int64_t m, int64_t n, int64_t k, bool rowmax) {
         const int64_t tiles = fth::ceil_div(m, c.bm) * fth::ceil_div(n, c.bn);
         for (int s = 1; s <= (rowmax ? 1 : 16); ++s) {
             const int64_t per = fth::ceil_div(ktiles, s);
-            if (s > 1 && (per < 8 || (int64_t)(s - 1) * per >= ktiles)) break;
-            const int64_t rounds = fth::ceil_div(tiles * s, (int64_t)cus * c.per_cu);
-            double us = rounds * (2.0 * c.bm * c.bn * kBK * per * c.per_cu * cus / c.rate * 1e-6 + 3.0) + 2.0;
+            if (s > 1 && (per < 8 || (s - 1) * per >= ktiles)) break;
+            const int64_t most = fth::ceil_div(tiles * s, (int64_t)cus);
+            const double one = 2.0 * c.bm * c.bn * kBK * per * cus * 1e-6;
+            double us = 2.0 + 2.0 * most / kResident[t];
+            us += kResident[t] == 1 ? most * one / c.rate[0] : (most / 2) * 2 * one / c.rate[1] + (most % 2) * one / c.rate[0];
             if (s > 1) us += (s + 1.0) * m * n * 4 / 4e6 + 4.0;
             if (best.tile < 0 || us < best.us) best = {t, s, (int)per, us};
         }
@@ -513,14 +530,10 @@ template <int BM, int BN, int WM, int WN, bool ROWMAX> int32_t launch_planes(Pla
     return FTH_OK;
 }
 
-int32_t launch_split(const float *x, unsigned char *planes, int64_t rows, int64_t k, int64_t rs, int64_t ks, hipStream_t st) {
-    const int blocks = (int)fth::ceil_div(rows, 16), ktiles = (int)fth::ceil_div(k, kBK);
-    if (ks == 1)
-        split_rows_kernel<<<dim3((unsigned)fth::ceil_div(ktiles, 4), (unsigned)blocks), dim3(256), 0, st>>>(x, planes, rows, k, rs, blocks, ktiles);
-    else
-        split_cols_kernel<<<dim3((unsigned)fth::ceil_div(blocks, 4), (unsigned)ktiles), dim3(256), 0, st>>>(x, planes, rows, k, ks, blocks);
-    FTH_CHECK_LAUNCH("gemm_split");
-    return FTH_OK;
+SplitArgs split_args(const float *x, unsigned char *planes, int64_t rows, int64_t k, int64_t rs, int64_t ks) {
+    SplitArgs o{x, planes, rows, k, ks == 1 ? rs : ks, (int)fth::ceil_div(rows, 16), (int)fth::ceil_div(k, kBK), ks == 1, 0};
+    o.groups = o.by_k ? fth::ceil_div(o.ktiles, 4) * o.blocks : fth::ceil_div(o.blocks, 4) * o.ktiles;
+    return o;
 }
 
 int32_t run_split(const fth::SplitGemm &g, const Choice &ch, unsigned char *scratch, hipStream_t st) {
@@ -536,15 +549,16 @@ int32_t run_split(const fth::SplitGemm &g, const Choice &ch, unsigned char *scra
     p.a = pa;
     p.b = pb;
     p.partial = reinterpret_cast<float *>(pb + plane_bytes(g.n, g.k));
-    if (int32_t rc = launch_split(g.a, pa, g.m, g.k, g.a_rs, g.a_ks, st)) return rc;
-    if (int32_t rc = launch_split(g.b, pb, g.n, g.k, g.b_rs, g.b_ks, st)) return rc;
+    const SplitArgs sa = split_args(g.a, pa, g.m, g.k, g.a_rs, g.a_ks), sb = split_args(g.b, pb, g.n, g.k, g.b_rs, g.b_ks);
+    split_kernel<<<dim3((unsigned)(sa.groups + sb.groups)), dim3(256), 0, st>>>(sa, sb);
+    FTH_CHECK_LAUNCH("gemm_split");
     int32_t rc = FTH_OK;
     switch (ch.tile) {
         case 0:
-            rc = g.rowmax ? launch_planes<128, 256, 2, 4, true>(p, kTiles[0].per_cu, st) : launch_planes<128, 256, 2, 4, false>(p, kTiles[0].per_cu, st);
+            rc = g.rowmax ? launch_planes<128, 256, 2, 4, true>(p, kResident[0], st) : launch_planes<128, 256, 2, 4, false>(p, kResident[0], st);
             break;
-        case 1: rc = launch_planes<128, 192, 2, 4, false>(p, kTiles[1].per_cu, st); break;
-        default: rc = launch_planes<64, 128, 2, 2, false>(p, kTiles[2].per_cu, st); break;
+        case 1: rc = launch_planes<128, 192, 2, 4, false>(p, kResident[1], st); break;
+        default: rc = launch_planes<64, 128, 2, 2, false>(p, kResident[2], st); break;
     }
     if (rc || ch.splits == 1) return rc;
     plane_reduce_kernel<<<dim3((unsigned)fth::ceil_div(g.m * g.n, 256)), dim3(256), 0, st>>>(p);
@@ -560,25 +574,27 @@ size_t scratch_bytes(int64_t m, int64_t n, int64_t k, const Choice &ch) {
 
 namespace fth {
 
-bool split_gemm_pays(int64_t m, int64_t n, int64_t k) {
-    if (m < 64 || n < 64 || k < 128 || m > (1 << 20) || n > (1 << 20) || k > (1 << 20) || m * n > ((int64_t)1 << 31)) return false;
+bool split_gemm_pays(int64_t m, int64_t n, int64_t k, bool fp32_direct) {
+    // Under 1.5 GFLOP the fp32 path has its own small kernels and the launches decide: a 128 x 256 x 256 block would lose 26 us.
+    if (m < 64 || n < 64 || k < 128 || 2.0 * m * n * k < 1.5e9 || m > (1 << 20) || n > (1 << 20) || k > (1 << 20) || m * n > ((int64_t)1 << 31)) return false;
     const Choice ch = choose(m, n, k, false);
     if (scratch_bytes(m, n, k, ch) > kScratchBound) return false;
-    // The planes: 10 bytes an element at 3.5 TB/s and two launches; the fp32 kernel: 130 TFLOP/s.
-    const double us = ch.us + 10.0 * k * (m + n) / 3.5e6 + 5.0;
-    return us < 0.95 * 2.0 * m * n * k / 130e6;
+    // This path: the product, and the planes at 10 bytes an element, 4.5 TB/s and 3 us. The fp32 kernels: 130 TFLOP/s and 16 us
+    // (whole-tile effects and the fix-up pass of a split K) with direct-to-LDS operands, 0.6 of that without.
+    // us, fp32 -> split: 2331 x 768 x 768 44 -> 32, 768 x 768 x 2331 (A stored [k, m]) 62 -> 39, 4000 x 1024 x 1024 83 -> 55; where
+    // the line is, 1024^3 32 -> 29; below it, 512 x 768 x 768 21 -> 21 and 1000 x 512 x 512 17 -> 20.
+    const double ideal = 2.0 * m * n * k / 130e6;
+    return ch.us + 10.0 * k * (m + n) / 4.5e6 + 3.0 < 0.95 * ((fp32_direct ? ideal : 1.7 * ideal) + 16.0);
 }
 
 bool split_gemm(const SplitGemm &g, hipStream_t st, int32_t *rc) {
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return false;
     const Choice ch = choose(g.m, g.n, g.k, g.rowmax != nullptr);
     // The scratch belongs to the stream; the lock keeps another thread's product on the same stream from being queued between
     // the planes and their reader.
     static std::mutex *mu = new std::mutex();
     std::lock_guard<std::mutex> lock(*mu);
     void *scratch = nullptr;
-    if (stream_split_workspace(st, scratch_bytes(g.m, g.n, g.k, ch), &scratch)) return false;
+    if (!stream_split_workspace(st, scratch_bytes(g.m, g.n, g.k, ch), &scratch)) return false;
     *rc = run_split(g, ch, static_cast<unsigned char *>(scratch), st);
     return true;
 }
