@@ -15,10 +15,11 @@
 // split again by each tile that reads it, and the loop stayed at 190-230 TFLOP/s (of fp32 products) where this one reaches
 // 240-263.
 //
-// What the split cannot represent is found in the results. An infinity, a NaN or a float that rounds up to a bf16 infinity
-// leaves a non-finite sum; magnitudes whose lowest bits fall below the bf16 subnormals (operands under 2^-109) can only
-// matter in a result under 2^-100. A wavefront that holds a non-finite sum or a non-zero one under 2^-100 computes its part
-// of the tile again from the fp32 operands on fp32 MFMAs.
+// What the split cannot represent is found in the results. Operands of 2^24 and more, infinities, NaN and non-zero ones of
+// 2^-134 and less (which would vanish) are written as NaN planes and leave NaN sums. Operands under 2^-109 lose their lowest
+// bits, 2^-134 each at most; beside a partner under 2^24 that is 2^-110 per product, which can matter only in a sum under
+// 2^-70. A wavefront that holds a non-finite sum or a non-zero one under 2^-70 computes its part of the tile again from the
+// fp32 operands on fp32 MFMAs.
 //
 // replaces gemm::sgemm / sgemm_bt / sgemm_tb (crates/ft-kernel-cpu/src/lib.rs:1310-1338, 1430-1524) for large products.
 
@@ -37,7 +38,8 @@ constexpr int kGroupM = 8;
 constexpr int kBK = 32;       // k of a K-tile: one 16 x 16 x 32 MFMA
 constexpr int kPlanes = 3;
 constexpr int kBlock = 1024;  // bytes of one plane of 16 rows x 32 k
-constexpr float kTiny = 0x1p-100f;
+constexpr float kTiny = 0x1p-70f;
+constexpr uint32_t kTooLarge = 0x4b800000u, kTooSmall = 0x00008000u;  // bits of 2^24 and of 2^-134
 
 using bf16x8 = __attribute__((ext_vector_type(8))) __bf16;
 using bf16x2 = __attribute__((ext_vector_type(2))) __bf16;
@@ -52,6 +54,12 @@ __device__ __forceinline__ uint32_t pack_bf16(float x, float y) {
 }
 __device__ __forceinline__ float lo_f32(uint32_t p) { return __builtin_bit_cast(float, p << 16); }
 __device__ __forceinline__ float hi_f32(uint32_t p) { return __builtin_bit_cast(float, p & 0xffff0000u); }
+
+// NaN in the place of a float that the parts cannot stand for.
+__device__ __forceinline__ float representable(float x) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, x) & 0x7fffffffu;
+    return u >= kTooLarge || u - 1u < kTooSmall ? __builtin_nanf("") : x;
+}
 
 // The three parts of two floats, one dword each.
 __device__ __forceinline__ void split2(float x, float y, uint32_t &p0, uint32_t &p1, uint32_t &p2) {
@@ -77,7 +85,7 @@ __device__ __forceinline__ void store_chunk(const float (&v)[8], unsigned char *
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         uint32_t p0, p1, p2;
-        split2(v[2 * e], v[2 * e + 1], p0, p1, p2);
+        split2(representable(v[2 * e]), representable(v[2 * e + 1]), p0, p1, p2);
         w[0][e] = p0;
         w[1][e] = p1;
         w[2][e] = p2;

@@ -88,6 +88,22 @@ def test_split_product_values_the_parts_cannot_hold(hip):
     assert got[1000, 1500] == np.float32(np.finfo(np.float32).max) * np.float32(0.5)
 
 
+@pytest.mark.parametrize("small,large", [(-120, 60), (-128, 20), (-140, 40), (-100, 23)])
+def test_split_product_small_beside_large(hip, small, large):
+    """A row whose low bits (or all of them) lie below the bf16 subnormals, times columns large enough to bring the sums back:
+    the same bound as for ordinary operands (the sums of a subnormal row too: its floats are exact)."""
+    m, n, k = 2048, 2304, 768
+    rng = np.random.default_rng(small + large + 500)
+    a, b = rng.standard_normal((m, k), np.float32), rng.standard_normal((n, k), np.float32)
+    a[11] = np.ldexp(a[11], small)
+    b[100:160] = np.ldexp(b[100:160], large)
+    got = _gemm(hip, m, n, k, a, b, trans_b=True).astype(np.float64)
+    for rows, cols in ((slice(11, 12), slice(100, 160)), (slice(0, 11), slice(90, 170)), (slice(11, 12), slice(160, 400))):
+        ref = a[rows].astype(np.float64) @ b[cols].T.astype(np.float64)
+        floor = np.sqrt(ref.size) * 2.0 ** -126  # results that are subnormal themselves
+        assert np.linalg.norm(got[rows, cols] - ref) <= _bound(k) * np.linalg.norm(ref) + floor
+
+
 def test_split_product_is_repeatable_and_padding_is_not_read_into_it(hip):
     m, n, k = 4097, 3077, 1001
     rng = np.random.default_rng(4)
