@@ -1261,7 +1261,8 @@ struct StreamWorkspace {
     void *partials = nullptr;
     size_t partial_bytes = 0;
 };
-// slot 0: split-tile accumulators; slot 1: transposed copy of a [k, m] A operand; slot 2: planes of the split product.
+// slot 0: split-tile accumulators; slot 1: transposed copy of a [k, m] A operand; slot 2: planes of the split product;
+// slot 3: shares of few-query attention.
 //
 // A block that a larger request outgrows is retired, never handed back to the shared pool: kernels
 // queued on the stream may still be using it, the pool serves every stream and thread (so "ordered
@@ -1657,17 +1658,16 @@ template <typename T> int32_t launch_trans_a(GemmArgs<T> &p, const fth_gemm_desc
 }  // namespace
 
 namespace fth {
-int32_t stream_workspace(hipStream_t st, size_t bytes, void **ws) { return get_workspace(st, bytes, ws, 0); }
-bool stream_split_workspace(hipStream_t st, size_t bytes, void **ws) {
+bool try_stream_workspace(hipStream_t st, size_t bytes, StreamBlock use, void **ws) {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &capture) != hipSuccess) return false;
     if (capture != hipStreamCaptureStatusNone) {  // no allocation inside a capture
         WorkspaceTable &t = workspace_table();
         std::lock_guard<std::mutex> lock(t.mu);
-        auto it = t.table.find(std::make_pair(st, 2));
+        auto it = t.table.find(std::make_pair(st, (int)use));
         if (it == t.table.end() || it->second.partial_bytes < bytes) return false;
     }
-    return get_workspace(st, bytes, ws, 2) == FTH_OK;
+    return get_workspace(st, bytes, ws, use) == FTH_OK;
 }
 int64_t gemm_rowmax_groups(int64_t n) { return fth::ceil_div(n, 128) * 2; }
 bool gemm_f32_nt_rowmax(int64_t m, int64_t n, int64_t k, const float *a, const float *b, float *c, float *rowmax, hipStream_t st,

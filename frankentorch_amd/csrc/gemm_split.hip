@@ -602,7 +602,7 @@ bool split_gemm(const SplitGemm &g, hipStream_t st, int32_t *rc) {
     static std::mutex *mu = new std::mutex();
     std::lock_guard<std::mutex> lock(*mu);
     void *scratch = nullptr;
-    if (!stream_split_workspace(st, scratch_bytes(g.m, g.n, g.k, ch), &scratch)) return false;
+    if (!try_stream_workspace(st, scratch_bytes(g.m, g.n, g.k, ch), kSplitPlanes, &scratch)) return false;
     *rc = run_split(g, ch, static_cast<unsigned char *>(scratch), st);
     return true;
 }

@@ -1123,10 +1123,12 @@ int32_t sdpa_entry(const fth_sdpa_desc *d, double scale, const T *q, const T *k,
                                 al16(q) && al16(k) && al16(v) && al16(out) &&
                                 d->k_row_stride < (1 << 22) && d->v_row_stride < (1 << 22);  // a tile's lane offsets fit 32 bits
         // Few queries against a cache: the kernels below pad them to 32 or 128 query rows and read K and V once per query head.
-        if (strides_ok && fth::sdpa_decode_applies(*d))
-            return fth::sdpa_decode_f32(*d, (float)scale, reinterpret_cast<const float *>(q), reinterpret_cast<const float *>(k),
-                                        reinterpret_cast<const float *>(v), reinterpret_cast<const float *>(a.mask), mask_bh_stride,
-                                        reinterpret_cast<float *>(out), st);
+        int32_t rc = FTH_OK;
+        if (strides_ok && fth::sdpa_decode_applies(*d) &&
+            fth::sdpa_decode_f32(*d, (float)scale, reinterpret_cast<const float *>(q), reinterpret_cast<const float *>(k),
+                                 reinterpret_cast<const float *>(v), reinterpret_cast<const float *>(a.mask), mask_bh_stride,
+                                 reinterpret_cast<float *>(out), st, &rc))
+            return rc;
         // the unmasked MFMA kernels take the row maximum on the raw scores, which needs a positive scale
         if (strides_ok && d->d_k == d->d_v && d->seq_k > 0 && (masked || scale > T(0))) {
             // Too few 32-query blocks to give every compute unit one: the key-split kernel (one launch, no LDS staging)

@@ -22,6 +22,7 @@
 // Semantics of sdpa_forward_f32 / sdpa_forward_masked_f64 (crates/ft-kernel-cpu/src/lib.rs:5200-5284, 4661-4741): scale after
 // the product, additive mask, softmax over all keys; a row with every key hidden is NaN.
 
+#include <mutex>
 #include <type_traits>
 
 #include "common.hpp"
@@ -266,19 +267,21 @@ template <int D, int QT> __global__ __launch_bounds__(256) void sdpa_decode_merg
     *reinterpret_cast<F4 *>(p.out + batch * p.d.o_batch_stride + h * p.d.o_head_stride + qi * p.d.o_row_stride + 4 * c) = y;
 }
 
-template <int D, int QT> int32_t launch(DecodeArgs &a, hipStream_t st) {
+// *done stays false, with nothing launched, when the grid or the scratch memory cannot be had.
+template <int D, int QT> int32_t launch(DecodeArgs &a, hipStream_t st, bool *done) {
     constexpr int ROWS = 16 * QT;
     a.row_tiles = (int)fth::ceil_div((int64_t)a.group * a.d.seq_q, ROWS);
     const int64_t units = a.d.num_bh / a.group * a.row_tiles;
     const int64_t grid = units * a.nsplit;
-    FTH_ARG(grid <= 2147483647LL, "sdpa: grid too large");
+    if (grid > 2147483647LL) return FTH_OK;
     if (a.nsplit > 1) {
         void *ws = nullptr;
         const int64_t slots = grid * ROWS;
-        if (int32_t rc = fth::stream_workspace(st, (size_t)(slots * (D + 2)) * sizeof(float), &ws)) return rc;
+        if (!fth::try_stream_workspace(st, (size_t)(slots * (D + 2)) * sizeof(float), fth::kDecodeShares, &ws)) return FTH_OK;
         a.part_o = static_cast<float *>(ws);
         a.part_ml = a.part_o + slots * D;
     }
+    *done = true;
     if (a.mask) sdpa_decode_kernel<D, QT, true><<<dim3((unsigned)grid), dim3(64), 0, st>>>(a);
     else sdpa_decode_kernel<D, QT, false><<<dim3((unsigned)grid), dim3(64), 0, st>>>(a);
     FTH_CHECK_LAUNCH("sdpa_decode");
@@ -290,9 +293,9 @@ template <int D, int QT> int32_t launch(DecodeArgs &a, hipStream_t st) {
     return FTH_OK;
 }
 
-template <int D> int32_t launch_rows(DecodeArgs &a, hipStream_t st) {
+template <int D> int32_t launch_rows(DecodeArgs &a, hipStream_t st, bool *done) {
     // one row tile of 16 where the rows fit it, else tiles of 32
-    return (int64_t)a.group * a.d.seq_q <= 16 ? launch<D, 1>(a, st) : launch<D, 2>(a, st);
+    return (int64_t)a.group * a.d.seq_q <= 16 ? launch<D, 1>(a, st, done) : launch<D, 2>(a, st, done);
 }
 
 }  // namespace
@@ -306,8 +309,8 @@ bool sdpa_decode_applies(const fth_sdpa_desc &d) {
            d.seq_k * d.k_row_stride < ((int64_t)1 << 30) && d.seq_k * d.v_row_stride < ((int64_t)1 << 30);
 }
 
-int32_t sdpa_decode_f32(const fth_sdpa_desc &d, float scale, const float *q, const float *k, const float *v, const float *mask,
-                        int64_t mask_bh_stride, float *out, hipStream_t st) {
+bool sdpa_decode_f32(const fth_sdpa_desc &d, float scale, const float *q, const float *k, const float *v, const float *mask,
+                     int64_t mask_bh_stride, float *out, hipStream_t st, int32_t *rc) {
     DecodeArgs a;
     a.q = q; a.k = k; a.v = v; a.mask = mask; a.out = out;
     a.part_o = a.part_ml = nullptr;
@@ -325,9 +328,12 @@ int32_t sdpa_decode_f32(const fth_sdpa_desc &d, float scale, const float *q, con
     want = want < 1 ? 1 : want > most ? most : want;
     a.tiles_per_split = (int)fth::ceil_div(tiles, want);
     a.nsplit = (int)fth::ceil_div(tiles, a.tiles_per_split);
-    if (d.d_k == 128) return launch_rows<128>(a, st);
-    if (d.d_k == 64) return launch_rows<64>(a, st);
-    return launch_rows<32>(a, st);
+    // The scratch belongs to the stream; the lock keeps another thread's call on it from being queued before the merge.
+    static std::mutex *mu = new std::mutex();
+    std::lock_guard<std::mutex> lock(*mu);
+    bool done = false;
+    *rc = d.d_k == 128 ? launch_rows<128>(a, st, &done) : d.d_k == 64 ? launch_rows<64>(a, st, &done) : launch_rows<32>(a, st, &done);
+    return done;
 }
 
 }  // namespace fth
