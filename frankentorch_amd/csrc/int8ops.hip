@@ -8,6 +8,7 @@
 // the order of the sum and every output equals the reference's bit for bit; the three float operations
 // of the dequantisation are kept apart (this file is built without contraction).
 //
+// Up to 64 rows take i8_skinny_kernel (described there); more rows the tiled kernel:
 // Product kernel: v_mfma_i32_32x32x32_i8, 256 x 256 output tile per workgroup (2 x 2 wavefronts of 128 x 128;
 // 128 x 128 tiles for problems with few tiles), K in steps of 64 bytes through a ring of four LDS stages filled by global_load_lds_dwordx4 (a
 // stage of this kernel is only 256 MFMA cycles per wavefront, far less than a memory round trip, so three
@@ -415,9 +416,90 @@ int32_t quantize_entry(const float *x, int64_t rows, int64_t cols, int8_t *q, fl
     else if (vec && cols <= 2048) quantize_rows_vec_kernel<2><<<dim3((unsigned)rows), dim3(256), 0, st>>>(x, cols, q, scales);
     else if (vec && cols <= 4096) quantize_rows_vec_kernel<4><<<dim3((unsigned)rows), dim3(256), 0, st>>>(x, cols, q, scales);
     else if (vec && cols <= 8192) quantize_rows_vec_kernel<8><<<dim3((unsigned)rows), dim3(256), 0, st>>>(x, cols, q, scales);
+    // (16 rows of 11008, product included: 39.7 us with the plain kernel, 18.8 us with this one)
+    else if (vec && cols <= 16384) quantize_rows_vec_kernel<16><<<dim3((unsigned)rows), dim3(256), 0, st>>>(x, cols, q, scales);
     else quantize_rows_kernel<<<dim3((unsigned)rows), dim3(256), 0, st>>>(x, cols, q, scales);
     FTH_CHECK_LAUNCH("quantize_rows_i8");
     return FTH_OK;
+}
+
+// Up to 16 MT rows of activations (the tokens of a decode step): bound by reading the weights once, so the split of the work
+// is by output columns, 16 NT a workgroup, and inside it by K: eight wavefronts take a run of 64-byte K steps each, straight from
+// memory to the matrix units (nothing is read twice, so nothing goes through LDS), UN steps requested ahead. The integer
+// partial sums meet in LDS; their order does not matter. Rows past m / n are clamped on the load side and never stored.
+// The activations are read again by each workgroup, out of L2; from 17 rows on that traffic is as much as the weights', so
+// NT = 2 halves it where there are columns enough.
+// Whole call with the quantiser, weights rotating through 270 MB, 128 x 128 tiles -> here: 1 x 4096 x 4096 (m x k x n)
+// 20.4 -> 8.4 us, 13 x 4096 x 11008 28.2 -> 16.9 us, 32 x 4096 x 4096 25.4 -> 11.6 us.
+template <int MT, int NT>
+__global__ __launch_bounds__(512) void i8_skinny_kernel(const I8Args p) {
+    constexpr int NW = 8, UN = MT + NT <= 3 ? 8 : 4;
+    __shared__ int red[NW][MT * NT * 4][kWave];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, lq = lane >> 4;
+    const int64_t n0 = (int64_t)blockIdx.x * (16 * NT);
+    const int8_t *w[NT], *x[MT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const int64_t row = n0 + j * 16 + l16 < p.n ? n0 + j * 16 + l16 : p.n - 1;
+        w[j] = p.b + row * p.k + lq * 16;
+    }
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        const int64_t row = t * 16 + l16 < p.m ? t * 16 + l16 : p.m - 1;
+        x[t] = p.a + row * p.k + lq * 16;
+    }
+    const int steps = (int)(p.k / 64), per = (steps + NW - 1) / NW;
+    int s = wave * per;
+    const int end = s + per < steps ? s + per : steps;
+    V4i acc[MT][NT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[t][j] = V4i{0, 0, 0, 0};
+    for (; s + UN <= end; s += UN) {
+        V4i wv[UN][NT], xv[UN][MT];
+#pragma unroll
+        for (int u = 0; u < UN; ++u) {
+#pragma unroll
+            for (int j = 0; j < NT; ++j) wv[u][j] = *reinterpret_cast<const V4i *>(w[j] + (int64_t)(s + u) * 64);
+#pragma unroll
+            for (int t = 0; t < MT; ++t) xv[u][t] = *reinterpret_cast<const V4i *>(x[t] + (int64_t)(s + u) * 64);
+        }
+#pragma unroll
+        for (int u = 0; u < UN; ++u)
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) acc[t][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xv[u][t], wv[u][j], acc[t][j], 0, 0, 0);
+    }
+    for (; s < end; ++s) {
+        V4i wv[NT];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) wv[j] = *reinterpret_cast<const V4i *>(w[j] + (int64_t)s * 64);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            const V4i xv = *reinterpret_cast<const V4i *>(x[t] + (int64_t)s * 64);
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[t][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xv, wv[j], acc[t][j], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) red[wave][(t * NT + j) * 4 + r][lane] = acc[t][j][r];
+    __syncthreads();
+    for (int i = wave; i < MT * NT * 4; i += NW) {  // accumulator element r of a lane: row 4 (lane / 16) + r, column lane % 16
+        const int64_t row = i / (4 * NT) * 16 + lq * 4 + (i & 3), col = n0 + (i / 4) % NT * 16 + l16;
+        if (row >= p.m || col >= p.n) continue;
+        uint32_t sum = 0;  // wraps as the matrix units' accumulators do
+#pragma unroll
+        for (int v = 0; v < NW; ++v) sum += (uint32_t)red[v][i][lane];
+        float y = (float)(int)sum * p.a_scales[row] * p.b_scales[col];
+        if (p.bias) y += p.bias[col];
+        p.c[row * p.n + col] = y;
+    }
 }
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -459,6 +541,20 @@ int32_t fth_dev_linear_int8_prequantized_f32(const int8_t *x_i8, const float *a_
             return e ? std::atoi(e) : 0;
         }();
         const bool big = forced == 256 || forced == 512 || (forced != 128 && tiles256 >= cus && k >= 2048);
+        // Rows of one to four 16-row MFMA tiles: a 128-row tile would be mostly padding and leave the chip short of workgroups.
+        // At the upper end of the rule the two are close where n is large: 64 x 4096 x 11008 35.3 -> 33.3 us, 64 x 4096 x 4096
+        // 29.5 -> 16.1 us. Past it the activations would be read from L2 more often than the weights from memory.
+        if (m <= 64 && forced == 0) {
+            const bool wide = n >= 32 * (int64_t)cus;  // 32 columns a workgroup still give every compute unit one: half the activation reads
+            const dim3 grid((unsigned)fth::ceil_div(n, 16)), grid2((unsigned)fth::ceil_div(n, 32));
+            if (m <= 16) i8_skinny_kernel<1, 1><<<grid, dim3(512), 0, st>>>(p);
+            else if (m <= 32 && wide) i8_skinny_kernel<2, 2><<<grid2, dim3(512), 0, st>>>(p);
+            else if (m <= 32) i8_skinny_kernel<2, 1><<<grid, dim3(512), 0, st>>>(p);
+            else if (wide) i8_skinny_kernel<4, 2><<<grid2, dim3(512), 0, st>>>(p);
+            else i8_skinny_kernel<4, 1><<<grid, dim3(512), 0, st>>>(p);
+            FTH_CHECK_LAUNCH("i8_skinny");
+            return FTH_OK;
+        }
         int32_t rc;
         if (!big) rc = launch_i8_gemm<2, 2, 2, 2>(p, st);
         else if (forced == 256) rc = launch_i8_gemm<4, 4, 2, 2>(p, st);  // four wavefronts of 128 x 128 (kept for comparison)

@@ -82,6 +82,16 @@ def test_linear_int8_dynamic_is_bit_exact(hip, oracle, m, k, n, with_bias):
         assert (ref * y).sum() / np.sqrt((ref * ref).sum() * (y * y).sum()) > 0.999
 
 
+# few rows: edges of the 16-row tiles, ragged columns, K shorter than one step a wavefront, whole and broken runs of it
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 32, 33, 63, 64, 65])
+@pytest.mark.parametrize("k,n", [(64, 16), (448, 1), (576, 53), (4096, 130), (11008, 33), (576, 8209), (16384, 17), (16448, 16)])
+def test_few_rows_are_bit_exact(hip, oracle, m, k, n):
+    x, w, bias = synth.normal(43, "x", (m, k), 0.0, 3.0), synth.normal(43, "w", (n, k), 0.0, 0.5), synth.normal(43, "b", (n,))
+    w_i8, w_scales = oracle.quantize_rows_i8(w)
+    for b in (bias, None):
+        assert np.array_equal(_bits(_linear(hip, x, w_i8, w_scales, b)), _bits(oracle.linear_int8_dynamic(x, w_i8, w_scales, b)))
+
+
 def test_extreme_integers_do_not_overflow(hip, oracle):
     """Every product +-127 * +-127 with the same sign over K = 4096: |acc| = 66 064 384, far inside int32."""
     m, k, n = 64, 4096, 128
