@@ -21,6 +21,7 @@ LIB_PATH = os.path.join(PKG_DIR, "libft_kernel_hip.so")
 HIP_SOURCES = [
     "runtime.hip",
     "staging.hip",
+    "stream_scratch.hip",
     "rowops.hip",
     "indexops.hip",
     "gemm.hip",

@@ -27,13 +27,6 @@ hipStream_t resolve_stream(fth_stream s);
 // Number of compute units of device 0 (cached).
 int compute_units();
 
-// Scratch memory of the stream, one block per stream and use: for kernels launched on it right away (their successors on the
-// stream run after them). The caller holds a lock of its own from here until its last launch, so that another thread's kernels
-// on the same stream do not come between. Kept and grown, at most 1 GiB is asked for. False when it cannot be had; while the
-// stream is being captured, when it would have to grow.
-enum StreamBlock { kSplitPlanes = 2, kDecodeShares = 3 };
-bool try_stream_workspace(hipStream_t st, size_t bytes, StreamBlock use, void **ws);
-
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Softmax over contiguous rows too long or too ragged for the 128-bit row kernels (any length up to 65 536 floats /

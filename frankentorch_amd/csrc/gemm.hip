@@ -49,6 +49,7 @@
 #include "devmath.hpp"
 #include "gemm_split.hpp"
 #include "pool.hpp"
+#include "stream_scratch.hpp"
 
 namespace {
 
@@ -1261,8 +1262,7 @@ struct StreamWorkspace {
     void *partials = nullptr;
     size_t partial_bytes = 0;
 };
-// slot 0: split-tile accumulators; slot 1: transposed copy of a [k, m] A operand; slot 2: planes of the split product;
-// slot 3: shares of few-query attention.
+// slot 0: split-tile accumulators; slot 1: transposed copy of a [k, m] A operand.
 //
 // A block that a larger request outgrows is retired, never handed back to the shared pool: kernels
 // queued on the stream may still be using it, the pool serves every stream and thread (so "ordered
@@ -1658,17 +1658,6 @@ template <typename T> int32_t launch_trans_a(GemmArgs<T> &p, const fth_gemm_desc
 }  // namespace
 
 namespace fth {
-bool try_stream_workspace(hipStream_t st, size_t bytes, StreamBlock use, void **ws) {
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &capture) != hipSuccess) return false;
-    if (capture != hipStreamCaptureStatusNone) {  // no allocation inside a capture
-        WorkspaceTable &t = workspace_table();
-        std::lock_guard<std::mutex> lock(t.mu);
-        auto it = t.table.find(std::make_pair(st, (int)use));
-        if (it == t.table.end() || it->second.partial_bytes < bytes) return false;
-    }
-    return get_workspace(st, bytes, ws, use) == FTH_OK;
-}
 int64_t gemm_rowmax_groups(int64_t n) { return fth::ceil_div(n, 128) * 2; }
 bool gemm_f32_nt_rowmax(int64_t m, int64_t n, int64_t k, const float *a, const float *b, float *c, float *rowmax, hipStream_t st,
                         int32_t *rc) {
@@ -1713,9 +1702,11 @@ int32_t fth_dev_linear_argmax_f32(const float *x, const float *w, int64_t rows, 
 
 int32_t fth_device_workspace_info(uint64_t *live_bytes, uint64_t *retired_bytes) {
     WorkspaceTable &t = workspace_table();
+    uint64_t live = 0, retired = 0;
+    fth::stream_scratch_stats(&live, &retired);
     std::lock_guard<std::mutex> lock(t.mu);
-    if (live_bytes) *live_bytes = t.live_bytes;
-    if (retired_bytes) *retired_bytes = t.retired_bytes;
+    if (live_bytes) *live_bytes = t.live_bytes + live;
+    if (retired_bytes) *retired_bytes = t.retired_bytes + retired;
     return FTH_OK;
 }
 

@@ -24,11 +24,11 @@
 // replaces gemm::sgemm / sgemm_bt / sgemm_tb (crates/ft-kernel-cpu/src/lib.rs:1310-1338, 1430-1524) for large products.
 
 #include <cfloat>
-#include <mutex>
 
 #include "common.hpp"
 #include "devmath.hpp"
 #include "gemm_split.hpp"
+#include "stream_scratch.hpp"
 
 namespace {
 
@@ -521,8 +521,6 @@ Choice choose(int64_t m, int64_t n, int64_t k, bool rowmax) {
 
 size_t plane_bytes(int64_t rows, int64_t k) { return (size_t)(fth::ceil_div(k, kBK) * kPlanes * fth::ceil_div(rows, 16)) * kBlock; }
 
-constexpr size_t kScratchBound = (size_t)1 << 30;  // planes and partial sums of one product
-
 template <int BM, int BN, int WM, int WN, bool ROWMAX> int32_t launch_planes(PlaneArgs &p, int per_cu, hipStream_t st) {
     constexpr int smem = 2 * kPlanes * (BM + BN) * 64;
     auto kern = plane_gemm_kernel<BM, BN, WM, WN, ROWMAX>;
@@ -586,7 +584,7 @@ bool split_gemm_pays(int64_t m, int64_t n, int64_t k, bool fp32_direct) {
     // Under 1.5 GFLOP the fp32 path has its own small kernels and the launches decide: a 128 x 256 x 256 block would lose 26 us.
     if (m < 64 || n < 64 || k < 128 || 2.0 * m * n * k < 1.5e9 || m > (1 << 20) || n > (1 << 20) || k > (1 << 20) || m * n > ((int64_t)1 << 31)) return false;
     const Choice ch = choose(m, n, k, false);
-    if (scratch_bytes(m, n, k, ch) > kScratchBound) return false;
+    if (scratch_bytes(m, n, k, ch) > kStreamScratchMost) return false;
     // This path: the product, and the planes at 10 bytes an element, 4.5 TB/s and 3 us. The fp32 kernels: 130 TFLOP/s and 16 us
     // (whole-tile effects and the fix-up pass of a split K) with direct-to-LDS operands, 0.6 of that without.
     // us, fp32 -> split: 2331 x 768 x 768 44 -> 32, 768 x 768 x 2331 (A stored [k, m]) 62 -> 39, 4000 x 1024 x 1024 83 -> 55; where
@@ -597,12 +595,9 @@ bool split_gemm_pays(int64_t m, int64_t n, int64_t k, bool fp32_direct) {
 
 bool split_gemm(const SplitGemm &g, hipStream_t st, int32_t *rc) {
     const Choice ch = choose(g.m, g.n, g.k, g.rowmax != nullptr);
-    // The scratch belongs to the stream; the lock keeps another thread's product on the same stream from being queued between
-    // the planes and their reader.
-    static std::mutex *mu = new std::mutex();
-    std::lock_guard<std::mutex> lock(*mu);
-    void *scratch = nullptr;
-    if (!try_stream_workspace(st, scratch_bytes(g.m, g.n, g.k, ch), kSplitPlanes, &scratch)) return false;
+    StreamScratch lease;
+    void *scratch = lease.get(st, ScratchUse::SplitPlanes, scratch_bytes(g.m, g.n, g.k, ch));
+    if (!scratch) return false;
     *rc = run_split(g, ch, static_cast<unsigned char *>(scratch), st);
     return true;
 }

@@ -29,6 +29,7 @@
 
 #include "common.hpp"
 #include "pool.hpp"
+#include "stream_scratch.hpp"
 
 // ---------------------------------------------------------------------------------------------
 // Pool
@@ -109,6 +110,7 @@ void pool_stats(uint64_t *in_use, uint64_t *cached) {
 
 int32_t pool_trim() {
     if (!available()) return FTH_OK;
+    release_stream_scratch();
     Pool &p = pool();
     (void)hipDeviceSynchronize();
     std::lock_guard<std::mutex> lock(p.mu);
@@ -326,6 +328,7 @@ struct fth_encoder {
     Stack stack;
     std::map<GraphKey, hipGraphExec_t> graphs;
     std::vector<hipGraph_t> graph_templates;
+    std::vector<unsigned long long> captures;  // their ids: each owns the scratch its products were given
 };
 
 struct fth_gpt2 {
@@ -551,6 +554,7 @@ int32_t fth_encoder_free(fth_encoder *e) {
     if (fth::available()) (void)hipDeviceSynchronize();
     for (auto &kv : e->graphs) (void)hipGraphExecDestroy(kv.second);
     for (hipGraph_t g : e->graph_templates) (void)hipGraphDestroy(g);
+    for (unsigned long long id : e->captures) fth::release_capture_scratch(id);
     delete e;
     return FTH_OK;
 }
@@ -608,8 +612,8 @@ int32_t fth_encoder_forward_graph(fth_encoder *e, const float *x_dev, int64_t ba
         // One eager pass first: it sizes the workspaces and sets kernel attributes, neither of
         // which may happen while the stream is capturing. The capture itself records kernel
         // launches only (no memset nodes). The addresses recorded are the caller's two buffers,
-        // this encoder's own activations (owned until fth_encoder_free) and the stream's GEMM
-        // split-tile workspace, which is never released.
+        // this encoder's own activations and the scratch of this capture (both owned until
+        // fth_encoder_free) and the stream's GEMM split-tile workspace, which is never released.
         if (int32_t rc = fth_encoder_forward_dev(e, x_dev, batch, seq, out_dev, s)) return rc;
         FTH_HIP(hipStreamSynchronize(st));
         std::lock_guard<std::mutex> lock(e->stack.mu);
@@ -618,21 +622,28 @@ int32_t fth_encoder_forward_graph(fth_encoder *e, const float *x_dev, int64_t ba
             exec = it->second;
         } else {
             FTH_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+            const unsigned long long id = fth::capture_id(st);
             int32_t rc = e->stack.run(x_dev, batch, seq, out_dev, nullptr, s);
             hipGraph_t graph = nullptr;
             hipError_t ce = hipStreamEndCapture(st, &graph);
             if (rc) {
                 if (graph) (void)hipGraphDestroy(graph);
+                fth::release_capture_scratch(id);
                 return rc;
             }
-            if (ce != hipSuccess) return fth::hip_fail(ce, "hipStreamEndCapture");
+            if (ce != hipSuccess) {
+                fth::release_capture_scratch(id);
+                return fth::hip_fail(ce, "hipStreamEndCapture");
+            }
             hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
             if (ie != hipSuccess) {
                 (void)hipGraphDestroy(graph);
+                fth::release_capture_scratch(id);
                 return fth::hip_fail(ie, "hipGraphInstantiate");
             }
             e->graphs[key] = exec;
             e->graph_templates.push_back(graph);  // kept until fth_encoder_free, with its executable
+            e->captures.push_back(id);
         }
     }
     FTH_HIP(hipGraphLaunch(exec, st));

@@ -22,11 +22,12 @@
 // Semantics of sdpa_forward_f32 / sdpa_forward_masked_f64 (crates/ft-kernel-cpu/src/lib.rs:5200-5284, 4661-4741): scale after
 // the product, additive mask, softmax over all keys; a row with every key hidden is NaN.
 
-#include <mutex>
+#include <optional>
 #include <type_traits>
 
 #include "common.hpp"
 #include "sdpa_decode.hpp"
+#include "stream_scratch.hpp"
 
 namespace {
 
@@ -274,10 +275,11 @@ template <int D, int QT> int32_t launch(DecodeArgs &a, hipStream_t st, bool *don
     const int64_t units = a.d.num_bh / a.group * a.row_tiles;
     const int64_t grid = units * a.nsplit;
     if (grid > 2147483647LL) return FTH_OK;
+    std::optional<fth::StreamScratch> lease;  // until the merge is queued
     if (a.nsplit > 1) {
-        void *ws = nullptr;
         const int64_t slots = grid * ROWS;
-        if (!fth::try_stream_workspace(st, (size_t)(slots * (D + 2)) * sizeof(float), fth::kDecodeShares, &ws)) return FTH_OK;
+        void *ws = lease.emplace().get(st, fth::ScratchUse::DecodeShares, (size_t)(slots * (D + 2)) * sizeof(float));
+        if (!ws) return FTH_OK;
         a.part_o = static_cast<float *>(ws);
         a.part_ml = a.part_o + slots * D;
     }
@@ -328,9 +330,6 @@ bool sdpa_decode_f32(const fth_sdpa_desc &d, float scale, const float *q, const 
     want = want < 1 ? 1 : want > most ? most : want;
     a.tiles_per_split = (int)fth::ceil_div(tiles, want);
     a.nsplit = (int)fth::ceil_div(tiles, a.tiles_per_split);
-    // The scratch belongs to the stream; the lock keeps another thread's call on it from being queued before the merge.
-    static std::mutex *mu = new std::mutex();
-    std::lock_guard<std::mutex> lock(*mu);
     bool done = false;
     *rc = d.d_k == 128 ? launch_rows<128>(a, st, &done) : d.d_k == 64 ? launch_rows<64>(a, st, &done) : launch_rows<32>(a, st, &done);
     return done;

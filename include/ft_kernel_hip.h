@@ -126,10 +126,17 @@ int32_t fth_memcpy_d2d(void *dst_dev, const void *src_dev, size_t bytes);
 int32_t fth_memset_zero(void *dst_dev, size_t bytes);
 /* Free and total device memory in bytes as the driver reports them (hipMemGetInfo). */
 int32_t fth_device_memory_info(uint64_t *free_bytes, uint64_t *total_bytes);
-/* Device memory the GEMM unit holds for split-tile accumulators and transposed operands: `live_bytes` in the blocks in
- * use (one per stream and purpose, grown geometrically), `retired_bytes` in outgrown blocks that are kept because
- * queued kernels or a captured graph may still address them (less than `live_bytes` while no single request exceeds
- * 4 GiB). Either pointer may be NULL. The reference's CPU kernels keep no such state. */
+/* Device memory the library holds as workspaces of its own: `live_bytes` in the blocks in use, `retired_bytes` in outgrown
+ * blocks that are kept because queued kernels (or, for the first kind, a captured graph) may still address them. Two kinds:
+ *  - split-tile accumulators and transposed operands of fth_dev_gemm_*: one block per stream and purpose, grown
+ *    geometrically and never freed (retired blocks below `live_bytes` while no single request exceeds 4 GiB). A captured graph
+ *    records the stream's block: do not replay it beside products on the stream it was captured on.
+ *  - bf16 planes of large fp32 products and partial results of few-query attention: at most 1 GiB per stream and purpose and
+ *    less than as much again retired, all given back by fth_pool_trim. A capture gets blocks that nothing else uses, so its
+ *    graph may be replayed on any stream beside anything; the encoder's graphs give theirs back in fth_encoder_free, a
+ *    caller's own graphs hold theirs for good (4 GiB in all; past that, on hipStreamPerThread, and where memory is short, the
+ *    calls run kernels that need no such scratch, whose results differ in rounding).
+ * Either pointer may be NULL. The reference's CPU kernels keep no such state. */
 int32_t fth_device_workspace_info(uint64_t *live_bytes, uint64_t *retired_bytes);
 
 typedef void *fth_stream; /* a hipStream_t; NULL selects the library's own ordered stream */
@@ -681,8 +688,8 @@ int32_t fth_encoder_forward(fth_encoder *e, const float *input, int64_t batch, i
 int32_t fth_encoder_forward_dev(fth_encoder *e, const float *x_dev, int64_t batch, int64_t seq, float *out_dev, fth_stream s);
 /* Captures forward_dev for (x_dev, out_dev, batch, seq, s) into a HIP graph and replays it: one
  * launch per forward. The graph holds device addresses: the caller's two buffers must stay valid
- * while the encoder lives; the encoder's activations and the stream's GEMM split-tile workspace it
- * also records are never released before fth_encoder_free. Returns FTH_ERR_UNAVAILABLE while a
+ * while the encoder lives; the encoder's activations, the graph's own scratch and the stream's GEMM
+ * split-tile workspace it also records are not released before fth_encoder_free. Returns FTH_ERR_UNAVAILABLE while a
  * rocprofiler tool library is loaded in the process (trace the eager entry point instead). */
 int32_t fth_encoder_forward_graph(fth_encoder *e, const float *x_dev, int64_t batch, int64_t seq, float *out_dev, fth_stream s);
 
