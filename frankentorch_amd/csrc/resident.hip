@@ -80,7 +80,10 @@ int32_t pool_alloc(void **dptr, size_t bytes) {
             trim_locked(p);
             e = hipMalloc(&ptr, cls);
         }
-        if (e != hipSuccess) return hip_fail(e, "hipMalloc");
+        if (e != hipSuccess) {
+            (void)hipGetLastError();  // or the next launch check would report it
+            return hip_fail(e, "hipMalloc");
+        }
     }
     p.live[ptr] = cls;
     p.in_use += cls;

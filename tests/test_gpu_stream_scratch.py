@@ -175,6 +175,14 @@ def test_trim_gives_the_streams_blocks_back(hip):
     assert np.array_equal(_eager(hip, op, s), want)
 
 
+def test_a_refused_allocation_leaves_no_error_behind(hip):
+    t = C.c_void_p()
+    assert _lib.load().fth_tensor_alloc(C.c_int64(1 << 30), C.c_int64(1 << 20), C.byref(t)) != 0
+    x = DeviceBuffer.from_host(np.ones(1000, np.float32))
+    hip.add(x, x, x, 1000)  # its launch check would report the refusal
+    assert np.all(x.to_host() == 2.0)
+
+
 CHILD = """
 import sys
 sys.path[:0] = [%(root)r, %(root)r + "/tests"]
