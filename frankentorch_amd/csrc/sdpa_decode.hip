@@ -307,8 +307,10 @@ namespace fth {
 // seq_q <= 8: the larger tiles of csrc/sdpa.hip pad to 32 or 128 queries and read K and V once per query head. Measured at one
 // query they are 4 to 10 times slower.
 bool sdpa_decode_applies(const fth_sdpa_desc &d) {
-    return d.causal == 0 && d.seq_q <= 8 && d.seq_k > 0 && d.d_k == d.d_v && (d.d_k == 128 || d.d_k == 64 || d.d_k == 32) &&
-           d.seq_k * d.k_row_stride < ((int64_t)1 << 30) && d.seq_k * d.v_row_stride < ((int64_t)1 << 30);
+    // a head's K and V are addressed through unsigned 32-bit offsets, key numbers are ints with room for the last share
+    auto span_ok = [&](int64_t row_stride) { return row_stride >= 0 && d.seq_k * row_stride < ((int64_t)1 << 30); };
+    return d.causal == 0 && d.seq_q <= 8 && d.seq_k > 0 && d.seq_k <= ((int64_t)1 << 28) && d.d_k == d.d_v &&
+           (d.d_k == 128 || d.d_k == 64 || d.d_k == 32) && span_ok(d.k_row_stride) && span_ok(d.v_row_stride);
 }
 
 bool sdpa_decode_f32(const fth_sdpa_desc &d, float scale, const float *q, const float *k, const float *v, const float *mask,

@@ -49,3 +49,43 @@ def test_few_queries_against_a_cache(hip, oracle, shape, mask_kind):
         assert rel_err(got[ok], ref[ok]) <= TOL_GEMM_F32
     expanded = run(np.repeat(k, hq // hkv, axis=1), np.repeat(v, hq // hkv, axis=1), hq)
     assert np.array_equal(got.view(np.uint32), expanded.view(np.uint32))
+
+
+def _strided(hip, batch, hq, hkv, sq, sk, d, q, k, v, scale, mask=None):
+    """q, k, v are (buffer, batch stride, head stride, row stride, offset) in elements; the output is contiguous."""
+    from frankentorch_amd import _lib
+    a = _lib.SdpaDesc()
+    a.num_bh, a.heads, a.seq_q, a.seq_k, a.d_k, a.d_v = batch * hq, hq, sq, sk, d, d
+    for n, t in (("q", q), ("k", k), ("v", v)):
+        for f, x in zip(("batch", "head", "row"), t[1:4]):
+            setattr(a, "%s_%s_stride" % (n, f), x)
+    a.o_batch_stride, a.o_head_stride, a.o_row_stride = hq * sq * d, sq * d, d
+    a.causal, a.kv_group = 0, hq // hkv if hq != hkv else 0
+    out = DeviceBuffer.from_host(np.full((batch, hq, sq, d), 7.0, np.float32))
+    ptrs = [t[0].view(t[4]) for t in (q, k, v)]
+    if mask is None:
+        hip.sdpa_forward(a, scale, *ptrs, out)
+    else:
+        hip.sdpa_forward_masked(a, scale, *ptrs, DeviceBuffer.from_host(mask), 0, out)
+    return out.to_host()
+
+
+@pytest.mark.parametrize("sk", [1, 70, 300])
+@pytest.mark.parametrize("reverse", [False, True])
+def test_caches_as_they_lie_in_memory(hip, oracle, sk, reverse):
+    """Caches stored [batch, key, head, d] with room for more keys, read forwards and from the last key back (negative row
+    strides), beside NaN in everything that is not part of the problem."""
+    batch, hq, hkv, sq, d, room, pad = 2, 8, 4, 2, 64, 13, 8
+    q, k, v = (synth.normal(52, t, s) for t, s in (("q", (batch, hq, sq, d)), ("k", (batch, hkv, sk, d)), ("v", (batch, hkv, sk, d))))
+    row, bat = hkv * (d + pad), (sk + room) * hkv * (d + pad)
+    views = []
+    for t in (k, v):
+        store = np.full((batch, sk + room, hkv, d + pad), np.nan, np.float32)
+        store[:, :sk, :, :d] = t.transpose(0, 2, 1, 3)[:, ::-1] if reverse else t.transpose(0, 2, 1, 3)
+        views.append((DeviceBuffer.from_host(store), bat, d + pad, -row if reverse else row, (sk - 1) * row if reverse else 0))
+    qs = np.full((batch, sq, hq, d + 4), np.nan, np.float32)
+    qs[..., :d] = q.transpose(0, 2, 1, 3)
+    qv = (DeviceBuffer.from_host(qs), sq * hq * (d + 4), d + 4, hq * (d + 4), 0)
+    got = _strided(hip, batch, hq, hkv, sq, sk, d, qv, *views, np.float32(0.125))
+    ref = oracle.sdpa_forward_masked_gqa(q, k, v, np.float32(0.125), np.zeros((sq, sk), np.float32))
+    assert rel_err(got, ref) <= TOL_GEMM_F32
