@@ -1142,9 +1142,10 @@ int32_t sdpa_entry(const fth_sdpa_desc *d, double scale, const T *q, const T *k,
                 if (d->d_k == 64) return launch_small_sdpa<64>(a, st);  // (128: the merge buffers would exceed 64 KiB of LDS)
                 if (d->d_k == 32) return launch_small_sdpa<32>(a, st);
             }
-            if (d->d_k == 128) return launch_mfma<128>(a, st);
-            if (d->d_k == 64) return launch_mfma<64>(a, st);
-            if (d->d_k == 32) return launch_mfma<32>(a, st);
+            const bool forwards = d->k_row_stride >= 0 && d->v_row_stride >= 0;  // a tile's lane offsets are unsigned
+            if (forwards && d->d_k == 128) return launch_mfma<128>(a, st);
+            if (forwards && d->d_k == 64) return launch_mfma<64>(a, st);
+            if (forwards && d->d_k == 32) return launch_mfma<32>(a, st);
         }
     }
     if constexpr (std::is_same<T, double>::value) {
@@ -1158,7 +1159,7 @@ int32_t sdpa_entry(const fth_sdpa_desc *d, double scale, const T *q, const T *k,
             return e && std::atoi(e) != 0;
         }();
         // (the tile loads address a head's K and V through 32-bit byte offsets)
-        const bool span_ok = (d->seq_k + 16) * d->k_row_stride < ((int64_t)1 << 28) && (d->seq_k + 16) * d->v_row_stride < ((int64_t)1 << 28);
+        const bool span_ok = d->k_row_stride >= 0 && d->v_row_stride >= 0 && (d->seq_k + 16) * d->k_row_stride < ((int64_t)1 << 28) && (d->seq_k + 16) * d->v_row_stride < ((int64_t)1 << 28);
         if (strides_ok && span_ok && d->d_k == d->d_v && d->seq_k > 0 && !generic_only) {
             if (d->d_k == 128) return launch_mfma_f64<128>(a, st);
             if (d->d_k == 64) return launch_mfma_f64<64>(a, st);

@@ -51,7 +51,7 @@ def test_few_queries_against_a_cache(hip, oracle, shape, mask_kind):
     assert np.array_equal(got.view(np.uint32), expanded.view(np.uint32))
 
 
-def _strided(hip, batch, hq, hkv, sq, sk, d, q, k, v, scale, mask=None):
+def _strided(hip, batch, hq, hkv, sq, sk, d, q, k, v, scale, mask=None, dtype=np.float32):
     """q, k, v are (buffer, batch stride, head stride, row stride, offset) in elements; the output is contiguous."""
     from frankentorch_amd import _lib
     a = _lib.SdpaDesc()
@@ -61,7 +61,7 @@ def _strided(hip, batch, hq, hkv, sq, sk, d, q, k, v, scale, mask=None):
             setattr(a, "%s_%s_stride" % (n, f), x)
     a.o_batch_stride, a.o_head_stride, a.o_row_stride = hq * sq * d, sq * d, d
     a.causal, a.kv_group = 0, hq // hkv if hq != hkv else 0
-    out = DeviceBuffer.from_host(np.full((batch, hq, sq, d), 7.0, np.float32))
+    out = DeviceBuffer.from_host(np.full((batch, hq, sq, d), 7.0, dtype))
     ptrs = [t[0].view(t[4]) for t in (q, k, v)]
     if mask is None:
         hip.sdpa_forward(a, scale, *ptrs, out)
@@ -89,3 +89,15 @@ def test_caches_as_they_lie_in_memory(hip, oracle, sk, reverse):
     got = _strided(hip, batch, hq, hkv, sq, sk, d, qv, *views, np.float32(0.125))
     ref = oracle.sdpa_forward_masked_gqa(q, k, v, np.float32(0.125), np.zeros((sq, sk), np.float32))
     assert rel_err(got, ref) <= TOL_GEMM_F32
+
+
+@pytest.mark.parametrize("sq,d,masked,dtype", [(2, 64, True, np.float32), (70, 128, False, np.float32), (70, 64, True, np.float32), (70, 64, False, np.float64)])
+def test_a_cache_read_backwards_on_the_other_kernels(hip, oracle, sq, d, masked, dtype):
+    """Negative row strides where the tiled kernels' unsigned lane offsets cannot go: the general kernel answers."""
+    batch, hq, hkv, sk = 1, 4, 2, 77
+    q, k, v = (synth.normal(53, t, s, dtype=dtype) for t, s in (("q", (batch, hq, sq, d)), ("k", (batch, hkv, sk, d)), ("v", (batch, hkv, sk, d))))
+    views = [(DeviceBuffer.from_host(np.ascontiguousarray(t[:, :, ::-1])), hkv * sk * d, sk * d, -d, (sk - 1) * d) for t in (k, v)]
+    mask = synth.normal(53, "m", (sq, sk), 0.0, 0.5, dtype=dtype) if masked else None
+    got = _strided(hip, batch, hq, hkv, sq, sk, d, (DeviceBuffer.from_host(q), hq * sq * d, sq * d, d, 0), *views, dtype(0.125), mask, dtype)
+    ref = oracle.sdpa_forward_masked_gqa(q, k, v, dtype(0.125), mask if masked else np.zeros((sq, sk), dtype))
+    assert rel_err(got, ref) <= (TOL_GEMM_F32 if dtype == np.float32 else 1e-12)
