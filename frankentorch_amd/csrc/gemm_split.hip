@@ -15,11 +15,12 @@
 // split again by each tile that reads it, and the loop stayed at 190-230 TFLOP/s (of fp32 products) where this one reaches
 // 240-263.
 //
-// What the split cannot represent is found in the results. Operands of 2^24 and more, infinities, NaN and non-zero ones of
-// 2^-134 and less (which would vanish) are written as NaN planes and leave NaN sums. Operands under 2^-109 lose their lowest
-// bits, 2^-134 each at most; beside a partner under 2^24 that is 2^-110 per product, which can matter only in a sum under
-// 2^-70. A wavefront that holds a non-finite sum or a non-zero one under 2^-70 computes its part of the tile again from the
-// fp32 operands on fp32 MFMAs.
+// What the split cannot stand for is found in the results. Non-zero operands under 2^-110, whose third part would lie below the
+// bf16 subnormals, operands of 2^53 and more, whose sums of up to 2^20 products could overflow where fp32 arithmetic does not,
+// infinities and NaN are written as NaN planes and leave NaN sums; every other operand is exactly the sum of its parts. In
+// a sum under 2^-100 products of the lower parts may have been rounded at the end of the fp32 range (the matrix unit keeps
+// subnormals, measured). A wavefront that holds a NaN or a non-zero sum under 2^-100 computes its part of the tile again from
+// the fp32 operands on fp32 MFMAs.
 //
 // replaces gemm::sgemm / sgemm_bt / sgemm_tb (crates/ft-kernel-cpu/src/lib.rs:1310-1338, 1430-1524) for large products.
 
@@ -38,8 +39,8 @@ constexpr int kGroupM = 8;
 constexpr int kBK = 32;       // k of a K-tile: one 16 x 16 x 32 MFMA
 constexpr int kPlanes = 3;
 constexpr int kBlock = 1024;  // bytes of one plane of 16 rows x 32 k
-constexpr float kTiny = 0x1p-70f;
-constexpr uint32_t kTooLarge = 0x4b800000u, kTooSmall = 0x00008000u;  // bits of 2^24 and of 2^-134
+constexpr float kTiny = 0x1p-100f;
+constexpr uint32_t kTooLarge = 0x5a000000u, kTooSmall = 0x08800000u;  // bits of 2^53 and of 2^-110
 
 using bf16x8 = __attribute__((ext_vector_type(8))) __bf16;
 using bf16x2 = __attribute__((ext_vector_type(2))) __bf16;
@@ -58,7 +59,7 @@ __device__ __forceinline__ float hi_f32(uint32_t p) { return __builtin_bit_cast(
 // NaN in the place of a float that the parts cannot stand for.
 __device__ __forceinline__ float representable(float x) {
     const uint32_t u = __builtin_bit_cast(uint32_t, x) & 0x7fffffffu;
-    return u >= kTooLarge || u - 1u < kTooSmall ? __builtin_nanf("") : x;
+    return u >= kTooLarge || u - 1u < kTooSmall - 1u ? __builtin_nanf("") : x;  // (zero wraps round)
 }
 
 // The three parts of two floats, one dword each.
@@ -339,7 +340,7 @@ __global__ __launch_bounds__(WM *WN *kWave, 2) void plane_gemm_kernel(const Plan
                     big = nan_max(big, __builtin_fabsf(acc[i][j][e]));
                     small = __builtin_fminf(small, __builtin_fabsf(acc[i][j][e]));
                 }
-        if (__builtin_amdgcn_ballot_w64(!(big <= FLT_MAX) || small < kTiny)) {  // rare: look closer (an exact zero is nothing to worry about)
+        if (__builtin_amdgcn_ballot_w64(!(big <= FLT_MAX) || small < kTiny)) {  // rare: look closer (exact zeros are exact)
             bool doubt = !(big <= FLT_MAX);
 #pragma unroll
             for (int i = 0; i < TM; ++i)

@@ -88,7 +88,8 @@ def test_split_product_values_the_parts_cannot_hold(hip):
     assert got[1000, 1500] == np.float32(np.finfo(np.float32).max) * np.float32(0.5)
 
 
-@pytest.mark.parametrize("small,large", [(-120, 60), (-128, 20), (-140, 40), (-100, 23)])
+# either side of the limits on operands (2^-110 and 2^53) and on sums (2^-100)
+@pytest.mark.parametrize("small,large", [(-120, 60), (-128, 20), (-140, 40), (-100, 23), (0, 25), (3, 48), (0, 53), (-105, 48), (-60, -45), (-104, 0)])
 def test_split_product_small_beside_large(hip, small, large):
     """A row whose low bits (or all of them) lie below the bf16 subnormals, times columns large enough to bring the sums back:
     the same bound as for ordinary operands (the sums of a subnormal row too: its floats are exact)."""
@@ -102,6 +103,21 @@ def test_split_product_small_beside_large(hip, small, large):
         ref = a[rows].astype(np.float64) @ b[cols].T.astype(np.float64)
         floor = np.sqrt(ref.size) * 2.0 ** -126  # results that are subnormal themselves
         assert np.linalg.norm(got[rows, cols] - ref) <= _bound(k) * np.linalg.norm(ref) + floor
+
+
+def test_split_product_cancelling_to_the_lowest_bits(hip):
+    """Two products that cancel but for bits far below bf16's: what is left is the exact difference, for operands small enough
+    that their lower parts are subnormal too."""
+    m, n, k = 2048, 2304, 768
+    a, b = np.zeros((m, k), np.float32), np.zeros((n, k), np.float32)
+    cases = [(2.0 ** -130, 2.0 ** -5, 2.0 ** 23), (2.0 ** -130, 2.0 ** -5, 2.0 ** 40), (2.0 ** -109, 2.0 ** -23, 2.0 ** 40), (2.0 ** -112, 2.0 ** -20, 2.0 ** 20),
+             (1.0, 2.0 ** -23, 1.0), (2.0 ** 40, 2.0 ** -23, 2.0 ** -20)]
+    for i, (x, d, y) in enumerate(cases):
+        a[5 + 70 * i, 0], a[5 + 70 * i, 41] = x * (1 + d), -x
+        b[7 + 70 * i, 0] = b[7 + 70 * i, 41] = y
+    got = _gemm(hip, m, n, k, a, b, trans_b=True)
+    for i, (x, d, y) in enumerate(cases):
+        assert got[5 + 70 * i, 7 + 70 * i] == np.float32(x * d * y), (i, x, d, y)
 
 
 def test_split_product_is_repeatable_and_padding_is_not_read_into_it(hip):
