@@ -2,12 +2,17 @@
 //
 // A float has 24 significant bits; three bf16 values hold 8 each. Rounding to nearest three times, x = x0 + x1 + x2 EXACTLY
 // (x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1, which has at most 8 significant bits left), so nothing of an operand
-// is given up. Of the nine products of two such sums six are formed, x0 y0, x0 y1, x1 y0, x1 y1, x0 y2, x2 y0, each exact in
-// the matrix unit and summed in fp32; the three left out are below 2^-24 |x y| together and of either sign (root mean square
-// 2^-26 |x y|). Six bf16 MFMAs of 32 k cost 96 cycles where the fp32 MFMAs cost 256. The sum is rounded 6 times per 32 k
-// instead of 8 times or more, which is why the result is closer to the exact one than the fp32 MFMA kernel's: relative
-// 2-norm error against 64-bit sums, normal operands, K 768 / 3072 / 4096: 4.2e-7 / 8.6e-7 / 1.00e-6 here, 4.95e-7 / 9.9e-7 /
-// 1.15e-6 there.
+// is given up. Of the nine products of two such sums six are formed, x0 y0, x0 y1, x1 y0, x1 y1, x0 y2, x2 y0, and summed in
+// fp32; the three left out are below 2^-24 |x y| together and of either sign. Six bf16 MFMAs of 32 k cost 96 cycles where the
+// fp32 MFMAs cost 256. x0 y0 has an accumulator of its own: the other five are 2^-8 of it and less, and each of them added to
+// the full sum would round that sum again (several times an MFMA, which adds in groups), so they are kept apart until the end
+// of the tile. Relative 2-norm error against 64-bit sums, this kernel / the fp32 MFMA kernel:
+//   normal operands, K 768, 3072, 4096, 50257: 1.6e-7 / 4.95e-7, 3.4e-7 / 9.9e-7, 4.0e-7 / 1.15e-6, 3.5e-7 / 1.7e-6
+//   of one sign (uniform), the same K:         1.5e-7 / 4.2e-7,  3.0e-7 / 8.3e-7, 3.0e-7 / 8.4e-7,  1.0e-7 / 6.1e-7
+//   ReLU of normal, the same K:                1.2e-7 / 3.5e-7,  2.7e-7 / 7.0e-7, 3.2e-7 / 8.1e-7,  2.9e-7 / 1.2e-6
+// (With one accumulator for all six: 4.2e-7 / 8.6e-7 / 1.00e-6 / 1.1e-6 on normal operands, and worse than the fp32 kernel by a
+// sixth on ReLU ones.) A sum of a single non-zero product is the one place where the left-out terms show: 2.6e-8 / 2.5e-8, the
+// largest error 1.7 / 1.0 units of 2^-24.
 //
 // Two passes. split_kernel writes an operand's three planes once, in the order in which the product
 // reads them; the product then moves planes to LDS with direct loads and has no vector arithmetic in its loop. Splitting
@@ -151,18 +156,18 @@ struct PlaneArgs {
     int ktiles;              // of the whole product
     int splits, kt_per;      // the K-tiles are cut into `splits` runs of kt_per (the last one shorter)
     int tiles_m, tiles_n;
-    int64_t tiles;
+    int tiles;
     float *partial;          // splits > 1: [splits][m][n] sums without epilogue
     int order;               // tile order inside a group of tile rows, as in the fp32 kernel: 1 walks along the rows of C
     int64_t rowmax_groups;
 };
 
-__device__ __forceinline__ void tile_of_id(int64_t id, int tiles_m, int tiles_n, int order, int &tm, int &tn) {
-    const int64_t group = (int64_t)kGroupM * tiles_n;
-    const int64_t g = id / group;
-    const int first_m = (int)(g * kGroupM);
+__device__ __forceinline__ void tile_of_id(int id, int tiles_m, int tiles_n, int order, int &tm, int &tn) {
+    const int group = kGroupM * tiles_n;
+    const int g = id / group;
+    const int first_m = g * kGroupM;
     const int gm = (tiles_m - first_m) < kGroupM ? (tiles_m - first_m) : kGroupM;
-    const int in_g = (int)(id - g * group);
+    const int in_g = id - g * group;
     tm = first_m + (order ? in_g / tiles_n : in_g % gm);
     tn = order ? in_g % tiles_n : in_g / gm;
 }
@@ -224,20 +229,20 @@ __global__ __launch_bounds__(WM *WN *kWave, 2) void plane_gemm_kernel(const Plan
     const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)reinterpret_cast<uintptr_t>(smem));
     const int grid = (int)gridDim.x;
     const int vb = xcd_contiguous_id((int)blockIdx.x, grid);
-    const int64_t items = p.tiles * p.splits;
+    const int items = p.tiles * p.splits;
     if (vb >= items) return;
 
-    auto run_of = [&](int64_t item, int &first) __attribute__((always_inline)) {
-        const int s = (int)(item / p.tiles);
+    auto run_of = [&](int item, int &first) __attribute__((always_inline)) {
+        const int s = item / p.tiles;
         first = s * p.kt_per;
         const int rest = p.ktiles - first;
         return rest < p.kt_per ? rest : p.kt_per;
     };
     // ---- loader: one K-tile ahead of the operand reads ----
-    int64_t ld_item = vb;
+    int ld_item = vb;
     int ld_left = 0;  // K-tiles of ld_item still to request
     const unsigned char *ak = nullptr, *bk = nullptr;
-    unsigned a_off[LA], b_off[LB];
+    unsigned a_off[LA], b_off[LB];  // byte offsets of this wavefront's blocks (uniform)
     const int64_t a_step = (int64_t)p.a_blocks * kPlanes * kBlock, b_step = (int64_t)p.b_blocks * kPlanes * kBlock;
     auto setup = [&]() __attribute__((always_inline)) {
         int tm, tn, first;
@@ -250,14 +255,14 @@ __global__ __launch_bounds__(WM *WN *kWave, 2) void plane_gemm_kernel(const Plan
             const int c = i * NW + wave;
             int blk = tm * (BM / 16) + c % (BM / 16);
             blk = blk < p.a_blocks ? blk : p.a_blocks - 1;
-            a_off[i] = (unsigned)(c / (BM / 16) * p.a_blocks + blk) * (unsigned)kBlock + lane * 16u;
+            a_off[i] = (unsigned)(c / (BM / 16) * p.a_blocks + blk) * (unsigned)kBlock;
         }
 #pragma unroll
         for (int i = 0; i < LB; ++i) {
             const int c = i * NW + wave;
             int blk = tn * (BN / 16) + c % (BN / 16);
             blk = blk < p.b_blocks ? blk : p.b_blocks - 1;
-            b_off[i] = (unsigned)(c / (BN / 16) * p.b_blocks + blk) * (unsigned)kBlock + lane * 16u;
+            b_off[i] = (unsigned)(c / (BN / 16) * p.b_blocks + blk) * (unsigned)kBlock;
         }
     };
     const unsigned wdst = lds0 + (unsigned)wave * kBlock;
@@ -265,10 +270,10 @@ __global__ __launch_bounds__(WM *WN *kWave, 2) void plane_gemm_kernel(const Plan
         if (ld_left == 0) return;  // past the last K-tile of this workgroup
 #pragma unroll
         for (int i = 0; i < LA; ++i)
-            if (A_CH % NW == 0 || i + 1 < LA || i * NW + wave < A_CH) load_to_lds_16(ak, a_off[i], wdst + buf * BUF + i * NW * kBlock);
+            if (A_CH % NW == 0 || i + 1 < LA || i * NW + wave < A_CH) load_to_lds_16(ak + a_off[i], lane * 16u, wdst + buf * BUF + i * NW * kBlock);
 #pragma unroll
         for (int i = 0; i < LB; ++i)
-            if (B_CH % NW == 0 || i + 1 < LB || i * NW + wave < B_CH) load_to_lds_16(bk, b_off[i], wdst + buf * BUF + (A_CH + i * NW) * kBlock);
+            if (B_CH % NW == 0 || i + 1 < LB || i * NW + wave < B_CH) load_to_lds_16(bk + b_off[i], lane * 16u, wdst + buf * BUF + (A_CH + i * NW) * kBlock);
         ak += a_step;
         bk += b_step;
         if (--ld_left == 0) {
@@ -286,23 +291,23 @@ __global__ __launch_bounds__(WM *WN *kWave, 2) void plane_gemm_kernel(const Plan
 #pragma unroll
         for (int j = 0; j < TN; ++j) f.b[j] = *reinterpret_cast<const bf16x8 *>(s0 + s * BN * 64 + b_rd + j * kBlock);
     };
-    f32x4 acc[TM][TN];
-    auto mul = [&](const Frag &fa, const Frag &fb) __attribute__((always_inline)) {
+    f32x4 acc[TM][TN], low[TM][TN];  // sums of x0 y0, and of the five products with a lower part
+    auto mul = [&](f32x4 (&to)[TM][TN], const Frag &fa, const Frag &fb) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb.b[j], fa.a[i], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < TN; ++j) to[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb.b[j], fa.a[i], to[i][j], 0, 0, 0);
     };
-    auto zero = [&]() __attribute__((always_inline)) {
+    auto zero = [&](f32x4 (&to)[TM][TN]) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < TN; ++j) to[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     };
 
     // This wavefront's part of a tile again, from the fp32 operands.
-    auto again = [&](int64_t m0, int64_t n0, int first, int nk) __attribute__((always_inline)) {
-        zero();
+    auto again = [&](int64_t m0, int64_t n0, int first, int nk, int l16, int lq) __attribute__((always_inline)) {
+        zero(acc);
         const fth::SplitGemm &g = p.g;
         const int64_t k_end = (int64_t)(first + nk) * kBK < g.k ? (int64_t)(first + nk) * kBK : g.k;
         for (int64_t k0 = (int64_t)first * kBK; k0 < k_end; k0 += 16) {
@@ -326,10 +331,17 @@ __global__ __launch_bounds__(WM *WN *kWave, 2) void plane_gemm_kernel(const Plan
         }
     };
 
-    auto finish = [&](int64_t item, int first, int nk) __attribute__((always_inline)) {
+    auto finish = [&](int item, int first, int nk) __attribute__((always_inline)) {
+        int at = lane;
+        asm volatile("" : "+v"(at));  // nothing of the output's addresses is worked out ahead of the loop and held through it
+        const int l16 = at & 15, lq = at >> 4;
         int tm, tn;
         tile_of_id(item % p.tiles, p.tiles_m, p.tiles_n, p.order, tm, tn);
         const int64_t m0 = (int64_t)tm * BM + wm0, n0 = (int64_t)tn * BN + wn0;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] += low[i][j];
         float big = 0.f, small = FLT_MAX;
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -348,11 +360,11 @@ __global__ __launch_bounds__(WM *WN *kWave, 2) void plane_gemm_kernel(const Plan
                 for (int j = 0; j < TN; ++j)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) doubt = doubt || (acc[i][j][e] != 0.f && __builtin_fabsf(acc[i][j][e]) < kTiny);
-            if (__builtin_amdgcn_ballot_w64(doubt)) again(m0, n0, first, nk);
+            if (__builtin_amdgcn_ballot_w64(doubt)) again(m0, n0, first, nk, l16, lq);
         }
         const int64_t m = p.g.m, n = p.g.n;
         const bool parts = p.splits > 1;
-        float *c = parts ? p.partial + (item / p.tiles) * m * n : p.g.c;
+        float *c = parts ? p.partial + (int64_t)(item / p.tiles) * m * n : p.g.c;
         const int64_t ldc = parts ? n : p.g.ldc;
         if (!parts) {
             if (p.g.alpha != 1.f) {
@@ -424,49 +436,49 @@ __global__ __launch_bounds__(WM *WN *kWave, 2) void plane_gemm_kernel(const Plan
         }
     };
 
-    Frag f0, f1, g1, g2;
-    int64_t item = vb;
-    int first = 0, nk = __builtin_amdgcn_readfirstlane(run_of(item, first)), kt = 0;
-    zero();
+    Frag f0, f1, f2;  // this K-tile's operands by plane
+    auto fetch_all = [&](int buf) __attribute__((always_inline)) {
+        fetch(f1, buf, 1);
+        fetch(f0, buf, 0);
+        fetch(f2, buf, 2);
+    };
+    // One K-tile. The next K-tile's own loads have landed behind the wait, everyone's behind the barrier, and everyone has this
+    // K-tile's operands in registers. After the last K-tile of a tile the reads fetch what is left there.
+    auto step = [&](int buf) __attribute__((always_inline)) {
+        mul(low, f1, f1);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+        __syncthreads();
+        issue(buf);
+        mul(low, f1, f0);
+        mul(low, f0, f1);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(f1, buf ^ 1, 1);
+        mul(low, f2, f0);
+        mul(low, f0, f2);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(f2, buf ^ 1, 2);
+        mul(acc, f0, f0);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(f0, buf ^ 1, 0);
+    };
+    int buf = 0;
     setup();
     issue(0);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): own part landed
     __syncthreads();
     issue(1);
-    fetch(f0, 0, 0);
-    fetch(g1, 0, 1);
-    fetch(g2, 0, 2);
-    // One K-tile; false when it was the last one. The next K-tile's own loads have landed behind the wait, everyone's behind the
-    // barrier, and everyone has this K-tile's operands in registers. After the last K-tile the reads fetch what is left there.
-    auto step = [&](int buf, const Frag &cur, Frag &nxt) __attribute__((always_inline)) {
-        __builtin_amdgcn_s_waitcnt(0x0F70);
-        __syncthreads();
-        issue(buf);
-        mul(cur, g2);
-        mul(g2, cur);
-        __builtin_amdgcn_sched_barrier(0);
-        fetch(g2, buf ^ 1, 2);
-        fetch(nxt, buf ^ 1, 0);
-        mul(g1, g1);
-        mul(g1, cur);
-        mul(cur, g1);
-        __builtin_amdgcn_sched_barrier(0);
-        fetch(g1, buf ^ 1, 1);
-        mul(cur, cur);
-        __builtin_amdgcn_sched_barrier(0);
-        if (++kt < nk) return true;
+    for (int item = vb; item < items; item += grid) {
+        int first;
+        const int nk = __builtin_amdgcn_readfirstlane(run_of(item, first));
+        zero(acc);
+        zero(low);
+        fetch_all(buf);  // (nothing of the next tile is held in registers across the output)
+        for (int kt = 0; kt < nk; ++kt) {
+            step(buf);
+            buf ^= 1;
+        }
         finish(item, first, nk);
-        item += grid;
-        if (item >= items) return false;
-        nk = __builtin_amdgcn_readfirstlane(run_of(item, first));
-        kt = 0;
-        zero();
-        fetch(nxt, buf ^ 1, 0);  // again: nothing of the next tile is held in registers across the output
-        fetch(g1, buf ^ 1, 1);
-        fetch(g2, buf ^ 1, 2);
-        return true;
-    };
-    while (step(0, f0, f1) && step(1, f1, f0)) {
     }
 }
 
@@ -529,7 +541,7 @@ template <int BM, int BN, int WM, int WN, bool ROWMAX> int32_t launch_planes(Pla
     FTH_HIP(ready);
     p.tiles_m = (int)fth::ceil_div(p.g.m, BM);
     p.tiles_n = (int)fth::ceil_div(p.g.n, BN);
-    p.tiles = (int64_t)p.tiles_m * p.tiles_n;
+    p.tiles = p.tiles_m * p.tiles_n;  // (m n is at most 2^31)
     p.order = p.tiles_n > p.tiles_m ? 1 : 0;
     const int64_t slots = (int64_t)(fth::compute_units() > 0 ? fth::compute_units() : 256) * per_cu, items = p.tiles * p.splits;
     kern<<<dim3((unsigned)(items < slots ? items : slots)), dim3(WM * WN * kWave), smem, st>>>(p);
