@@ -196,13 +196,13 @@ __device__ __forceinline__ float gelu_tanh(float x) {
     return x / (1.0f + __builtin_amdgcn_exp2f(u * -2.8853900817779268f));
 }
 
-// Four k of one operand row for the fp32 MFMAs, zero beyond the operand's k.
-__device__ __forceinline__ f32x4 four_k(const float *row, int64_t ks, int64_t k0, int64_t k_end) {
+// Four k of one operand row for the fp32 MFMAs: the first `left` of them from p on, ks apart, the others zero.
+__device__ __forceinline__ f32x4 four_k(const float *p, int64_t ks, int left) {
+    if (ks == 1 && left >= 4) return *reinterpret_cast<const f32x4_any *>(p);
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if (ks == 1 && k0 + 4 <= k_end) return *reinterpret_cast<const f32x4_any *>(row + k0);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-        if (k0 + e < k_end) v[e] = row[(k0 + e) * ks];
+        if (e < left) v[e] = p[e * ks];
     return v;
 }
 
@@ -305,29 +305,53 @@ __global__ __launch_bounds__(WM *WN *kWave, 2) void plane_gemm_kernel(const Plan
             for (int j = 0; j < TN; ++j) to[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     };
 
-    // This wavefront's part of a tile again, from the fp32 operands.
+    // This wavefront's part of a tile again, from the fp32 operands. us, fp32 kernels / here with one NaN in A / with every sum
+    // computed again: 4096^3 935 / 930 / 1690, 8192 x 3072 x 768 284 / 234 / 481, 2331 x 768 x 768 40 / 74 / 72 (a tile's second
+    // pass is a chain of its own K on one wavefront).
     auto again = [&](int64_t m0, int64_t n0, int first, int nk, int l16, int lq) __attribute__((always_inline)) {
         zero(acc);
         const fth::SplitGemm &g = p.g;
-        const int64_t k_end = (int64_t)(first + nk) * kBK < g.k ? (int64_t)(first + nk) * kBK : g.k;
-        for (int64_t k0 = (int64_t)first * kBK; k0 < k_end; k0 += 16) {
-            f32x4 av[TM];
+        const int k_first = first * kBK + lq * 4;
+        int left = (int)((first + nk) * kBK < g.k ? (first + nk) * kBK : g.k) - k_first;  // k of this lane's row pieces still to load
+        const float *pa[TM], *pb[TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const int64_t row = m0 + i * 16 + l16;
+            pa[i] = g.a + (row < g.m ? row : g.m - 1) * g.a_rs + k_first * g.a_ks;
+        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int64_t col = n0 + j * 16 + l16;
+            pb[j] = g.b + (col < g.n ? col : g.n - 1) * g.b_rs + k_first * g.b_ks;
+        }
+        f32x4 av[TM], bv[TN];
+        auto load = [&]() __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
-                int64_t row = m0 + i * 16 + l16;
-                row = row < g.m ? row : g.m - 1;
-                av[i] = four_k(g.a + row * g.a_rs, g.a_ks, k0 + lq * 4, k_end);
+                av[i] = four_k(pa[i], g.a_ks, left);
+                pa[i] += 16 * g.a_ks;
             }
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
-                int64_t col = n0 + j * 16 + l16;
-                col = col < g.n ? col : g.n - 1;
-                const f32x4 bv = four_k(g.b + col * g.b_rs, g.b_ks, k0 + lq * 4, k_end);
+                bv[j] = four_k(pb[j], g.b_ks, left);
+                pb[j] += 16 * g.b_ks;
+            }
+            left -= 16;
+        };
+        load();
+        for (int it = 0; it < 2 * nk; ++it) {  // 16 k at a time, the next ones requested ahead of this one's MFMAs
+            f32x4 ma[TM], mb[TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) ma[i] = av[i];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) mb[j] = bv[j];
+            load();
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[e], av[i][e], acc[i][j], 0, 0, 0);
-            }
+                    for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(mb[j][e], ma[i][e], acc[i][j], 0, 0, 0);
         }
     };
 
