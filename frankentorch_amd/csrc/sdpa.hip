@@ -1122,23 +1122,24 @@ int32_t sdpa_entry(const fth_sdpa_desc *d, double scale, const T *q, const T *k,
                                 m4(d->o_batch_stride) && m4(d->o_head_stride) && m4(d->o_row_stride) &&
                                 al16(q) && al16(k) && al16(v) && al16(out) &&
                                 d->k_row_stride < (1 << 22) && d->v_row_stride < (1 << 22);  // a tile's lane offsets fit 32 bits
+        // Too few 32-query blocks to give every compute unit one: the key-split kernel (one launch, no LDS staging)
+        static const int small_knob = [] {
+            const char *e = std::getenv("FT_HIP_SDPA_SMALL");  // tuning knob: 0 disables the small-problem kernel, 2 forces it
+            return e ? std::atoi(e) : 1;
+        }();
+        const int cus = fth::compute_units() > 0 ? fth::compute_units() : 256;
+        const bool small_takes = !masked && scale > T(0) && small_knob != 0 && (small_knob == 2 || d->num_bh * fth::ceil_div(d->seq_q, 32) <= cus) &&
+                                 d->seq_k <= 4096 && d->d_k == d->d_v && (d->d_k == 64 || d->d_k == 32);
         // Few queries against a cache: the kernels below pad them to 32 or 128 query rows and read K and V once per query head.
         int32_t rc = FTH_OK;
-        if (strides_ok && fth::sdpa_decode_applies(*d) &&
+        if (strides_ok && fth::sdpa_decode_applies(*d, small_takes) &&
             fth::sdpa_decode_f32(*d, (float)scale, reinterpret_cast<const float *>(q), reinterpret_cast<const float *>(k),
                                  reinterpret_cast<const float *>(v), reinterpret_cast<const float *>(a.mask), mask_bh_stride,
-                                 reinterpret_cast<float *>(out), st, &rc))
+                                 reinterpret_cast<float *>(out), small_takes, st, &rc))
             return rc;
         // the unmasked MFMA kernels take the row maximum on the raw scores, which needs a positive scale
         if (strides_ok && d->d_k == d->d_v && d->seq_k > 0 && (masked || scale > T(0))) {
-            // Too few 32-query blocks to give every compute unit one: the key-split kernel (one launch, no LDS staging)
-            static const int small_knob = [] {
-                const char *e = std::getenv("FT_HIP_SDPA_SMALL");  // tuning knob: 0 disables the small-problem kernel, 2 forces it
-                return e ? std::atoi(e) : 1;
-            }();
-            const bool small_off = small_knob == 0;
-            const int cus = fth::compute_units() > 0 ? fth::compute_units() : 256;
-            if (!masked && !small_off && (small_knob == 2 || d->num_bh * fth::ceil_div(d->seq_q, 32) <= cus) && d->seq_k <= 4096) {
+            if (small_takes) {
                 if (d->d_k == 64) return launch_small_sdpa<64>(a, st);  // (128: the merge buffers would exceed 64 KiB of LDS)
                 if (d->d_k == 32) return launch_small_sdpa<32>(a, st);
             }

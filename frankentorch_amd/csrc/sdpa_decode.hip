@@ -12,8 +12,8 @@
 //   * the K loads of the next tile are issued as soon as the scores have consumed this one's, the V loads before the scores,
 //     so both are in flight under the softmax;
 //   * the shares of a row are merged by a second small kernel in key order (partial maximum, sum and unnormalised output).
-// The number of shares depends on (num_bh, seq_k) alone -- not on how many query heads share a K/V head -- so a grouped call
-// and the same call on repeated K/V heads give the same bits.
+// The number of shares depends on (num_bh, seq_k), the head size and whether there is a mask -- not on how many query heads
+// share a K/V head -- so a grouped call and the same call on repeated K/V heads give the same bits.
 // Rows past group x seq_q are padding (the matrix pipe runs at 0.3 of its rate even for one row of 16, under the loads).
 //
 // Measured at 16 sequences, 32 query heads on 8 K/V heads, 3967 keys, D 128, per-row mask (529 MB): 1108 us on the 128-query
@@ -296,17 +296,27 @@ template <int D, int QT> int32_t launch(DecodeArgs &a, hipStream_t st, bool *don
 }
 
 template <int D> int32_t launch_rows(DecodeArgs &a, hipStream_t st, bool *done) {
-    // one row tile of 16 where the rows fit it, else tiles of 32
-    return (int64_t)a.group * a.d.seq_q <= 16 ? launch<D, 1>(a, st, done) : launch<D, 2>(a, st, done);
+    // Row tiles of 16 where the rows fit one, and up to 2048 keys (more tiles, which the chip has room for: 32 query heads on 8
+    // K/V heads, 8 queries, 128 keys of 64: 11.9 -> 9.4 us); else of 32, which read K and V half as often (4096 keys: 34 against
+    // 36 us). A row is computed alike in both.
+    return (int64_t)a.group * a.d.seq_q <= 16 || a.d.seq_k <= 2048 ? launch<D, 1>(a, st, done) : launch<D, 2>(a, st, done);
 }
 
 }  // namespace
 
 namespace fth {
 
-// seq_q <= 8: the larger tiles of csrc/sdpa.hip pad to 32 or 128 queries and read K and V once per query head. Measured at one
-// query they are 4 to 10 times slower.
-bool sdpa_decode_applies(const fth_sdpa_desc &d) {
+// seq_q <= 8: the tiled kernels of csrc/sdpa.hip pad to 128 queries and read K and V once per query head: 2 times slower at 16
+// keys, 4 to 10 times at 4096. Its key-split kernel for small problems (short_alternative: it would take the call otherwise)
+// needs one launch where this one needs a second for the merge, and is the faster one past the 64 keys of a single share while K
+// is short. us, that kernel / this one, 12 heads of 64, one query: 64 keys 7.6 / 5.8, 128 keys 7.9 / 9.2, 256 keys 10.9 / 9.6,
+// 4096 keys 97 / 32; of 32: 256 keys 7.5 / 8.1, 512 keys 11.0 / 9.3. With more than 128 query heads and 5 to 8 queries the line
+// is at twice that (256 heads, 384 keys of 64: 14.9 / 18.6). Neither the number of K/V heads nor that of shares decides, so a
+// grouped call and the same call on repeated K/V heads take the same path; the price is up to a tenth on 192 to 256 ungrouped
+// heads of up to 1024 keys (512 keys of 64: 18.9 / 19.9), where grouped ones gain a third to a half.
+bool sdpa_decode_applies(const fth_sdpa_desc &d, bool short_alternative) {
+    const int64_t line = d.num_bh > 128 && d.seq_q > 4 ? 32768 : 16384;
+    if (short_alternative && d.seq_k > 64 && d.seq_k * d.d_k < line) return false;
     // a head's K and V are addressed through unsigned 32-bit offsets, key numbers are ints with room for the last share
     auto span_ok = [&](int64_t row_stride) { return row_stride >= 0 && d.seq_k * row_stride < ((int64_t)1 << 30); };
     return d.causal == 0 && d.seq_q <= 8 && d.seq_k > 0 && d.seq_k <= ((int64_t)1 << 28) && d.d_k == d.d_v &&
@@ -314,7 +324,7 @@ bool sdpa_decode_applies(const fth_sdpa_desc &d) {
 }
 
 bool sdpa_decode_f32(const fth_sdpa_desc &d, float scale, const float *q, const float *k, const float *v, const float *mask,
-                     int64_t mask_bh_stride, float *out, hipStream_t st, int32_t *rc) {
+                     int64_t mask_bh_stride, float *out, bool short_alternative, hipStream_t st, int32_t *rc) {
     DecodeArgs a;
     a.q = q; a.k = k; a.v = v; a.mask = mask; a.out = out;
     a.part_o = a.part_ml = nullptr;
@@ -325,9 +335,11 @@ bool sdpa_decode_f32(const fth_sdpa_desc &d, float scale, const float *q, const 
     a.kv_heads = (int)(d.heads / a.group);
     a.row_tiles = 1;
     // Shares of the keys: about 8192 (query head, share) pairs, which is 8 wavefronts per compute unit even where four query
-    // heads ride on one K/V head; at least two 32-key tiles per share.
+    // heads ride on one K/V head; at least two 32-key tiles per share. Half of that without a mask at head sizes 32 and 64, where
+    // the merge weighs more: 256 heads on 256 K/V heads, 2048 keys of 64 62 -> 56 us, on 32 K/V heads 23 -> 18 us (with a mask at
+    // head size 128 and 4 queries, 256 heads on 32, 4096 keys it would cost 52 -> 65 us).
     const int64_t tiles = fth::ceil_div(d.seq_k, kTile);
-    int64_t want = 8192 / (d.num_bh > 0 ? d.num_bh : 1);
+    int64_t want = (short_alternative ? 4096 : 8192) / (d.num_bh > 0 ? d.num_bh : 1);
     const int64_t most = tiles / 2 > 0 ? tiles / 2 : 1;
     want = want < 1 ? 1 : want > most ? most : want;
     a.tiles_per_split = (int)fth::ceil_div(tiles, want);

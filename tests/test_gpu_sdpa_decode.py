@@ -13,7 +13,9 @@ pytestmark = pytest.mark.gpu
 
 # (batch, h_q, h_kv, seq_q, seq_k, d)
 SHAPES = [(1, 1, 1, 1, 1, 64), (2, 4, 4, 1, 31, 32), (1, 8, 2, 4, 32, 64), (1, 8, 2, 4, 33, 128), (2, 17, 1, 1, 64, 32), (1, 8, 1, 4, 65, 64),
-          (1, 6, 2, 8, 130, 128), (1, 33, 1, 1, 97, 64), (3, 32, 8, 1, 397, 128), (1, 4, 1, 8, 1027, 64), (1, 8, 8, 2, 4099, 128), (1, 9, 1, 8, 200, 32)]
+          (1, 6, 2, 8, 130, 128), (1, 33, 1, 1, 97, 64), (3, 32, 8, 1, 397, 128), (1, 4, 1, 8, 1027, 64), (1, 8, 8, 2, 4099, 128), (1, 9, 1, 8, 200, 32),
+          # more than 16 rows on a K/V head and more than 2048 keys: tiles of 32 rows; more heads than 128, either side of that line
+          (1, 32, 1, 1, 2500, 32), (1, 17, 1, 2, 2049, 128), (1, 24, 1, 3, 3000, 64), (1, 24, 1, 3, 2048, 64), (5, 32, 8, 5, 500, 64), (5, 32, 32, 8, 513, 64)]
 
 
 @pytest.mark.parametrize("shape", SHAPES)
