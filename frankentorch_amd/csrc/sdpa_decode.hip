@@ -63,11 +63,16 @@ template <int NE> struct VRow {  // NE consecutive floats of a V row
         for (int i = 0; i < NE / 4; ++i) v[i] = reinterpret_cast<const F4 *>(p)[i];
     }
     __device__ __forceinline__ float get(int e) const { return v[e / 4][e % 4]; }
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int i = 0; i < NE / 4; ++i) v[i] = F4{0.f, 0.f, 0.f, 0.f};
+    }
 };
 template <> struct VRow<2> {
     float2 v;
     __device__ __forceinline__ void load(const float *p) { v = *reinterpret_cast<const float2 *>(p); }
     __device__ __forceinline__ float get(int e) const { return e == 0 ? v.x : v.y; }
+    __device__ __forceinline__ void clear() { v = make_float2(0.f, 0.f); }
 };
 
 template <int D, int QT, bool MASK>
@@ -197,6 +202,13 @@ __global__ __launch_bounds__(64, QT == 1 ? 2 : 1) void sdpa_decode_kernel(const 
             for (int e = 0; e < NE; ++e)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) o[t][e][r] *= alpha;
+        }
+        if (key0 + kTile > seq_k) {  // weight 0 times an infinite value would be NaN
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (key0 + 16 * s + 4 * g + r >= seq_k) vf[s][r].clear();
         }
 #pragma unroll
         for (int s = 0; s < 2; ++s)

@@ -93,6 +93,29 @@ def test_caches_as_they_lie_in_memory(hip, oracle, sk, reverse):
     assert rel_err(got, ref) <= TOL_GEMM_F32
 
 
+@pytest.mark.parametrize("sk", [1, 31, 33, 64, 300, 1030])
+@pytest.mark.parametrize("d,masked", [(128, False), (128, True), (64, True), (32, True)])
+def test_non_finite_values_at_the_last_key(hip, oracle, sk, d, masked):
+    """The last K/V row also stands in for the keys past it in its 32-key tile: an infinite value there is infinite in the output
+    (its weight is positive), not NaN; a NaN key is NaN everywhere; scales of either sign and zero."""
+    batch, hq, hkv, sq = 1, 4, 2, 2
+    for scale in (0.125, 0.0, -0.125):
+        for what in ("value", "key"):
+            q, k, v = (synth.normal(54, t, s) for t, s in (("q", (batch, hq, sq, d)), ("k", (batch, hkv, sk, d)), ("v", (batch, hkv, sk, d))))
+            if what == "value":
+                v[0, 0, -1, 3], v[0, 1, -1, 5] = np.inf, -np.inf
+            else:
+                k[0, 0, -1, 7] = np.nan
+            views = [(DeviceBuffer.from_host(t), hkv * sk * d, sk * d, d, 0) for t in (k, v)]
+            mask = synth.normal(54, "m", (sq, sk), 0.0, 0.5) if masked else None
+            got = _strided(hip, batch, hq, hkv, sq, sk, d, (DeviceBuffer.from_host(q), hq * sq * d, sq * d, d, 0), *views, np.float32(scale), mask)
+            ref = oracle.sdpa_forward_masked_gqa(q, k, v, np.float32(scale), mask if masked else np.zeros((sq, sk), np.float32))
+            fine = np.isfinite(ref)
+            assert np.array_equal(got[~fine], ref[~fine], equal_nan=True), (scale, what)
+            if fine.any():
+                assert rel_err(got[fine], ref[fine]) <= TOL_GEMM_F32
+
+
 @pytest.mark.parametrize("sq,d,masked,dtype", [(2, 64, True, np.float32), (70, 128, False, np.float32), (70, 64, True, np.float32), (70, 64, False, np.float64)])
 def test_a_cache_read_backwards_on_the_other_kernels(hip, oracle, sq, d, masked, dtype):
     """Negative row strides where the tiled kernels' unsigned lane offsets cannot go: the general kernel answers."""
