@@ -1556,19 +1556,18 @@ int32_t gemm_entry(const fth_gemm_desc *d, T alpha, const T *a, const T *b, T *c
         return FTH_OK;
     }
     if constexpr (std::is_same<T, float>::value) {
-        // Large single products: exact three-way bf16 split (gemm_split.hip). FT_HIP_GEMM_SPLIT=0 is a tuning knob.
-        static const bool split_off = [] {
-            const char *e = std::getenv("FT_HIP_GEMM_SPLIT");
-            return e && std::atoi(e) == 0;
-        }();
-        const bool direct = d->k % 32 == 0 && d->lda % 4 == 0 && d->ldb % 4 == 0 && (d->trans_b || d->n % 4 == 0) && (!d->trans_a || d->m % 4 == 0) &&
-                            ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15u) == 0;
-        if (!split_off && d->batch == 1 && fth::split_gemm_pays(d->m, d->n, d->k, direct)) {
-            fth::SplitGemm g{a, b, d->trans_a ? 1 : d->lda, d->trans_a ? d->lda : 1, d->trans_b ? d->ldb : 1, d->trans_b ? 1 : d->ldb,
-                             c, bias, residual, nullptr, d->m, d->n, d->k, d->ldc, alpha, d->epilogue};
-            int32_t rc = FTH_OK;
-            if (fth::split_gemm(g, st, &rc)) return rc;
-        }
+        // Large single products: three-way bf16 split (gemm_split.hip). A forced tile is one of the fp32 kernels'.
+        auto quads = [](const T *x, int64_t ld) { return ld % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0; };
+        const bool whole_b = quads(b, d->ldb) && (d->trans_b || d->n % 4 == 0);
+        const bool whole_a = quads(a, d->lda) && (!d->trans_a || d->m % 4 == 0);  // (else a [k, m] operand is copied)
+        const auto rival = !whole_b || d->k % 4 != 0 || !(whole_a || d->trans_a) ? fth::SplitRival::Single
+                           : d->k % 32 != 0                                      ? fth::SplitRival::Vector
+                           : whole_a                                             ? fth::SplitRival::Direct
+                                                                                 : fth::SplitRival::Copied;
+        const fth::SplitGemm g{a, b, d->trans_a ? 1 : d->lda, d->trans_a ? d->lda : 1, d->trans_b ? d->ldb : 1, d->trans_b ? 1 : d->ldb,
+                               c, bias, residual, nullptr, d->m, d->n, d->k, d->ldc, alpha, d->epilogue};
+        int32_t rc = FTH_OK;
+        if (d->batch == 1 && forced_tile() < 0 && fth::split_gemm_pays(g, rival) && fth::split_gemm(g, st, &rc)) return rc;
     }
     if (d->trans_a) return launch_trans_a<T>(p, d, st);
     constexpr int EPV = Mfma<T>::EPV;
@@ -1605,10 +1604,8 @@ bool launch_nt_rowmax(int64_t m, int64_t n, int64_t k, const float *a, const flo
     }();
     if (direct_off || m <= 0 || n <= 0 || k <= 0 || k % 32 != 0 || !al(a) || !al(b) || k > lim || n > lim || big_tiles < cus || forced_tile() > 0)
         return false;
-    if (fth::split_gemm_pays(m, n, k, true)) {
-        fth::SplitGemm g{a, b, k, 1, k, 1, c, nullptr, nullptr, rowmax, m, n, k, n, 1.f, 0};
-        if (fth::split_gemm(g, st, rc)) return true;
-    }
+    const fth::SplitGemm g{a, b, k, 1, k, 1, c, nullptr, nullptr, rowmax, m, n, k, n, 1.f, 0};
+    if (forced_tile() < 0 && fth::split_gemm_pays(g, fth::SplitRival::Direct) && fth::split_gemm(g, st, rc)) return true;
     GemmArgs<float> p;
     p.a = a; p.b = b; p.c = c; p.bias = nullptr; p.residual = nullptr;
     p.m = m; p.n = n; p.k = k;

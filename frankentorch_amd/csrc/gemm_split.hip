@@ -30,6 +30,7 @@
 // replaces gemm::sgemm / sgemm_bt / sgemm_tb (crates/ft-kernel-cpu/src/lib.rs:1310-1338, 1430-1524) for large products.
 
 #include <cfloat>
+#include <cstdlib>
 
 #include "common.hpp"
 #include "devmath.hpp"
@@ -617,17 +618,36 @@ size_t scratch_bytes(int64_t m, int64_t n, int64_t k, const Choice &ch) {
 
 namespace fth {
 
-bool split_gemm_pays(int64_t m, int64_t n, int64_t k, bool fp32_direct) {
+bool split_gemm_pays(const SplitGemm &g, SplitRival rival) {
+    static const bool off = [] {
+        const char *e = std::getenv("FT_HIP_GEMM_SPLIT");  // tuning knob: 0 keeps large products on fp32 MFMAs
+        return e && std::atoi(e) == 0;
+    }();
     // Under 1.5 GFLOP the fp32 path has its own small kernels and the launches decide: a 128 x 256 x 256 block would lose 26 us.
-    if (m < 64 || n < 64 || k < 128 || 2.0 * m * n * k < 1.5e9 || m > (1 << 20) || n > (1 << 20) || k > (1 << 20) || m * n > ((int64_t)1 << 31)) return false;
-    const Choice ch = choose(m, n, k, false);
+    const int64_t m = g.m, n = g.n, k = g.k;
+    const double flop = 2.0 * m * n * k;
+    if (off || m < 64 || n < 64 || k < 128 || flop < 1.5e9 || m > (1 << 20) || n > (1 << 20) || k > (1 << 20) || m * n > ((int64_t)1 << 31)) return false;
+    const Choice ch = choose(m, n, k, g.rowmax != nullptr);
     if (scratch_bytes(m, n, k, ch) > kStreamScratchMost) return false;
-    // This path: the product, and the planes at 10 bytes an element, 4.5 TB/s and 3 us. The fp32 kernels: 130 TFLOP/s and 16 us
-    // (whole-tile effects and the fix-up pass of a split K) with direct-to-LDS operands, 0.6 of that without.
-    // us, fp32 -> split: 2331 x 768 x 768 44 -> 32, 768 x 768 x 2331 (A stored [k, m]) 62 -> 39, 4000 x 1024 x 1024 83 -> 55; where
-    // the line is, 1024^3 32 -> 29; below it, 512 x 768 x 768 21 -> 21 and 1000 x 512 x 512 17 -> 20.
-    const double ideal = 2.0 * m * n * k / 130e6;
-    return ch.us + 10.0 * k * (m + n) / 4.5e6 + 3.0 < 0.95 * ((fp32_direct ? ideal : 1.7 * ideal) + 16.0);
+    // This path: the product, the planes at 10 bytes an element (12 where it is stored [k][rows]), 4.5 TB/s and 3 us, and for less
+    // than 256 k the output's way to memory. The fp32 kernels: 130 TFLOP/s and 16 us (whole-tile effects and the fix-up pass of a
+    // split K) with direct-to-LDS operands, but 7 us where 128 x 96 tiles come out even; 0.69 of that rate and 25 us with 128-bit
+    // loads, 0.59 and 16 us with single ones; the transposed copy of a ragged [k, m] operand. The second is the least certain of the three. us, fp32 -> split: 2331 x 768 x 768
+    // 44 -> 32, 768 x 768 x 2331 (A stored [k, m]) 62 -> 38, 4000 x 1024 x 1024 83 -> 55, 1414 x 2504 x 224 35 -> 23; near the line,
+    // 303 x 10360 x 288 35 -> 31, 360 x 528 x 4304 38 -> 32, 256 x 816 x 4479 46 -> 34; past it, 8192 x 768 x 128 20 -> 22, with B
+    // stored [k, n] 198 x 6752 x 7868 241 -> 265 and 256 x 5704 x 7844 209 -> 226.
+    const int64_t slots = 2 * (int64_t)(compute_units() > 0 ? compute_units() : 256);
+    const bool even = rival == SplitRival::Direct && g.a_ks == 1 && n % 96 == 0 && ceil_div(m, 128) * (n / 96) % slots == 0 &&
+                      ceil_div(m, 128) * ceil_div(n, 128) % slots != 0;  // (as the fp32 path chooses them)
+    const double out_us = k < 256 ? 4.0 * m * n / 6.5e6 : 0.0;
+    const double planes_us = ((g.a_ks == 1 ? 10.0 : 12.0) * m + (g.b_ks == 1 ? 10.0 : 12.0) * n) * k / 4.5e6 + 3.0;
+    const double ours = ch.us + planes_us + out_us, copy_us = g.a_ks == 1 ? 0.0 : 8.0 * m * k / 4.5e6;
+    switch (rival) {
+        case SplitRival::Direct: return ours < 0.95 * (flop / 130e6 + (even ? 7.0 : 16.0 + out_us));
+        case SplitRival::Copied: return ours < 1.08 * (flop / 130e6 + 16.0 + out_us + copy_us);
+        case SplitRival::Vector: return ours < 0.85 * (flop / (0.69 * 130e6) + 25.0 + out_us + copy_us);
+        default: return ours < 1.02 * (flop / (0.59 * 130e6) + 16.0 + out_us);
+    }
 }
 
 bool split_gemm(const SplitGemm &g, hipStream_t st, int32_t *rc) {

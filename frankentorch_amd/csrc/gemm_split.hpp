@@ -18,9 +18,11 @@ struct SplitGemm {
     int epilogue;
 };
 
-// True when the split product is the faster one for this shape and its planes fit the scratch bound. fp32_direct: the fp32
-// kernel it stands in for would read its operands straight into LDS.
-bool split_gemm_pays(int64_t m, int64_t n, int64_t k, bool fp32_direct);
+// How the fp32 kernel that the split product would stand in for reads its operands.
+enum class SplitRival { Direct, Copied, Vector, Single };  // straight into LDS, so after a transposed copy of A, in 128-bit loads, element by element
+
+// True when the split product is the faster one for this shape and its planes fit the scratch bound.
+bool split_gemm_pays(const SplitGemm &g, SplitRival rival);
 // Runs it. Returns false, with nothing launched, when the scratch memory cannot be had.
 bool split_gemm(const SplitGemm &g, hipStream_t st, int32_t *rc);
 
