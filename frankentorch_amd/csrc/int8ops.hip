@@ -542,9 +542,13 @@ int32_t fth_dev_linear_int8_prequantized_f32(const int8_t *x_i8, const float *a_
         }();
         const bool big = forced == 256 || forced == 512 || (forced != 128 && tiles256 >= cus && k >= 2048);
         // Rows of one to four 16-row MFMA tiles: a 128-row tile would be mostly padding and leave the chip short of workgroups.
-        // At the upper end of the rule the two are close where n is large: 64 x 4096 x 11008 35.3 -> 33.3 us, 64 x 4096 x 4096
-        // 29.5 -> 16.1 us. Past it the activations would be read from L2 more often than the weights from memory.
-        if (m <= 64 && forced == 0) {
+        // That stops being so once n is wide enough for 128-column tiles to fill the chip, the earlier the more rows read their
+        // activations again in every workgroup, the later the longer K. us with the quantiser, 128 x 128 tiles / few-row kernel,
+        // weights rotating through 300 MB: 64 x 4096 x 4096 (m x k x n) 29.5 / 16.1, x 11008 35.3 / 33.3, x 18432 37.1 / 45.9;
+        // 16 x 4096 x 18432 30.3 / 30.0, x 20480 24.0 / 27.3; 1 x 4096 x 24576 0.77 of the time, x 28672 25.1 / 25.1; k 11008:
+        // 16 x 32000 0.95 of the time, x 128256 368 / 397, 64 x 18432 74 / 95; k 768: 32 x 24576 0.78 of the time, x 32000 14.4 / 14.6.
+        const int64_t widest = cus * (int64_t)(m > 32 ? 64 : k >= 8192 ? (m <= 16 ? 128 : 96) : k < 2048 || m <= 4 ? 96 : m <= 16 ? 72 : 64);
+        if (m <= 64 && n <= widest && forced == 0) {
             const bool wide = n >= 32 * (int64_t)cus;  // 32 columns a workgroup still give every compute unit one: half the activation reads
             const dim3 grid((unsigned)fth::ceil_div(n, 16)), grid2((unsigned)fth::ceil_div(n, 32));
             if (m <= 16) i8_skinny_kernel<1, 1><<<grid, dim3(512), 0, st>>>(p);

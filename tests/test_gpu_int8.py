@@ -84,7 +84,7 @@ def test_linear_int8_dynamic_is_bit_exact(hip, oracle, m, k, n, with_bias):
 
 # few rows: edges of the 16-row tiles, ragged columns, K shorter than one step a wavefront, whole and broken runs of it
 @pytest.mark.parametrize("m", [1, 15, 16, 17, 32, 33, 63, 64, 65])
-@pytest.mark.parametrize("k,n", [(64, 16), (448, 1), (576, 53), (4096, 130), (11008, 33), (576, 8209), (16384, 17), (16448, 16)])
+@pytest.mark.parametrize("k,n", [(64, 16), (448, 1), (576, 53), (4096, 130), (11008, 33), (576, 8209), (16384, 17), (16448, 16), (192, 24577), (576, 18433)])
 def test_few_rows_are_bit_exact(hip, oracle, m, k, n):
     x, w, bias = synth.normal(43, "x", (m, k), 0.0, 3.0), synth.normal(43, "w", (n, k), 0.0, 0.5), synth.normal(43, "b", (n,))
     w_i8, w_scales = oracle.quantize_rows_i8(w)
