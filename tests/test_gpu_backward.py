@@ -76,8 +76,8 @@ def test_linear_backward(hip, oracle, batch, in_f, out_f, dtype):
 
 def test_linear_backward_at_the_benchmark_shape_sampled(hip, oracle):
     """Batch 8192, 768 -> 3072 (the FC1 layer of the GPT-2 shape): dx = dy . W is an 8192 x 768 x 3072 product with W stored
-    [k, n], which runs on 128 x 96 tiles (512 whole tiles, one per resident workgroup); dweight splits its 8192-deep reduction
-    across workgroups. Sampled rows of both against the checker's GEMM, dbias against its column sum, and a bitwise repeat."""
+    [k, n], dweight a 3072 x 768 x 8192 one with dy stored [k, m], its 8192-deep reduction split across workgroups. Both run on the
+    split product (on the fp32 kernels they are among the products of test_gpu_gemm_split.test_which_kernels_run). Sampled rows of both against the checker's GEMM, dbias against its column sum, and a bitwise repeat."""
     batch, in_f, out_f = 8192, 768, 3072
     dy = synth.normal(33, "dy", (batch, out_f))
     x = synth.normal(33, "x", (batch, in_f))

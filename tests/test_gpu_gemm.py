@@ -40,7 +40,8 @@ def test_gemm_matches_oracle(hip, oracle, m, n, k, trans_b, dtype):
 # K a whole number of 128-byte K-tiles with 16-byte aligned rows: the global->LDS direct kernels.
 # Ragged m / n (clamped edge rows and columns), one-row and one-vector extents, tile counts that
 # leave every workgroup a mix of whole and split tiles (several tiles per workgroup, K split 2-3 ways), and the GPT-2
-# O-projection shape at a short K, which the [n, k] fp32 form runs on 128 x 96 tiles (512 whole tiles, none split).
+# O-projection shape at a short K, which the [n, k] fp32 form runs on 128 x 96 tiles (512 whole tiles, none split). The fp32 ones
+# of 1.5 GFLOP and more run on the split product as single calls; their fp32 kernels are tested in batches below.
 DIRECT_SHAPES = [(200, 300, 96), (77, 52, 64), (130, 132, 512), (1, 4, 32), (1000, 8, 32), (129, 257 * 4, 160),
                  (2048, 2304, 768), (4096, 3072, 256), (2050, 1540, 288), (8192, 768, 64)]
 
@@ -64,6 +65,25 @@ def test_direct_to_lds_kernels(hip, oracle, m, n, k, trans_b, dtype):
     assert np.array_equal(got, (plain + bias) + res)                             # same roundings as the separate ops
     got = _run(hip, a, b, trans_b, bias, None, EPI_BIAS | EPI_GELU)
     assert rel_err(got[rows], oracle.gelu(ref + bias)) <= tol
+
+
+@pytest.mark.parametrize("m,n,k", [(2048, 2304, 768), (4096, 3072, 256), (2050, 1540, 288), (8192, 768, 64)])
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_direct_to_lds_kernels_in_batches(hip, oracle, m, n, k, trans_b):
+    """The shapes above that run on the split product as single fp32 calls, two at a time: the fp32 kernels with mixed whole and split
+    tiles, and whole 128 x 96 tiles."""
+    a = synth.uniform(2, "da2", (2, m, k), -1, 1)
+    b = synth.uniform(2, "db2", (2, n, k) if trans_b else (2, k, n), -1, 1)
+    bias = synth.normal(2, "dbias", (n,))
+    da, db, dbias, dc = DeviceBuffer.from_host(a), DeviceBuffer.from_host(b), DeviceBuffer.from_host(bias), DeviceBuffer((2, m, n))
+    hip.gemm(hip.gemm_desc(m, n, k, trans_b=trans_b, batch=2), da, db, dc)
+    plain = dc.to_host()
+    hip.gemm(hip.gemm_desc(m, n, k, trans_b=trans_b, batch=2, epilogue=EPI_BIAS), da, db, dc, dbias)
+    with_bias = dc.to_host()  # (not plain + bias bit for bit: 128 x 128 tiles without an epilogue run on other matrix instructions)
+    rows = np.unique(np.concatenate([np.arange(0, m, max(1, m // 37)), [m - 1]]))
+    for i in range(2):
+        ref = oracle.gemm(a[i][rows], b[i], trans_b)
+        assert rel_err(plain[i][rows], ref) <= TOL_GEMM_F32 and rel_err(with_bias[i][rows], ref + bias) <= TOL_GEMM_F32
 
 
 # A stored [k, m] (gemm::sgemm_tb / dgemm_tb): direct-to-LDS shapes, a ragged shape that goes through

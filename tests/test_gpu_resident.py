@@ -162,10 +162,11 @@ def test_block_equals_its_separate_launches_bit_for_bit(hip):
 
 
 def test_graph_replay_survives_a_larger_gemm_and_new_tensors_on_its_stream(hip):
-    """A captured graph keeps the address of the stream's GEMM split-tile workspace. A later, larger product on the same
-    stream outgrows that workspace; the old block must stay out of the pool, or a tensor allocated afterwards could be
-    handed the memory the replay still writes its partial tiles to."""
-    batch, seq, d, heads, f = 2, 1024, 512, 8, 2048  # 2048 tokens: the projections run the large-tile kernels with split tiles
+    """A captured graph keeps the addresses of scratch: the stream's GEMM split-tile workspace where a product splits tiles, and the
+    planes of its large fp32 products, which are its own. A later, larger product on the same stream outgrows the split-tile
+    workspace; the old block must stay out of the pool, or a tensor allocated afterwards could be handed the memory the replay
+    still writes its partial tiles to. (Planes outgrown beside a live graph: test_gpu_stream_scratch.)"""
+    batch, seq, d, heads, f = 2, 1024, 512, 8, 2048  # 2048 tokens: the projections run the split product
     layers = [make_layer(6, i, d, f, biases_zero=False) for i in range(2)]
     x = synth.normal(6, "x", (batch * seq, d))
     enc = fused.EncoderHip(d, heads, f, layers, 1e-5, causal=True)
