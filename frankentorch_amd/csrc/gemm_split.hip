@@ -18,7 +18,7 @@
 // reads them; the product then moves planes to LDS with direct loads and has no vector arithmetic in its loop. Splitting
 // inside the product was tried and costs more: vector instructions and MFMAs share issue cycles, every element would be
 // split again by each tile that reads it, and the loop stayed at 190-230 TFLOP/s (of fp32 products) where this one reaches
-// 240-263.
+// 240-264.
 //
 // What the split cannot stand for is found in the results. Non-zero operands under 2^-110, whose third part would lie below the
 // bf16 subnormals, operands of 2^53 and more, whose sums of up to 2^20 products could overflow where fp32 arithmetic does not,
@@ -210,11 +210,13 @@ __device__ __forceinline__ f32x4 four_k(const float *p, int64_t ks, int left) {
 // The product. WM x WN wavefronts share a BM x BN tile; a wavefront's operands of one K-tile are 3 (TM + TN) 128-bit LDS reads
 // for 6 TM TN MFMAs. Two LDS buffers of a K-tile's planes, one barrier a K-tile: behind it the loads of the K-tile after
 // next are issued into the buffer that was just read out, and the operands of the next K-tile are read while this one's
-// MFMAs run, plane by plane as a plane's last MFMA has been issued (x2 y0 and x0 y2 first, x0 y0 last; only plane 0 needs
-// two register sets). The operands are passed (B, A): a lane then holds four neighbouring columns of one row of C, stored
-// as one vector. Persistent: workgroups walk the tiles `grid` apart, loads run ahead across tile borders.
-// Bound by the matrix units and the power they draw: 4096^3 263 TFLOP/s of fp32 products, 1.58 PFLOP/s of bf16 ones
-// (fp32 MFMA kernel: 146).
+// MFMAs run, plane by plane as a plane's last MFMA has been issued (x1 y1, x1 y0, x0 y1, then plane 2's, x0 y0 last). So one
+// register set holds each plane, and the barrier stands behind x1 y1, under which plane 0 arrives. 238 registers for a wavefront
+// of 64 x 64 with both accumulators, none spilled. The operands are passed (B, A): a lane then holds four neighbouring columns
+// of one row of C, stored as one vector. Persistent: workgroups walk the tiles `grid` apart, loads run ahead across tile borders.
+// Bound by the matrix units and the power they draw: 4096^3 264 TFLOP/s of fp32 products, 1.58 PFLOP/s of bf16 ones (fp32 MFMA
+// kernel: 146); by counter the matrix units are busy in 0.74 of the cycles at a clock of 1.7 GHz (nominal 2.4), without an LDS
+// bank conflict.
 template <int BM, int BN, int WM, int WN, bool ROWMAX>
 __global__ __launch_bounds__(WM *WN *kWave, 2) void plane_gemm_kernel(const PlaneArgs p) {
     constexpr int NW = WM * WN;
@@ -256,14 +258,14 @@ __global__ __launch_bounds__(WM *WN *kWave, 2) void plane_gemm_kernel(const Plan
             const int c = i * NW + wave;
             int blk = tm * (BM / 16) + c % (BM / 16);
             blk = blk < p.a_blocks ? blk : p.a_blocks - 1;
-            a_off[i] = (unsigned)(c / (BM / 16) * p.a_blocks + blk) * (unsigned)kBlock;
+            a_off[i] = __builtin_amdgcn_readfirstlane((unsigned)(c / (BM / 16) * p.a_blocks + blk) * (unsigned)kBlock);
         }
 #pragma unroll
         for (int i = 0; i < LB; ++i) {
             const int c = i * NW + wave;
             int blk = tn * (BN / 16) + c % (BN / 16);
             blk = blk < p.b_blocks ? blk : p.b_blocks - 1;
-            b_off[i] = (unsigned)(c / (BN / 16) * p.b_blocks + blk) * (unsigned)kBlock;
+            b_off[i] = __builtin_amdgcn_readfirstlane((unsigned)(c / (BN / 16) * p.b_blocks + blk) * (unsigned)kBlock);
         }
     };
     const unsigned wdst = lds0 + (unsigned)wave * kBlock;
