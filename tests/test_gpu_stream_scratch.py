@@ -4,6 +4,7 @@ import ctypes as C
 import os
 import subprocess
 import sys
+import threading
 
 import numpy as np
 import pytest
@@ -98,6 +99,32 @@ def test_graphs_of_one_capture_stream_replay_beside_each_other(hip, kind):
     for g in graphs:
         g.free()
     assert hip.gemm_workspace_info()[0] >= held[2]  # what a caller's graph was given stays
+
+
+def test_threads_on_one_stream(hip):
+    """Calls of several threads on one stream share its block: no thread's kernels come between another's two launches."""
+    s = Stream()
+    ops = [kind(hip, 90 + i) for i in range(2) for kind in (Product, Decode)]
+    want = [_eager(hip, op, s) for op in ops]
+    failed = []
+
+    def work(op):
+        try:
+            for _ in range(25):
+                op.launch(s.handle)
+        except Exception as e:  # noqa: BLE001 - reported below
+            failed.append(e)
+
+    for _ in range(3):
+        threads = [threading.Thread(target=work, args=(op,)) for op in ops]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        s.synchronize()
+        assert not failed
+        for op, w in zip(ops, want):
+            assert np.array_equal(op.out.to_host().view(np.uint32), w)
 
 
 def test_a_capture_without_a_warm_stream_gives_the_same_bits(hip):
