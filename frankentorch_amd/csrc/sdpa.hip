@@ -1132,7 +1132,7 @@ int32_t sdpa_entry(const fth_sdpa_desc *d, double scale, const T *q, const T *k,
                                  d->seq_k <= 4096 && d->d_k == d->d_v && (d->d_k == 64 || d->d_k == 32);
         // Few queries against a cache: the kernels below pad them to 32 or 128 query rows and read K and V once per query head.
         int32_t rc = FTH_OK;
-        if (strides_ok && fth::sdpa_decode_applies(*d, small_takes) &&
+        if (strides_ok && !(small_knob == 2 && small_takes) && fth::sdpa_decode_applies(*d, small_takes) &&
             fth::sdpa_decode_f32(*d, (float)scale, reinterpret_cast<const float *>(q), reinterpret_cast<const float *>(k),
                                  reinterpret_cast<const float *>(v), reinterpret_cast<const float *>(a.mask), mask_bh_stride,
                                  reinterpret_cast<float *>(out), small_takes, st, &rc))
