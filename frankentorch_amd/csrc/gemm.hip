@@ -1289,6 +1289,7 @@ int32_t get_workspace(hipStream_t st, size_t partial_bytes, void **partials, int
         size_t want = partial_bytes;
         if (w.partial_bytes && want < 2 * w.partial_bytes && w.partial_bytes <= ((size_t)1 << 31)) want = 2 * w.partial_bytes;
         void *fresh = nullptr;
+        const fth::AllocateInCapture allow;  // (a product that runs here only because its capture was given no planes)
         if (int32_t rc = fth::pool_alloc(&fresh, want)) {
             if (want == partial_bytes) return rc;
             want = partial_bytes;  // the doubled block did not fit: take exactly what is needed

@@ -35,7 +35,8 @@ State &state() {
     return *s;
 }
 
-// FT_HIP_STREAM_SCRATCH (testing): 0 = no scratch is ever given, 2 = every allocation is refused by the driver.
+// FT_HIP_STREAM_SCRATCH (testing): 0 = no scratch is ever given, 2 = every allocation is refused by the driver, 3 = none is given
+// inside captures.
 int knob() {
     static const int v = [] {
         const char *e = std::getenv("FT_HIP_STREAM_SCRATCH");
@@ -44,19 +45,14 @@ int knob() {
     return v;
 }
 
-// hipMalloc that is allowed beside and inside stream captures and leaves no error behind.
+// hipMalloc that leaves no error behind.
 void *try_malloc(size_t bytes) {
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
+    const AllocateInCapture allow;
     void *p = nullptr;
     if (hipMalloc(&p, knob() == 2 ? (size_t)1 << 50 : bytes) != hipSuccess) {
         (void)hipGetLastError();
         p = nullptr;
     }
-    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) (void)hipGetLastError();
     return p;
 }
 
@@ -74,12 +70,19 @@ bool capture_of(hipStream_t st, unsigned long long *id) {
 
 }  // namespace
 
+AllocateInCapture::AllocateInCapture() : changed_(hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess) {
+    if (!changed_) (void)hipGetLastError();
+}
+AllocateInCapture::~AllocateInCapture() {
+    if (changed_ && hipThreadExchangeStreamCaptureMode(&mode_) != hipSuccess) (void)hipGetLastError();
+}
+
 StreamScratch::StreamScratch() : lock_(state().mu) {}
 
 void *StreamScratch::get(hipStream_t st, ScratchUse use, size_t bytes) try {
     State &s = state();
     unsigned long long id = 0;
-    if (knob() == 0 || bytes > kStreamScratchMost || st == hipStreamPerThread || !capture_of(st, &id)) return nullptr;
+    if (knob() == 0 || bytes > kStreamScratchMost || st == hipStreamPerThread || !capture_of(st, &id) || (id && knob() == 3)) return nullptr;
     Block &b = id ? s.captured[CaptureKey(id, st, (int)use)] : s.own[std::make_pair(st, (int)use)];
     if (b.bytes >= bytes) return b.ptr;
     size_t want = 2 * b.bytes < kStreamScratchMost ? 2 * b.bytes : kStreamScratchMost;

@@ -28,6 +28,19 @@ class StreamScratch {
     std::lock_guard<std::mutex> lock_;
 };
 
+// While it lives, this thread may allocate beside and inside its own stream captures.
+class AllocateInCapture {
+   public:
+    AllocateInCapture();
+    ~AllocateInCapture();
+    AllocateInCapture(const AllocateInCapture &) = delete;
+    AllocateInCapture &operator=(const AllocateInCapture &) = delete;
+
+   private:
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+    bool changed_;
+};
+
 // The capture that `st` is recording, 0 for none.
 unsigned long long capture_id(hipStream_t st);
 // Frees what the capture was given. Its graph and executables are gone and none of their replays is running.

@@ -233,3 +233,38 @@ def test_without_scratch_the_other_kernels_answer(hip, tmp_path, knob):
         assert np.array_equal(got["arr_%d" % (2 * i)], got["arr_%d" % (2 * i + 1)])
         assert rel_err(got["arr_%d" % (2 * i)].view(np.float32), want) <= TOL_GEMM_F32
     assert got["live"] <= 512 * 2 * 128 * 128 * 4
+
+
+CAPTURE_CHILD = """
+import sys
+sys.path[:0] = [%(root)r, %(root)r + "/tests"]
+import numpy as np
+from frankentorch_amd import device as hip
+import test_gpu_stream_scratch as t
+out = {}
+for name, kind in (("decode", t.Decode), ("product", t.Product)):
+    op, s = kind(hip, 70), t.Stream()
+    out[name + "_eager"] = t._eager(hip, op, s)
+    g = t.Graph(s, op.launch)
+    for i in range(3):
+        g.replay(s)
+        s.synchronize()
+        out[name + "_%%d" %% i] = op.out.to_host()
+        t._eager(hip, op, s)
+np.savez(sys.argv[1], **out)
+"""
+
+
+def test_a_capture_that_is_given_none(hip, tmp_path):
+    """FT_HIP_STREAM_SCRATCH=3: eager calls have their scratch, the capture does not and records the other kernels, whose own
+    workspace no eager call has sized."""
+    path = str(tmp_path / "out.npz")
+    subprocess.run([sys.executable, "-c", CAPTURE_CHILD % {"root": ROOT}, path], check=True, timeout=100, env=dict(os.environ, FT_HIP_STREAM_SCRATCH="3"))
+    got = np.load(path)
+    for name, kind in (("decode", Decode), ("product", Product)):
+        want = _eager(hip, kind(hip, 70), Stream())
+        assert np.array_equal(got[name + "_eager"], want)
+        for i in range(3):
+            assert rel_err(got["%s_%d" % (name, i)], want.view(np.float32)) <= TOL_GEMM_F32
+            assert np.array_equal(got["%s_%d" % (name, i)], got[name + "_0"])
+        assert not np.array_equal(got[name + "_0"].view(np.uint32), want)  # other kernels, other rounding
