@@ -28,6 +28,7 @@ HIP_SOURCES = [
     "gemm_split.hip",
     "sdpa.hip",
     "sdpa_decode.hip",
+    "sdpa_split.hip",
     "backward.hip",
     "sdpa_bwd.hip",
     "lossops.hip",

@@ -1,12 +1,9 @@
 // fp32 matrix products on the bf16 matrix units.
 //
-// A float has 24 significant bits; three bf16 values hold 8 each. Rounding to nearest three times, x = x0 + x1 + x2 EXACTLY
-// (x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1, which has at most 8 significant bits left), so nothing of an operand
-// is given up. Of the nine products of two such sums six are formed, x0 y0, x0 y1, x1 y0, x1 y1, x0 y2, x2 y0, and summed in
-// fp32; the three left out are below 2^-24 |x y| together and of either sign. Six bf16 MFMAs of 32 k cost 96 cycles where the
-// fp32 MFMAs cost 256. x0 y0 has an accumulator of its own: the other five are 2^-8 of it and less, and each of them added to
-// the full sum would round that sum again (several times an MFMA, which adds in groups), so they are kept apart until the end
-// of the tile. Relative 2-norm error against 64-bit sums, this kernel / the fp32 MFMA kernel:
+// Each operand is split into three bf16 parts that sum to it exactly (split_bf16.hpp); six products of parts are formed and summed
+// in fp32. Six bf16 MFMAs of 32 k cost 96 cycles where the fp32 MFMAs cost 256. x0 y0 has an accumulator of its own: the other
+// five are 2^-8 of it and less, and each of them added to the full sum would round that sum again (several times an MFMA, which
+// adds in groups), so they are kept apart until the end of the tile. Relative 2-norm error against 64-bit sums, this kernel / the fp32 MFMA kernel:
 //   normal operands, K 768, 3072, 4096, 50257: 1.6e-7 / 4.95e-7, 3.4e-7 / 9.9e-7, 4.0e-7 / 1.15e-6, 3.5e-7 / 1.7e-6
 //   of one sign (uniform), the same K:         1.5e-7 / 4.2e-7,  3.0e-7 / 8.3e-7, 3.0e-7 / 8.4e-7,  1.0e-7 / 6.1e-7
 //   ReLU of normal, the same K:                1.2e-7 / 3.5e-7,  2.7e-7 / 7.0e-7, 3.2e-7 / 8.1e-7,  2.9e-7 / 1.2e-6
@@ -35,6 +32,7 @@
 #include "common.hpp"
 #include "devmath.hpp"
 #include "gemm_split.hpp"
+#include "split_bf16.hpp"
 #include "stream_scratch.hpp"
 
 namespace {
@@ -43,40 +41,20 @@ constexpr int kWave = 64;
 constexpr int kXcds = 8;
 constexpr int kGroupM = 8;
 constexpr int kBK = 32;       // k of a K-tile: one 16 x 16 x 32 MFMA
-constexpr int kPlanes = 3;
 constexpr int kBlock = 1024;  // bytes of one plane of 16 rows x 32 k
 constexpr float kTiny = 0x1p-100f;
 constexpr uint32_t kTooLarge = 0x5a000000u, kTooSmall = 0x08800000u;  // bits of 2^53 and of 2^-110
 
-using bf16x8 = __attribute__((ext_vector_type(8))) __bf16;
-using bf16x2 = __attribute__((ext_vector_type(2))) __bf16;
-using f32x2 = __attribute__((ext_vector_type(2))) float;
-using f32x4 = __attribute__((ext_vector_type(4))) float;
-using u32x4 = __attribute__((ext_vector_type(4))) uint32_t;
+using fth::bf16x8;
+using fth::f32x4;
+using fth::kPlanes;
+using fth::u32x4;
 typedef f32x4 f32x4_any __attribute__((aligned(4)));  // 128-bit access at any float
-
-__device__ __forceinline__ uint32_t pack_bf16(float x, float y) {
-    const f32x2 v = {x, y};
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));  // v_cvt_pk_bf16_f32: to nearest even
-}
-__device__ __forceinline__ float lo_f32(uint32_t p) { return __builtin_bit_cast(float, p << 16); }
-__device__ __forceinline__ float hi_f32(uint32_t p) { return __builtin_bit_cast(float, p & 0xffff0000u); }
 
 // NaN in the place of a float that the parts cannot stand for.
 __device__ __forceinline__ float representable(float x) {
     const uint32_t u = __builtin_bit_cast(uint32_t, x) & 0x7fffffffu;
     return u >= kTooLarge || u - 1u < kTooSmall - 1u ? __builtin_nanf("") : x;  // (zero wraps round)
-}
-
-// The three parts of two floats, one dword each.
-__device__ __forceinline__ void split2(float x, float y, uint32_t &p0, uint32_t &p1, uint32_t &p2) {
-    p0 = pack_bf16(x, y);
-    x -= lo_f32(p0);
-    y -= hi_f32(p0);
-    p1 = pack_bf16(x, y);
-    x -= lo_f32(p1);
-    y -= hi_f32(p1);
-    p2 = pack_bf16(x, y);
 }
 
 // Planes of an operand: [K-tile][plane][16-row block][16 rows][4 chunks of 8 k], a 16-byte chunk at slot chunk ^ swz(row) of
@@ -88,15 +66,11 @@ __device__ __forceinline__ int swz(int row) {
 }
 
 __device__ __forceinline__ void store_chunk(const float (&v)[8], unsigned char *planes, int64_t kt, int blocks, int64_t row, int chunk) {
-    u32x4 w[kPlanes];
+    float r[8];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        uint32_t p0, p1, p2;
-        split2(representable(v[2 * e]), representable(v[2 * e + 1]), p0, p1, p2);
-        w[0][e] = p0;
-        w[1][e] = p1;
-        w[2][e] = p2;
-    }
+    for (int e = 0; e < 8; ++e) r[e] = representable(v[e]);
+    u32x4 w[kPlanes];
+    fth::split8(r, w);
 #pragma unroll
     for (int s = 0; s < kPlanes; ++s)
         *reinterpret_cast<u32x4 *>(planes + (kt * kPlanes + s) * blocks * kBlock + row * 64 + ((chunk ^ swz((int)(row & 15))) << 4)) = w[s];
