@@ -25,6 +25,7 @@ HIP_SOURCES = [
     "rowops.hip",
     "indexops.hip",
     "gemm.hip",
+    "gemm_small.hip",
     "gemm_split.hip",
     "sdpa.hip",
     "sdpa_decode.hip",

@@ -47,6 +47,7 @@
 
 #include "common.hpp"
 #include "devmath.hpp"
+#include "gemm_small.hpp"
 #include "gemm_split.hpp"
 #include "pool.hpp"
 #include "stream_scratch.hpp"
@@ -1148,11 +1149,11 @@ __global__ __launch_bounds__(64 * NW) void gemm_small_kernel(const GemmArgs<floa
     }
 }
 
-// The same for long reductions (k >= 512) with 16 x 16 output tiles (v_mfma_f32_16x16x4_f32): four times the workgroups, and
+// The same for long reductions (k >= 512) against a [k, n] B with 16 x 16 output tiles (v_mfma_f32_16x16x4_f32; [n, k]: gemm_small.hip): four times the workgroups, and
 // a wavefront load covers 64 contiguous bytes of each of 16 rows instead of 32 bytes of each of 32. With 32 x 32 tiles a
 // [128, 256] x k = 1024 product kept only 32 compute units busy and each spent its time moving 256 KiB of operands through its
 // one vector memory pipe.
-template <int NW, bool TRANS_B>
+template <int NW>
 __global__ __launch_bounds__(64 * NW) void gemm_small16_kernel(const GemmArgs<float> p) {
     using M = Mfma<float>;
     typedef float Acc4 __attribute__((ext_vector_type(4)));
@@ -1171,18 +1172,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_small16_kernel(const GemmArgs<fl
     ar = ar < p.m ? ar : p.m - 1;
     br = br < p.n ? br : p.n - 1;
     const float *ap = A + ar * p.lda + 4 * g;
-    const float *bp = TRANS_B ? B + br * p.ldb + 4 * g : B + (int64_t)(4 * g) * p.ldb + br;
+    const float *bp = B + (int64_t)(4 * g) * p.ldb + br;
     Acc4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 8
     for (int t = g0; t < g1; ++t) {
         const float4 av = *reinterpret_cast<const float4 *>(ap + 16 * t);
-        float4 bv;
-        if (TRANS_B) {
-            bv = *reinterpret_cast<const float4 *>(bp + 16 * t);
-        } else {
-            const float *bk = bp + (int64_t)(16 * t) * p.ldb;
-            bv = make_float4(bk[0], bk[p.ldb], bk[2 * p.ldb], bk[3 * p.ldb]);
-        }
+        const float *bk = bp + (int64_t)(16 * t) * p.ldb;
+        const float4 bv = make_float4(bk[0], bk[p.ldb], bk[2 * p.ldb], bk[3 * p.ldb]);
         // step i contracts k = 16 t + 4 g + i over the four lane groups
         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av.x, bv.x, acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av.y, bv.y, acc, 0, 0, 0);
@@ -1227,10 +1223,10 @@ template <bool TRANS_B> bool launch_small(GemmArgs<float> &p, int64_t batch, boo
     const int64_t tiles16 = fth::ceil_div(p.m, 16) * fth::ceil_div(p.n, 16);
     if (p.k < 512) {
         gemm_small_kernel<4, TRANS_B><<<grid, dim3(256), 0, st>>>(p);
-    } else if (p.k % 16 == 0 && tiles16 * batch <= 4096) {  // long reduction, few tiles: 16 x 16 tiles on four times the compute units
+    } else if (!TRANS_B && p.k % 16 == 0 && tiles16 * batch <= 4096) {  // long reduction, few tiles: 16 x 16 tiles on four times the compute units
         p.tiles_m = (int)fth::ceil_div(p.m, 16);
         p.tiles_n = (int)fth::ceil_div(p.n, 16);
-        gemm_small16_kernel<8, TRANS_B><<<dim3((unsigned)tiles16, (unsigned)batch), dim3(512), 0, st>>>(p);
+        gemm_small16_kernel<8><<<dim3((unsigned)tiles16, (unsigned)batch), dim3(512), 0, st>>>(p);
     } else if (p.k <= 512) {
         gemm_small_kernel<4, TRANS_B><<<grid, dim3(256), 0, st>>>(p);
     } else {
@@ -1555,6 +1551,16 @@ int32_t gemm_entry(const fth_gemm_desc *d, T alpha, const T *a, const T *b, T *c
         gemm_k0_kernel<T><<<dim3((unsigned)grid, (unsigned)d->batch), dim3(256), 0, st>>>(p);
         FTH_CHECK_LAUNCH("gemm_k0");
         return FTH_OK;
+    }
+    if constexpr (std::is_same<T, float>::value) {
+        // Few rows or little work: K split over the wavefronts of a workgroup (gemm_small.hip).
+        auto rows16 = [](const T *x, int64_t ld, int64_t stride) { return ld % 4 == 0 && stride % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0; };
+        const fth::SmallGemm small{a, b, c, bias, residual, d->m, d->n, d->k, d->lda, d->ldb, d->ldc, d->stride_a, d->stride_b, d->stride_c, d->batch,
+                                   alpha, d->epilogue, d->trans_b != 0};
+        int32_t small_rc = FTH_OK;
+        if (!d->trans_a && forced_tile() < 0 && rows16(a, d->lda, d->stride_a) && (!d->trans_b || rows16(b, d->ldb, d->stride_b)) &&
+            fth::small_gemm(small, st, &small_rc))
+            return small_rc;
     }
     if constexpr (std::is_same<T, float>::value) {
         // Large single products: three-way bf16 split (gemm_split.hip). A forced tile is one of the fp32 kernels'.
