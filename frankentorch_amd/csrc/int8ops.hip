@@ -502,6 +502,106 @@ __global__ __launch_bounds__(512) void i8_skinny_kernel(const I8Args p) {
     }
 }
 
+// The same with the loads turned round: 64 bytes of a row are taken by four neighbouring lanes and brought into the MFMA layout
+// through the wavefront's own LDS (no barrier: its LDS instructions execute in order). In the MFMA layout itself neighbouring
+// lanes read different rows, and a compute unit then takes in 16 bytes a cycle instead of 64, which is what binds once the
+// activations that each workgroup reads again are as much as its weights. U steps are in flight.
+// Whole call with the quantiser, weights rotating through 300 MB, i8_skinny_kernel -> here: 13 x 4096 x 11008 16.9 -> 15.9 us, 32 x
+// 4096 x 11008 23.3 -> 19.5, 64 x 4096 x 4096 17.3 -> 15.3; on the other side 13 x 4096 x 4096 10.15 / 10.5, 1 x 4096 x 11008 13.4 / 13.9, and
+// short K, where the staging is not covered: 64 x 768 x 11008 11.2 / 14.0.
+template <int MT, int NT>
+__global__ __launch_bounds__(512) void i8_skinny_quad_kernel(const I8Args p) {
+    constexpr int NW = 8, U = 4, TILE = 1024, SLOT = (MT + NT) * TILE;  // a tile: 16 rows x 64 bytes
+    __shared__ __attribute__((aligned(16))) unsigned char smem[NW][2 * SLOT];
+    static_assert(MT * NT * 1024 <= 2 * SLOT, "a wavefront's partial sums reuse its staging area");
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, lq = lane >> 4, qrow = lane >> 2, qc = lane & 3;
+    const int64_t n0 = (int64_t)blockIdx.x * (16 * NT);
+    const int8_t *w[NT], *x[MT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const int64_t row = n0 + j * 16 + qrow < p.n ? n0 + j * 16 + qrow : p.n - 1;
+        w[j] = p.b + row * p.k + qc * 16;
+    }
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        const int64_t row = t * 16 + qrow < p.m ? t * 16 + qrow : p.m - 1;
+        x[t] = p.a + row * p.k + qc * 16;
+    }
+    const int steps = (int)(p.k / 64), per = (steps + NW - 1) / NW;
+    const int first = wave * per, end = first + per < steps ? first + per : steps;
+    V4i acc[MT][NT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[t][j] = V4i{0, 0, 0, 0};
+    V4i wv[U][NT], xv[U][MT];
+    auto load = [&](int u, int step) __attribute__((always_inline)) {
+        const int64_t at = (int64_t)(step < steps ? step : steps - 1) * 64;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) wv[u][j] = *reinterpret_cast<const V4i *>(w[j] + at);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) xv[u][t] = *reinterpret_cast<const V4i *>(x[t] + at);
+    };
+    // chunk c of row r in slot c ^ f(r): the 128-bit reads of 16 rows at one chunk touch every bank once
+    auto f = [](int r) { const int t = r >> 2; return (((t ^ (t >> 1)) & 1) << 1) | ((t >> 1) & 1); };
+    const int wr = qrow * 64 + ((qc ^ f(qrow)) << 4), rd = l16 * 64 + ((lq ^ f(l16)) << 4);
+    unsigned char *area = smem[wave];
+    auto stage = [&](int u) __attribute__((always_inline)) {
+        unsigned char *s = area + (u & 1) * SLOT + wr;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) *reinterpret_cast<V4i *>(s + j * TILE) = wv[u][j];
+#pragma unroll
+        for (int t = 0; t < MT; ++t) *reinterpret_cast<V4i *>(s + (NT + t) * TILE) = xv[u][t];
+    };
+    auto multiply = [&](int u) __attribute__((always_inline)) {
+        const unsigned char *s = area + (u & 1) * SLOT + rd;
+        V4i b[NT];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) b[j] = *reinterpret_cast<const V4i *>(s + j * TILE);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            const V4i a = *reinterpret_cast<const V4i *>(s + (NT + t) * TILE);
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[t][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b[j], acc[t][j], 0, 0, 0);
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < U; ++u) load(u, first + u);
+    int s = first;
+    for (; s + U < end; s += U) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            stage(u);
+            load(u, s + U + u);
+            multiply(u);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (s + u < end) {
+            stage(u);
+            multiply(u);
+        }
+    int *mine = reinterpret_cast<int *>(area);
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) mine[((t * NT + j) * 4 + r) * kWave + lane] = acc[t][j][r];
+    __syncthreads();
+    for (int i = wave; i < MT * NT * 4; i += NW) {  // accumulator element r of a lane: row 4 (lane / 16) + r, column lane % 16
+        const int64_t row = i / (4 * NT) * 16 + lq * 4 + (i & 3), col = n0 + (i / 4) % NT * 16 + l16;
+        if (row >= p.m || col >= p.n) continue;
+        uint32_t sum = 0;  // wraps as the matrix units' accumulators do
+#pragma unroll
+        for (int v = 0; v < NW; ++v) sum += (uint32_t)reinterpret_cast<const int *>(smem[v])[i * kWave + lane];
+        float y = (float)(int)sum * p.a_scales[row] * p.b_scales[col];
+        if (p.bias) y += p.bias[col];
+        p.c[row * p.n + col] = y;
+    }
+}
+
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 }  // namespace
@@ -551,11 +651,15 @@ int32_t fth_dev_linear_int8_prequantized_f32(const int8_t *x_i8, const float *a_
         if (m <= 64 && n <= widest && forced == 0) {
             const bool wide = n >= 32 * (int64_t)cus;  // 32 columns a workgroup still give every compute unit one: half the activation reads
             const dim3 grid((unsigned)fth::ceil_div(n, 16)), grid2((unsigned)fth::ceil_div(n, 32));
-            if (m <= 16) i8_skinny_kernel<1, 1><<<grid, dim3(512), 0, st>>>(p);
-            else if (m <= 32 && wide) i8_skinny_kernel<2, 2><<<grid2, dim3(512), 0, st>>>(p);
-            else if (m <= 32) i8_skinny_kernel<2, 1><<<grid, dim3(512), 0, st>>>(p);
-            else if (wide) i8_skinny_kernel<4, 2><<<grid2, dim3(512), 0, st>>>(p);
-            else i8_skinny_kernel<4, 1><<<grid, dim3(512), 0, st>>>(p);
+            const auto launch = [&](auto quad, auto plain, const dim3 &g) {
+                if (k >= 2048 && (m > 16 || (m > 8 && n >= 8192))) quad<<<g, dim3(512), 0, st>>>(p);
+                else plain<<<g, dim3(512), 0, st>>>(p);
+            };
+            if (m <= 16) launch(i8_skinny_quad_kernel<1, 1>, i8_skinny_kernel<1, 1>, grid);
+            else if (m <= 32 && wide) launch(i8_skinny_quad_kernel<2, 2>, i8_skinny_kernel<2, 2>, grid2);
+            else if (m <= 32) launch(i8_skinny_quad_kernel<2, 1>, i8_skinny_kernel<2, 1>, grid);
+            else if (wide) launch(i8_skinny_quad_kernel<4, 2>, i8_skinny_kernel<4, 2>, grid2);
+            else launch(i8_skinny_quad_kernel<4, 1>, i8_skinny_kernel<4, 1>, grid);
             FTH_CHECK_LAUNCH("i8_skinny");
             return FTH_OK;
         }

@@ -92,6 +92,13 @@ def test_few_rows_are_bit_exact(hip, oracle, m, k, n):
         assert np.array_equal(_bits(_linear(hip, x, w_i8, w_scales, b)), _bits(oracle.linear_int8_dynamic(x, w_i8, w_scales, b)))
 
 
+# loads turned through LDS, with one and with two column tiles a workgroup: K steps that are no multiple of eight wavefronts, fewer
+# steps than slots, a last column tile of one column
+@pytest.mark.parametrize("m,k,n", [(9, 2112, 8193), (16, 4096, 8200), (17, 2048, 8209), (32, 2176, 8193), (33, 2112, 8224), (64, 2048, 8193), (64, 3008, 40)])
+def test_few_rows_loaded_by_quads_are_bit_exact(hip, oracle, m, k, n):
+    test_few_rows_are_bit_exact(hip, oracle, m, k, n)
+
+
 def test_extreme_integers_do_not_overflow(hip, oracle):
     """Every product +-127 * +-127 with the same sign over K = 4096: |acc| = 66 064 384, far inside int32."""
     m, k, n = 64, 4096, 128
