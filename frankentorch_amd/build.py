@@ -26,6 +26,7 @@ HIP_SOURCES = [
     "indexops.hip",
     "gemm.hip",
     "gemm_small.hip",
+    "gemm_f64.hip",
     "gemm_split.hip",
     "sdpa.hip",
     "sdpa_decode.hip",

@@ -47,6 +47,7 @@
 
 #include "common.hpp"
 #include "devmath.hpp"
+#include "gemm_f64.hpp"
 #include "gemm_small.hpp"
 #include "gemm_split.hpp"
 #include "pool.hpp"
@@ -1575,6 +1576,13 @@ int32_t gemm_entry(const fth_gemm_desc *d, T alpha, const T *a, const T *b, T *c
                                c, bias, residual, nullptr, d->m, d->n, d->k, d->ldc, alpha, d->epilogue};
         int32_t rc = FTH_OK;
         if (d->batch == 1 && forced_tile() < 0 && fth::split_gemm_pays(g, rival) && fth::split_gemm(g, st, &rc)) return rc;
+    }
+    if constexpr (std::is_same<T, double>::value) {
+        // Products that leave the large tiles short of work, or ragged ones (gemm_f64.hip).
+        const fth::SmallGemm64 small{a, b, c, bias, residual, d->m, d->n, d->k, d->lda, d->ldb, d->ldc, d->stride_a, d->stride_b, d->stride_c, d->batch,
+                                     alpha, d->epilogue, d->trans_a != 0, d->trans_b != 0};
+        int32_t rc = FTH_OK;
+        if (forced_tile() < 0 && fth::small_gemm_f64(small, st, &rc)) return rc;
     }
     if (d->trans_a) return launch_trans_a<T>(p, d, st);
     constexpr int EPV = Mfma<T>::EPV;

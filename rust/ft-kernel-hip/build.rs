@@ -4,7 +4,7 @@
 // needed to build. `csrc/` and `include/` are the crate's copies of frankentorch_amd/csrc and include/.
 use std::{env, path::PathBuf, process::Command};
 
-const HIP_SOURCES: &[&str] = &["runtime.hip", "staging.hip", "stream_scratch.hip", "rowops.hip", "indexops.hip", "gemm.hip", "gemm_small.hip", "gemm_split.hip", "sdpa.hip", "sdpa_decode.hip", "sdpa_split.hip", "backward.hip", "sdpa_bwd.hip", "lossops.hip", "ingest.hip", "int8ops.hip", "host_api.hip", "resident.hip"];
+const HIP_SOURCES: &[&str] = &["runtime.hip", "staging.hip", "stream_scratch.hip", "rowops.hip", "indexops.hip", "gemm.hip", "gemm_small.hip", "gemm_f64.hip", "gemm_split.hip", "sdpa.hip", "sdpa_decode.hip", "sdpa_split.hip", "backward.hip", "sdpa_bwd.hip", "lossops.hip", "ingest.hip", "int8ops.hip", "host_api.hip", "resident.hip"];
 const HIPCC_FLAGS: &[&str] = &["-O3", "--offload-arch=gfx950", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument"];
 
 fn main() {
