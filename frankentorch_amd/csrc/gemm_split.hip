@@ -501,12 +501,14 @@ __global__ __launch_bounds__(256) void plane_reduce_kernel(const PlaneArgs p) {
 
 // ---- which tile, how many runs of K ----
 
-// One workgroup of 128 x 256 or 128 x 192 a compute unit, or two of 64 x 128. Rates are TFLOP/s of fp32 products with every
-// compute unit busy, measured on 4096^3, 8192 x 768 x 3072 and 2331 x 768 x 768; the small tile's with one and with two
-// workgroups on a compute unit.
+// One workgroup of 128 x 256, 128 x 192 or 128 x 128 a compute unit, or two of 64 x 128. Rates are TFLOP/s of fp32 products with every
+// compute unit busy, measured on 4096^3, 8192 x 768 x 3072, 4662 x 768 x 768 and 2331 x 768 x 768; the small tile's with one and with
+// two workgroups on a compute unit, the others' in one round and in more. The square tile is for products of which it makes one
+// round and the small one two (in full rounds it is behind the wide one: 4096^3 614 us, 581): 1031 x 3072
+// x 768 42.9 -> 39.2 us, planes included, 3000 x 1024 x 1024 52.0 -> 47.4, 4662 x 768 x 768 44.5 -> 42.3, 6000 x 512 x 512 35.3 -> 33.7.
 struct Tile { int bm, bn; double rate[2]; };
-constexpr Tile kTiles[] = {{128, 256, {250., 250.}}, {128, 192, {238., 238.}}, {64, 128, {145., 200.}}};
-constexpr int kResident[] = {1, 1, 2};
+constexpr Tile kTiles[] = {{128, 256, {250., 250.}}, {128, 192, {238., 238.}}, {64, 128, {145., 200.}}, {128, 128, {255., 225.}}};
+constexpr int kResident[] = {1, 1, 2, 1};
 
 struct Choice { int tile = -1, splits = 1, kt_per = 0; double us = 0; };
 
@@ -516,16 +518,16 @@ Choice choose(int64_t m, int64_t n, int64_t k, bool rowmax) {
     const int cus = fth::compute_units() > 0 ? fth::compute_units() : 256;
     const int64_t ktiles = fth::ceil_div(k, kBK);
     Choice best;
-    for (int t = 0; t < (rowmax ? 1 : 3); ++t) {
+    for (int t = 0; t < (rowmax ? 1 : 4); ++t) {
         const Tile &c = kTiles[t];
         const int64_t tiles = fth::ceil_div(m, c.bm) * fth::ceil_div(n, c.bn);
-        for (int s = 1; s <= (rowmax ? 1 : 16); ++s) {
+        for (int s = 1; s <= (rowmax || t == 3 ? 1 : 16); ++s) {  // (the square tile with a split K: 5246 x 320 x 896 43 us, 40 without it)
             const int64_t per = fth::ceil_div(ktiles, s);
             if (s > 1 && (per < 8 || (s - 1) * per >= ktiles)) break;
             const int64_t most = fth::ceil_div(tiles * s, (int64_t)cus);
             const double one = 2.0 * c.bm * c.bn * kBK * per * cus * 1e-6;
             double us = 2.0 + 2.0 * most / kResident[t];
-            us += kResident[t] == 1 ? most * one / c.rate[0] : (most / 2) * 2 * one / c.rate[1] + (most % 2) * one / c.rate[0];
+            us += kResident[t] == 1 ? most * one / c.rate[most > 1] : (most / 2) * 2 * one / c.rate[1] + (most % 2) * one / c.rate[0];
             if (s > 1) us += (s + 1.0) * m * n * 4 / 4e6 + 4.0;
             if (best.tile < 0 || us < best.us) best = {t, s, (int)per, us};
         }
@@ -578,7 +580,8 @@ int32_t run_split(const fth::SplitGemm &g, const Choice &ch, unsigned char *scra
             rc = g.rowmax ? launch_planes<128, 256, 2, 4, true>(p, kResident[0], st) : launch_planes<128, 256, 2, 4, false>(p, kResident[0], st);
             break;
         case 1: rc = launch_planes<128, 192, 2, 4, false>(p, kResident[1], st); break;
-        default: rc = launch_planes<64, 128, 2, 2, false>(p, kResident[2], st); break;
+        case 2: rc = launch_planes<64, 128, 2, 2, false>(p, kResident[2], st); break;
+        default: rc = launch_planes<128, 128, 2, 4, false>(p, kResident[3], st); break;
     }
     if (rc || ch.splits == 1) return rc;
     plane_reduce_kernel<<<dim3((unsigned)fth::ceil_div(g.m * g.n, 256)), dim3(256), 0, st>>>(p);
