@@ -28,9 +28,10 @@ def _run(hip, m, n, k, trans_b, batch=1, epilogue=0, alpha=1.0, pad=0):
 
 # tiles of one row and one column; ragged tiles; column tiles that are no multiple of eight (the XCD order's last run); wavefronts
 # without a group of k (K 272 over eight), partly filled slots, six slots (K 768, 3072), four wavefronts (many tiles), two row tiles
-# (1536 tiles and more, with an odd number of row tiles), the largest single row and the LM head's shape with few rows
+# (1536 tiles and more, with an odd number of row tiles), two column tiles as well (3072 and more, an odd number of them) and three row
+# tiles (6000 and more), the largest single row and the LM head's shape with few rows
 NT = [(1, 1, 256), (1, 17, 272), (16, 16, 256), (17, 33, 464), (37, 768, 3072), (5, 3072, 768), (64, 768, 1040), (37, 2304, 768), (128, 1016, 384),
-      (400, 2304, 768), (333, 1536, 512), (49, 8200, 256), (65, 10000, 768), (1, 50257, 768), (33, 20000, 272)]
+      (400, 2304, 768), (333, 1536, 512), (49, 8200, 256), (65, 10000, 768), (1, 50257, 768), (33, 20000, 272), (200, 3793, 272), (65, 20003, 256), (41, 33009, 272)]
 
 
 @pytest.mark.parametrize("m,n,k", NT)
