@@ -170,14 +170,15 @@ template <int NW, int MT, int NT, int U, bool TRANS_B> int32_t launch(const fth:
     return FTH_OK;
 }
 
-// Which form. Long reductions, or few tiles: eight wavefronts; otherwise four, whose partial tiles are less to add up; two row tiles
+// Which form. Few tiles, or long reductions but for very many: eight wavefronts; otherwise four, whose partial tiles are less to add up; two row tiles
 // a workgroup, then two column tiles as well, once there are workgroups enough: rows of A come from L2 less often. Six slots where they come out even (K 768 and 3072 over eight wavefronts).
 // us, eight wavefronts / four / four with two row tiles: 37 x 768 x 3072 9.2 / 13.6 / -, 37 x 2304 x 768 6.4 / 6.3 / 8.1, 200 x 1536 x 512
 // 8.2 / 7.0 / 7.8, 9 x 3072 x 768 5.1 / 5.7 / -, 64 x 50257 x 768 - / 87 / 79; with 2 x 2 tiles 65, 37 x 50257 x 768 58.6, with 3 x 2 55.6
-// (2 x 1: 62.3), 400 x 2304 x 768 20.2 (21.8); 64 x 10000 x 768 16.4 (16.1).
+// (2 x 1: 62.3), 400 x 2304 x 768 20.2 (21.8); 64 x 10000 x 768 16.4 (16.1). 64 x 32000 x 1024
+// eight wavefronts 75, four with 2 x 2 tiles 52.
 template <bool TRANS_B> int32_t choose(const fth::SmallGemm &g, hipStream_t st) {
     const int64_t tiles = fth::ceil_div(g.m, 16) * fth::ceil_div(g.n, 16) * g.batch, per = fth::ceil_div(g.k / 16, 8);
-    if (g.k >= 1024 || tiles <= 288) return per % 6 == 0 ? launch<8, 1, 1, 6, TRANS_B>(g, st) : launch<8, 1, 1, 4, TRANS_B>(g, st);
+    if (tiles <= 288 || (g.k >= 1024 && tiles < 1536)) return per % 6 == 0 ? launch<8, 1, 1, 6, TRANS_B>(g, st) : launch<8, 1, 1, 4, TRANS_B>(g, st);
     if (tiles < 1536 || g.m <= 16) return launch<4, 1, 1, 4, TRANS_B>(g, st);
     if constexpr (TRANS_B) {
         if (tiles >= 6000 && g.m > 32 && g.m <= 48) return launch<4, 3, 2, 2, true>(g, st);
