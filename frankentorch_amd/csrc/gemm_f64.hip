@@ -32,8 +32,12 @@ __device__ __forceinline__ int swz(int row) {
 }
 
 // KA, KB: K is the contiguous direction of A, of B.
+// Three wavefronts a SIMD are asked for where that keeps the accumulators out of the second half of the register file: without it 64
+// moves between the halves surround every 16 MFMAs and share their issue cycles (1000 x 1024 x 1021 with A stored [k, m] 53.9 -> 53.0 us,
+// 620 x 1572 x 1768 83.6 -> 75.9; 1021 x 1024 x 1000 53.5 -> 48.5). With B stored [n, k] its loads then lie closer to their use and rows
+// of odd length lose more than the moves cost (1524 x 1997 x 1375 221 -> 250), so that form stays as the compiler lays it out.
 template <int NW, int U, bool KA, bool KB>
-__global__ __launch_bounds__(64 * NW) void gemm_f64_kernel(const fth::SmallGemm64 p, const int tiles_m, const int tiles_n) {
+__global__ __launch_bounds__(64 * NW, NW == 4 && !KB ? 3 : 1) void gemm_f64_kernel(const fth::SmallGemm64 p, const int tiles_m, const int tiles_n) {
     constexpr int T = 2, TILE = 1024, STAGED = T * ((KA ? 1 : 0) + (KB ? 1 : 0)), SLOT = STAGED * TILE;  // a tile: 16 rows x 64 bytes
     constexpr int PART = T * T * 4 * 64 * 8;  // a wavefront's partial tile, in its accumulator layout
     constexpr int AREA = 2 * SLOT > PART ? 2 * SLOT : PART;
@@ -162,7 +166,11 @@ __global__ __launch_bounds__(64 * NW) void gemm_f64_kernel(const fth::SmallGemm6
 
 template <int NW, int U, bool KA, bool KB> int32_t launch(const fth::SmallGemm64 &g, hipStream_t st) {
     const int tiles_m = (int)fth::ceil_div(g.m, 32), tiles_n = (int)fth::ceil_div(g.n, 32);
-    gemm_f64_kernel<NW, U, KA, KB><<<dim3((unsigned)(tiles_m * tiles_n), (unsigned)g.batch), dim3(64 * NW), 0, st>>>(g, tiles_m, tiles_n);
+    // Four workgroups fit on a compute unit in this form; with a long K and more than one round of them, three share L2 better
+    // (us with four / three: 1500^3 181 / 167, 4001 x 4001 x 999 797 / 748; in one round 1021 x 1024 x 1000 48.8 / 52.1; with a short K
+    // 8000 x 500 x 250 60.9 / 65.4, 1768 x 1572 x 620 85 / 86), for which each takes 48 of the 160 KB of LDS.
+    const unsigned reserve = NW == 4 && KA && !KB && g.k >= 800 && (int64_t)tiles_m * tiles_n * g.batch > 1024 ? 16384 : 0;
+    gemm_f64_kernel<NW, U, KA, KB><<<dim3((unsigned)(tiles_m * tiles_n), (unsigned)g.batch), dim3(64 * NW), reserve, st>>>(g, tiles_m, tiles_n);
     FTH_CHECK_LAUNCH("gemm_f64");
     return FTH_OK;
 }
