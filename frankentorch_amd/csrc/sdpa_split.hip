@@ -16,10 +16,14 @@
 // values of one sign 6.7e-7 / 4.4e-7, half of them zero 4.8e-7 / 4.5e-7, scores of standard deviation 8 1.8e-6 / 6.8e-7.
 //
 // What the parts cannot stand for: infinities, NaN, operands of 2^53 and more in Q or K (whose sums could overflow where fp32
-// sums do not) and values of V under 2^-110 (whose third part lies below the bf16 subnormals) where the output is small as well.
-// A wavefront that finds a NaN or an infinity in its results, or is told of such operands, computes its 32 queries again with fp32
-// MFMAs (sdpa_rows.hpp). Tiny values in Q and K need nothing: with the partners below 2^53 and a scale of at most 2^20
-// what is lost of a score is below 2^-50.
+// sums do not), values of V under 2^-110 (whose third part lies below the bf16 subnormals) where the output is small as well, and
+// weights under 2^-110 where nothing else makes up the output. What a weight loses is below 2^-134 (it is 2^-126 or zero at the
+// least, and the largest of a row at least one), so an output is off by at most seq_k 2^-134 max |V|: nothing that counts where it is
+// 2^-96 max |V| or more. A smaller one that is not zero needs keys of large weight whose values are zero or next to it. (The largest
+// |V| is kept beside the smallest for this: 690.5 -> 695 us of the causal problem above.)
+// A wavefront that finds a NaN, an infinity or such an output in its results, or is told of such operands, computes its 32 queries
+// again with fp32 MFMAs (sdpa_rows.hpp). Tiny values in Q and K need nothing: with the partners below 2^53 and a scale of at most
+// 2^20 what is lost of a score is below 2^-50.
 //
 // replaces sdpa_forward_f32 (crates/ft-kernel-cpu/src/lib.rs:4572-4651, 5200-5284) for problems of many queries.
 
@@ -40,7 +44,7 @@ using fth::kPlanes;
 using fth::u32x4;
 
 constexpr int kXcds = 8;
-constexpr float kLarge = 0x1p53f, kTinyOut = 0x1p-100f;
+constexpr float kLarge = 0x1p53f, kTinyOut = 0x1p-100f, kTinyShare = 0x1p-96f;
 constexpr uint32_t kTinyBits = 0x08800000u;  // 2^-110
 constexpr float kLazy = 6.0f;                // log2 units by which a score may exceed the reference m before it moves
 
@@ -79,7 +83,7 @@ __global__ __launch_bounds__(64 * QW *KW, 2) void sdpa_split_kernel(const SplitS
     constexpr int XS = D == 128 ? 0 : 1;  // x(c) = c << XS
     static_assert(SUB >= 1 && NTH == 512, "a thread splits one chunk of K and one of V a stage");
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-    __shared__ int flags[2];  // operands of 2^53 and more, tiny values of V
+    __shared__ uint32_t flags[3];  // operands of 2^53 and more, tiny values of V, bits of the largest |V|
 
     const fth_sdpa_desc &d = p.d;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -147,7 +151,7 @@ __global__ __launch_bounds__(64 * QW *KW, 2) void sdpa_split_kernel(const SplitS
     constexpr int KROWS = 64 / RL, VW = D / 64;     // K rows a wavefront reads at once; wavefronts along a row of V
     f32x4 kreg[2];
     float vreg[8];
-    float k_max = 0.f;
+    float k_max = 0.f, v_max = 0.f;
     uint32_t v_min = 0xffffffffu;
     // Offsets that depend on the lane are worked out where they are used: registers are what this kernel is short of.
     auto my_lane = [&]() __attribute__((always_inline)) {
@@ -197,6 +201,8 @@ __global__ __launch_bounds__(64 * QW *KW, 2) void sdpa_split_kernel(const SplitS
             const uint32_t u = (__builtin_bit_cast(uint32_t, vreg[e]) << 1) - 1u;  // (zero wraps round)
             v_min = u < v_min ? u : v_min;
         }
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) v_max = __builtin_fmaxf(__builtin_fmaxf(v_max, __builtin_fabsf(vreg[e])), __builtin_fabsf(vreg[e + 1]));
         u32x4 w[kPlanes];
         fth::split8(vreg, w);
         unsigned char *dst = smem + (kt & 1) * STAGE + VOFF + ((wave / VW * D + (wave % VW) * 64 + my_lane()) << 4);
@@ -211,7 +217,7 @@ __global__ __launch_bounds__(64 * QW *KW, 2) void sdpa_split_kernel(const SplitS
         for (int r = 0; r < 16; ++r) o[e][r] = 0.f;
     float m_run = -__builtin_inff(), l_run = 0.f;
 
-    if (tid < 2) flags[tid] = 0;
+    if (tid < 3) flags[tid] = 0;
     load_k(0);
     store_k(0);
     __syncthreads();
@@ -368,9 +374,15 @@ __global__ __launch_bounds__(64 * QW *KW, 2) void sdpa_split_kernel(const SplitS
     // ---- what the parts could not stand for ----
     {
         const bool large = __builtin_amdgcn_ballot_w64(!(k_max < kLarge)) != 0, tiny = __builtin_amdgcn_ballot_w64(v_min < 2 * kTinyBits - 1u) != 0;
+        float vlo, vhi;
+        fth::both_halves(v_max, vlo, vhi);
+        v_max = __builtin_fmaxf(vlo, vhi);
+#pragma unroll
+        for (int step = 16; step > 0; step >>= 1) v_max = __builtin_fmaxf(v_max, __shfl_xor(v_max, step));
         if (lane == 0) {
             if (large) flags[0] = 1;
             if (tiny) flags[1] = 1;
+            atomicMax(&flags[2], __builtin_bit_cast(uint32_t, v_max));  // (floats that are not negative are in the order of their bits)
         }
     }
     if constexpr (KW == 2) {
@@ -404,6 +416,7 @@ __global__ __launch_bounds__(64 * QW *KW, 2) void sdpa_split_kernel(const SplitS
         l_run = llo + lhi;
     }
     float big = 0.f, small = FLT_MAX;
+    uint32_t least = 0xffffffffu;  // of the outputs that are not zero, as v_min
 #pragma unroll
     for (int e = 0; e < NDT; ++e)
 #pragma unroll
@@ -411,8 +424,12 @@ __global__ __launch_bounds__(64 * QW *KW, 2) void sdpa_split_kernel(const SplitS
             o[e][r] = o[e][r] / l_run;
             big = nan_max(big, __builtin_fabsf(o[e][r]));
             small = __builtin_fminf(small, __builtin_fabsf(o[e][r]));
+            const uint32_t u = (__builtin_bit_cast(uint32_t, o[e][r]) << 1) - 1u;
+            least = u < least ? u : least;
         }
-    const bool doubt = q_live && (!(big <= FLT_MAX) || q_large || flags[0] != 0 || (flags[1] != 0 && small < kTinyOut));
+    const float share = __builtin_fminf(__builtin_bit_cast(float, flags[2]), FLT_MAX) * kTinyShare;
+    const bool lost = least < __builtin_bit_cast(uint32_t, share) << 1;
+    const bool doubt = q_live && (!(big <= FLT_MAX) || q_large || flags[0] != 0 || (flags[1] != 0 && small < kTinyOut) || lost);
     if (__builtin_amdgcn_ballot_w64(doubt)) {
         const int k_last = d.causal && wave_last_q + 1 < seq_k ? wave_last_q + 1 : seq_k;
         Acc16 f[NDT];

@@ -86,6 +86,26 @@ def test_operands_the_parts_cannot_stand_for(hip, d, heads, sq, sk, causal):
     assert _rel(out[heads - 1], ref) <= 2.0e-8 * np.sqrt(sk) + 1.2e-7
 
 
+@pytest.mark.parametrize("d,heads,sq,sk", [(64, 300, 256, 80), (64, 40, 300, 200), (128, 7, 300, 200)])
+@pytest.mark.parametrize("values", [1.0, 2.0 ** 60, 2.0 ** 125])
+def test_weights_below_the_parts(hip, d, heads, sq, sk, values):
+    """The key that takes all weight has values of zero, and the others lie 60 to 87 nats lower: nothing but their weights, down to 2^-126,
+    makes up the outputs. The scores are exact, so a weight carries the rounding of its exponent of at most 128 (2^-18) and of log2(e)
+    (128 x 2^-26), times ln 2, and an ulp: 4e-6; a sum of one sign no more, and a few ulp of its own."""
+    rng = np.random.default_rng(sk)
+    q, k = np.zeros((heads, sq, d), np.float32), np.zeros((heads, sk, d), np.float32)
+    q[:, :, 0] = 8.0
+    top = np.linspace(61, 86.5, heads)[rng.permutation(heads)]
+    k[:, :, 0] = -np.round((top[:, None] + rng.random((heads, sk)) * 0.5) * 64) / 64
+    k[:, 3, 0] = 0.0
+    v = ((0.5 + 0.5 * rng.random((heads, sk, d))) * values).astype(np.float32)
+    v[:, 3] = 0.0
+    out = _run(hip, q, k, v, False, scale=0.125)
+    for h in np.argsort(top)[::max(1, heads // 12)].tolist() + [int(np.argmax(top))]:
+        ref = _ref(q[h], k[h], v[h], False, 0.125)
+        assert np.max(np.abs(out[h] / ref - 1)) <= 5e-6, "%.1f nats" % top[h]
+
+
 @pytest.mark.parametrize("d,heads", [(64, 300), (128, 4)])
 def test_scales_beyond_the_range_stay_on_fp32_units(hip, d, heads):
     q, k, v = _inputs(heads, 1, 256, 200, d)
