@@ -397,13 +397,23 @@ __global__ __launch_bounds__(64 * NW, 2) void sdpa_mfma_kernel(const SdpaArgs p)
                         l_run *= alpha;
                         m_run = m_new;
                     }
-                    const float neg_m = -m_run;
+                    float neg_m = -m_run, per_score = c2;
+                    // From 2^24 on the rounding of m is more than a log2 unit and from 2^31 on 2^(s * c2 - m) could leave the range in
+                    // either direction at the largest score: the difference to m is then taken from the rounded product, which is zero there.
+                    if (__any(__builtin_fabsf(m_run) >= 0x1p24f)) {
+#pragma unroll
+                        for (int j = 0; j < KS; ++j)
+#pragma unroll
+                            for (int r = 0; r < 16; ++r) s[j][r] = s[j][r] * c2 - m_run;
+                        neg_m = 0.f;
+                        per_score = 1.f;
+                    }
                     // ---- O^T += V_tile^T . P^T with the exponentials in the same instruction stream ----
 #pragma unroll
                     for (int j = 0; j < KS; ++j)
 #pragma unroll
                         for (int r = 0; r < 16; ++r) {
-                            const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j][r], c2, neg_m));
+                            const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j][r], per_score, neg_m));
                             psum += e;
                             const VV vv = *reinterpret_cast<const VV *>(vp + (32 * j + 8 * (r >> 2) + (r & 3)) * VP);
 #pragma unroll
@@ -927,10 +937,16 @@ __global__ __launch_bounds__(256) void sdpa_small_kernel(const SdpaArgs p) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) o[e][r] *= alpha;
         }
-        float psum = 0.f;
+        float psum = 0.f, neg_m = -m_ref, per_score = c2;
+        if (__any(__builtin_fabsf(m_ref) >= 0x1p24f)) {  // (as in sdpa_mfma_kernel)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = s[r] * c2 - m_ref;
+            neg_m = 0.f;
+            per_score = 1.f;
+        }
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], c2, -m_ref));
+            const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], per_score, neg_m));
             psum += e;
 #pragma unroll
             for (int ee = 0; ee < NDT; ++ee) o[ee] = __builtin_amdgcn_mfma_f32_32x32x2f32(vecn_get(vv[r], ee), e, o[ee], 0, 0, 0);

@@ -149,3 +149,21 @@ def test_fully_resident_causal_launch_sampled_heads(hip, oracle, bh, seq):
         assert rel_err(out[h:h + 1], ref) <= TOL_GEMM_F32
     assert np.array_equal(out[:, 0], v[:, 0])
     assert np.all(out.max(axis=1) <= v.max(axis=1) + 1e-5) and np.all(out.min(axis=1) >= v.min(axis=1) - 1e-5)
+
+
+@pytest.mark.parametrize("bh,sq,sk,d,causal", [(7, 300, 100, 128, False), (7, 300, 100, 128, True), (300, 256, 200, 32, False), (300, 130, 100, 32, True),
+                                               (7, 300, 200, 128, True), (300, 256, 200, 64, True), (40, 100, 90, 64, False)])
+def test_scores_far_beyond_the_exponent_range(hip, bh, sq, sk, d, causal):
+    """Scores of 2^35 to 2^60, whose float spacing is more than the exponent range: the largest takes all the weight. They carry an
+    error of 2^-24 of themselves, so two keys that are close exchange their places in a few rows of a hundred at most."""
+    rng = np.random.default_rng(sk + d)
+    q, k, v = (rng.standard_normal((bh, n, d)).astype(np.float32) for n in (sq, sk, sk))
+    k *= (np.float32(2.0) ** np.linspace(35, 60, bh).astype(np.float32).round())[:, None, None]
+    out = _run(hip, q, k, v, 1.0 / math.sqrt(d), causal)
+    assert np.isfinite(out).all()
+    for h in (0, bh // 2, bh - 1):
+        s = q[h].astype(np.float64) @ k[h].astype(np.float64).T
+        if causal:
+            s[np.arange(sq)[:, None] < np.arange(sk)] = -np.inf
+        rows = np.abs(out[h] - v[h][s.argmax(axis=1)]).max(axis=1) <= 1e-6
+        assert rows.mean() >= 0.97
