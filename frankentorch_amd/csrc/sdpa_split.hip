@@ -20,7 +20,7 @@
 // weights under 2^-110 where nothing else makes up the output. What a weight loses is below 2^-134 (it is 2^-126 or zero at the
 // least, and the largest of a row at least one), so an output is off by at most seq_k 2^-134 max |V|: nothing that counts where it is
 // 2^-96 max |V| or more. A smaller one that is not zero needs keys of large weight whose values are zero or next to it. (The largest
-// |V| is kept beside the smallest for this: 690.5 -> 695 us of the causal problem above.)
+// |V| is kept beside the smallest for this: 0.3 us a block, 14.0 -> 14.3 us for 64 heads of 130 tokens, 694 -> 696 for the causal problem above.)
 // A wavefront that finds a NaN, an infinity or such an output in its results, or is told of such operands, computes its 32 queries
 // again with fp32 MFMAs (sdpa_rows.hpp). Tiny values in Q and K need nothing: with the partners below 2^53 and a scale of at most
 // 2^20 what is lost of a score is below 2^-50.
@@ -29,6 +29,7 @@
 
 #include <cfloat>
 #include <cstdlib>
+#include <type_traits>
 
 #include "common.hpp"
 #include "sdpa_rows.hpp"
@@ -61,6 +62,23 @@ __device__ __forceinline__ float nan_max(float a, float b) { return __builtin_el
 __device__ __forceinline__ bf16x8 as_bf16(u32x4 w) { return __builtin_bit_cast(bf16x8, w); }
 __device__ __forceinline__ Acc16 mfma(bf16x8 a, bf16x8 b, Acc16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
 
+// Largest x of a wavefront (no NaN), in every lane: along rows of 16 lanes, then across them.
+__device__ __forceinline__ float wave_max(float x) {
+    auto step = [&](auto ctrl) __attribute__((always_inline)) {
+        const int y = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, false);
+        x = __builtin_fmaxf(x, __builtin_bit_cast(float, y));
+    };
+    step(std::integral_constant<int, 0x128>{});  // row_ror by 8, 4, 2, 1
+    step(std::integral_constant<int, 0x124>{});
+    step(std::integral_constant<int, 0x122>{});
+    step(std::integral_constant<int, 0x121>{});
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, x), false, false);
+    x = __builtin_fmaxf(__builtin_bit_cast(float, r[0]), __builtin_bit_cast(float, r[1]));
+    float lo, hi;
+    fth::both_halves(x, lo, hi);
+    return __builtin_fmaxf(lo, hi);
+}
+
 // QW wavefronts of 32 queries each times KW wavefronts along the keys; a stage of LDS holds KEYS keys, of which a wavefront takes SUB
 // sub-tiles of 32.
 //   S^T[key, query]: A = K parts from LDS (lane: key l % 32, eight d from 8 (l / 32) on), B = the wavefront's Q parts in registers.
@@ -83,7 +101,8 @@ __global__ __launch_bounds__(64 * QW *KW, 2) void sdpa_split_kernel(const SplitS
     constexpr int XS = D == 128 ? 0 : 1;  // x(c) = c << XS
     static_assert(SUB >= 1 && NTH == 512, "a thread splits one chunk of K and one of V a stage");
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-    __shared__ uint32_t flags[3];  // operands of 2^53 and more, tiny values of V, bits of the largest |V|
+    __shared__ int flags[2];  // operands of 2^53 and more, tiny values of V
+    __shared__ float largest[NW];  // |V| that each wavefront has split
 
     const fth_sdpa_desc &d = p.d;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -217,7 +236,7 @@ __global__ __launch_bounds__(64 * QW *KW, 2) void sdpa_split_kernel(const SplitS
         for (int r = 0; r < 16; ++r) o[e][r] = 0.f;
     float m_run = -__builtin_inff(), l_run = 0.f;
 
-    if (tid < 3) flags[tid] = 0;
+    if (tid < 2) flags[tid] = 0;
     load_k(0);
     store_k(0);
     __syncthreads();
@@ -374,15 +393,11 @@ __global__ __launch_bounds__(64 * QW *KW, 2) void sdpa_split_kernel(const SplitS
     // ---- what the parts could not stand for ----
     {
         const bool large = __builtin_amdgcn_ballot_w64(!(k_max < kLarge)) != 0, tiny = __builtin_amdgcn_ballot_w64(v_min < 2 * kTinyBits - 1u) != 0;
-        float vlo, vhi;
-        fth::both_halves(v_max, vlo, vhi);
-        v_max = __builtin_fmaxf(vlo, vhi);
-#pragma unroll
-        for (int step = 16; step > 0; step >>= 1) v_max = __builtin_fmaxf(v_max, __shfl_xor(v_max, step));
+        v_max = wave_max(v_max);
         if (lane == 0) {
             if (large) flags[0] = 1;
             if (tiny) flags[1] = 1;
-            atomicMax(&flags[2], __builtin_bit_cast(uint32_t, v_max));  // (floats that are not negative are in the order of their bits)
+            largest[wave] = v_max;
         }
     }
     if constexpr (KW == 2) {
@@ -416,20 +431,28 @@ __global__ __launch_bounds__(64 * QW *KW, 2) void sdpa_split_kernel(const SplitS
         l_run = llo + lhi;
     }
     float big = 0.f, small = FLT_MAX;
-    uint32_t least = 0xffffffffu;  // of the outputs that are not zero, as v_min
 #pragma unroll
     for (int e = 0; e < NDT; ++e)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
+        for (int r = 0; r < 16; r += 2) {
             o[e][r] = o[e][r] / l_run;
-            big = nan_max(big, __builtin_fabsf(o[e][r]));
-            small = __builtin_fminf(small, __builtin_fabsf(o[e][r]));
-            const uint32_t u = (__builtin_bit_cast(uint32_t, o[e][r]) << 1) - 1u;
-            least = u < least ? u : least;
+            o[e][r + 1] = o[e][r + 1] / l_run;
+            const float a = __builtin_fabsf(o[e][r]), b = __builtin_fabsf(o[e][r + 1]);
+            big = nan_max(nan_max(big, a), b);
+            small = __builtin_fminf(__builtin_fminf(small, a), b);
         }
-    const float share = __builtin_fminf(__builtin_bit_cast(float, flags[2]), FLT_MAX) * kTinyShare;
-    const bool lost = least < __builtin_bit_cast(uint32_t, share) << 1;
-    const bool doubt = q_live && (!(big <= FLT_MAX) || q_large || flags[0] != 0 || (flags[1] != 0 && small < kTinyOut) || lost);
+    bool doubt = !(big <= FLT_MAX) || q_large || flags[0] != 0 || (flags[1] != 0 && small < kTinyOut);
+    float share = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) share = __builtin_fmaxf(share, largest[w]);
+    share = __builtin_fminf(share, FLT_MAX) * kTinyShare;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(small < share) != 0, 0)) {  // (zeros do not count)
+#pragma unroll
+        for (int e = 0; e < NDT; ++e)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) doubt |= o[e][r] != 0.f && __builtin_fabsf(o[e][r]) < share;
+    }
+    doubt &= q_live;
     if (__builtin_amdgcn_ballot_w64(doubt)) {
         const int k_last = d.causal && wave_last_q + 1 < seq_k ? wave_last_q + 1 : seq_k;
         Acc16 f[NDT];
