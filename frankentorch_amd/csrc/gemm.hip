@@ -1554,16 +1554,6 @@ int32_t gemm_entry(const fth_gemm_desc *d, T alpha, const T *a, const T *b, T *c
         return FTH_OK;
     }
     if constexpr (std::is_same<T, float>::value) {
-        // Few rows or little work: K split over the wavefronts of a workgroup (gemm_small.hip).
-        auto rows16 = [](const T *x, int64_t ld, int64_t stride) { return ld % 4 == 0 && stride % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0; };
-        const fth::SmallGemm small{a, b, c, bias, residual, d->m, d->n, d->k, d->lda, d->ldb, d->ldc, d->stride_a, d->stride_b, d->stride_c, d->batch,
-                                   alpha, d->epilogue, d->trans_b != 0};
-        int32_t small_rc = FTH_OK;
-        if (!d->trans_a && forced_tile() < 0 && rows16(a, d->lda, d->stride_a) && (!d->trans_b || rows16(b, d->ldb, d->stride_b)) &&
-            fth::small_gemm(small, st, &small_rc))
-            return small_rc;
-    }
-    if constexpr (std::is_same<T, float>::value) {
         // Large single products: three-way bf16 split (gemm_split.hip). A forced tile is one of the fp32 kernels'.
         auto quads = [](const T *x, int64_t ld) { return ld % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0; };
         const bool whole_b = quads(b, d->ldb) && (d->trans_b || d->n % 4 == 0);
@@ -1576,6 +1566,18 @@ int32_t gemm_entry(const fth_gemm_desc *d, T alpha, const T *a, const T *b, T *c
                                c, bias, residual, nullptr, d->m, d->n, d->k, d->ldc, alpha, d->epilogue};
         int32_t rc = FTH_OK;
         if (d->batch == 1 && forced_tile() < 0 && fth::split_gemm_pays(g, rival) && fth::split_gemm(g, st, &rc)) return rc;
+    }
+    if constexpr (std::is_same<T, float>::value) {
+        // Few rows or little work: K split over the wavefronts of a workgroup (gemm_small.hip). Asked after the split product, whose sums are
+        // closer (661 x 2304 x 640 1.4e-7 against 2.3e-7 with four chains) and which takes single products from 1.5 GFLOP on where it pays:
+        // 661 x 2304 x 640 28.4 -> 26.9 us, 1159 x 1280 x 640 27.4 -> 28.1, 2257 x 640 x 640 26.8 -> 28.0.
+        auto rows16 = [](const T *x, int64_t ld, int64_t stride) { return ld % 4 == 0 && stride % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0; };
+        const fth::SmallGemm small{a, b, c, bias, residual, d->m, d->n, d->k, d->lda, d->ldb, d->ldc, d->stride_a, d->stride_b, d->stride_c, d->batch,
+                                   alpha, d->epilogue, d->trans_b != 0};
+        int32_t small_rc = FTH_OK;
+        if (!d->trans_a && forced_tile() < 0 && rows16(a, d->lda, d->stride_a) && (!d->trans_b || rows16(b, d->ldb, d->stride_b)) &&
+            fth::small_gemm(small, st, &small_rc))
+            return small_rc;
     }
     if constexpr (std::is_same<T, double>::value) {
         // Products that leave the large tiles short of work, or ragged ones (gemm_f64.hip).

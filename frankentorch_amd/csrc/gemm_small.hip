@@ -202,7 +202,7 @@ bool small_gemm(const SmallGemm &g, hipStream_t st, int32_t *rc) {
     // Where it is the fastest, us of the kernels behind it / here, from a sweep of 21 (n, k) pairs and 18 m, both forms of B:
     // [n, k] B: K of 256 and more (2048 x 1000 x 64 8.3 / 11.6, 333 x 8192 x 128 13.3 / 17.9, but 1024 x 768 x 256 15.6 / 8.9). Up to 64
     // rows at any size (64 x 50257 x 768 97 / 65, 48 x 4096 x 4096 38 / 31). More rows: under 1.5 GFLOP, where the split product begins
-    // (400 x 2304 x 768 28.8 / 20.9, 1600 x 1152 x 384 31.5 / 21.9), and around K 768 up to 2 GFLOP (1600 x 768 x 768 33.2 / 27.5, 128 x
+    // (400 x 2304 x 768 28.8 / 20.9, 1600 x 1152 x 384 31.5 / 21.9), and around K 768 up to 2 GFLOP where that one is not taken (1600 x 768 x 768 33.2 / 27.5, 128 x
     // 10000 x 768 34.7 / 29.4; not 2048 x 768 x 768 36.7 / 43.2, 1300 x 1536 x 512 25.7 / 27.7, 1300 x 384 x 1536 29.6 / 31.3).
     // [k, n] B, whose loads are in the MFMA layout to begin with: mid-sized products (400 x 2304 x 768 28.5 / 23.8, 1600 x 1152 x 384
     // 31.4 / 24.1; not 24 x 2304 x 768 5.75 / 6.6, 777 x 512 x 2048 30.1 / 37.3).

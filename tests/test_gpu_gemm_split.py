@@ -49,6 +49,16 @@ def test_split_product_forms(hip, m, n, k, form):
     assert _rel(got[rows], ref) <= _bound(k)
 
 
+@pytest.mark.parametrize("m,n,k", [(661, 2304, 640), (1159, 1280, 640), (2257, 640, 640)])
+def test_split_product_before_the_one_for_little_work(hip, m, n, k):
+    """Both take products of 1.5 to 2 GFLOP against [n, k] weights; the split one has the smaller error, 0.57e-8 sqrt(K) measured (four fp32
+    chains a product: 0.9e-8 sqrt(K))."""
+    rng = np.random.default_rng(m + n + k)
+    a, b = rng.standard_normal((m, k), np.float32), rng.standard_normal((n, k), np.float32)
+    rows = np.arange(0, m, 97)
+    assert _rel(_gemm(hip, m, n, k, a, b, trans_b=True)[rows], a[rows].astype(np.float64) @ b.T.astype(np.float64)) <= 0.7e-8 * np.sqrt(k)
+
+
 @pytest.mark.parametrize("m,n,k", [(4096, 3072, 768), (2048, 768, 11008), (2331, 768, 768), (768, 768, 50257)])
 @pytest.mark.parametrize("kind", ["one sign", "relu", "one term"])
 def test_split_product_of_other_operands(hip, m, n, k, kind):
