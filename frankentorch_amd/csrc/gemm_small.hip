@@ -227,10 +227,14 @@ bool small_gemm(const SmallGemm &g, hipStream_t st, int32_t *rc) {
     // rows at any size (64 x 50257 x 768 97 / 65, 48 x 4096 x 4096 38 / 31). More rows: under 1.5 GFLOP, where the split product begins
     // (400 x 2304 x 768 28.8 / 20.9, 1600 x 1152 x 384 31.5 / 21.9), and around K 768 up to 2 GFLOP where that one is not taken (1600 x 768 x 768 33.2 / 27.5, 128 x
     // 10000 x 768 34.7 / 29.4; not 2048 x 768 x 768 36.7 / 43.2, 1300 x 1536 x 512 25.7 / 27.7, 1300 x 384 x 1536 29.6 / 31.3).
+    // The longest K belong to the kernels that cut K over many workgroups, which these few tiles leave idle: 64 x 128 x 131072 192 / 217,
+    // 16 x 256 x 131072 187 / 216; but 64 x 128 x 98304 189 / 145, 64 x 64 x 100000 270 / 164, 64 x 512 x 65536 130 / 109, 128 x 128 x 40000
+    // 111 / 73, 64 x 4096 x 11008 105 / 85, and where there is too little work for them 1 x 128 x 262144 830 / 420, 64 x 32 x 200000 352 / 337.
+    // Batches: 64 x 64 x 4096, 32 of them 35 / 31, 64 x 256 x 16384, eight 88 / 75, 64 x 128 x 256, 200 of them 22.5 / 19.2.
     // [k, n] B, whose loads are in the MFMA layout to begin with: mid-sized products (400 x 2304 x 768 28.5 / 23.8, 1600 x 1152 x 384
     // 31.4 / 24.1; not 24 x 2304 x 768 5.75 / 6.6, 777 x 512 x 2048 30.1 / 37.3).
     if (g.trans_b) {
-        if (g.k < 256 || (g.m > 64 && flop >= (g.k >= 640 && g.k <= 1024 ? 2.0e9 : 1.5e9))) return false;
+        if (g.k < 256 || (g.m > 64 && flop >= (g.k >= 640 && g.k <= 1024 ? 2.0e9 : 1.5e9)) || (g.k > 114688 && flop > 1.0e9)) return false;
     } else if (g.k < 384 || g.k > 1536 || flop < 1.0e8 || flop >= 1.5e9) {
         return false;
     }

@@ -3,9 +3,14 @@ against 64-bit sums. Error on normal operands, whose sums have the size sqrt(K):
 the matrix unit), whose results are added one after another, at most K / 128 of them a wavefront, and then over the wavefronts
 (2.4e-8 sqrt(additions / 2): the mean rounding of an addition); a fifth is allowed on top, and three standard deviations of a root mean
 square over few outputs."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
+from conftest import ROOT
 from frankentorch_amd.device import EPI_BIAS, EPI_GELU, EPI_RESIDUAL, DeviceBuffer
 
 pytestmark = pytest.mark.gpu
@@ -64,3 +69,26 @@ def test_batches_pitches_and_epilogues(hip, trans_b, m, n, k):
     from scipy.special import erf
     ref = 0.5 * plain * (1 + erf(plain / np.sqrt(2)))
     assert np.max(np.abs(gelu - ref)) <= 1e-6 * np.max(np.abs(ref))
+
+
+CHILD = """
+import sys
+sys.path[:0] = [%(root)r, %(root)r + "/tests"]
+import numpy as np
+from frankentorch_amd import device as hip
+import test_gpu_gemm_small as t
+np.savez(sys.argv[1], **{str(i): t._run(hip, *s, True)[0] for i, s in enumerate(t.LONG)})
+"""
+LONG = [(64, 128, 131072), (16, 256, 131072), (64, 128, 98304), (1, 128, 131072)]
+
+
+def test_longest_reductions(hip, tmp_path):
+    """Few tiles and a K past the limit run on the kernels that cut K over workgroups, as they do with these kernels switched off (a child
+    process: the switch is read once); on this side of it they do not. Error: the large tiles' 1.8e-8 sqrt(K) at the most."""
+    path = str(tmp_path / "large.npz")
+    subprocess.run([sys.executable, "-c", CHILD % {"root": ROOT}, path], check=True, timeout=110, env=dict(os.environ, FT_HIP_GEMM_SMALL="0"))
+    large = np.load(path)
+    for i, (m, n, k) in enumerate(LONG):
+        got, ref = _run(hip, m, n, k, True)
+        assert np.linalg.norm(got - ref) <= 1.8e-8 * np.sqrt(k) * np.linalg.norm(ref)
+        assert np.array_equal(got, large[str(i)]) == (i < 2), (m, n, k)
