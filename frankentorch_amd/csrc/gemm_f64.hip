@@ -10,6 +10,10 @@
 // neighbouring lanes read different rows, and a compute unit then takes in 16 bytes a cycle instead of 64) and turned into the
 // MFMA layout through the wavefront's own LDS, whose instructions execute in order; one whose rows or columns are contiguous is in
 // that layout as it is read. A group is 8 k: lane group g of the wavefront holds k 2 g and 2 g + 1 of it. U groups are in flight.
+// SHORT: chains of 16 MFMAs are added to a sum with ordinary additions, so that the error does not grow with the root of K: a chain
+// of L MFMAs loses 9.6e-17 sqrt(L / 2). It is for few tiles, whose K the large-tile kernels cut over many workgroups. Relative
+// 2-norm error against extended precision, those kernels / one chain a wavefront / here: 64 x 600 x 1500 3.3e-16 / 4.8e-16 / 2.9e-16, 300 x 900 x
+// 2500 6.3e-16 / 8.2e-16 / 3.0e-16; us without and with it 17.7 / 17.7 (A stored [k, m] 18.4 / 19.4), 300 x 300 x 1500 21.0 / 22.4, 512^3 10.5 / 10.8.
 // Bound by the matrix units and the vector instructions that share their issue cycles: 1500^3 41 of the 78.6 TFLOP/s.
 
 #include "gemm_f64.hpp"
@@ -36,7 +40,7 @@ __device__ __forceinline__ int swz(int row) {
 // moves between the halves surround every 16 MFMAs and share their issue cycles (1000 x 1024 x 1021 with A stored [k, m] 53.9 -> 53.0 us,
 // 620 x 1572 x 1768 83.6 -> 75.9; 1021 x 1024 x 1000 53.5 -> 48.5). With B stored [n, k] its loads then lie closer to their use and rows
 // of odd length lose more than the moves cost (1524 x 1997 x 1375 221 -> 250), so that form stays as the compiler lays it out.
-template <int NW, int U, bool KA, bool KB>
+template <int NW, int U, bool SHORT, bool KA, bool KB>
 __global__ __launch_bounds__(64 * NW, NW == 4 && !KB ? 3 : 1) void gemm_f64_kernel(const fth::SmallGemm64 p, const int tiles_m, const int tiles_n) {
     constexpr int T = 2, TILE = 1024, STAGED = T * ((KA ? 1 : 0) + (KB ? 1 : 0)), SLOT = STAGED * TILE;  // a tile: 16 rows x 64 bytes
     constexpr int PART = T * T * 4 * 64 * 8;  // a wavefront's partial tile, in its accumulator layout
@@ -90,11 +94,21 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && !KB ? 3 : 1) void gemm_f64_kern
             if (KB) *reinterpret_cast<D2 *>(s + ((KA ? T : 0) + i) * TILE) = bv[u][i];
         }
     };
-    D4 acc[T][T];
+    D4 acc[T][T], sum[T][T];
+    auto clear = [](D4 (&x)[T][T]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < T; ++i)
+        for (int i = 0; i < T; ++i)
 #pragma unroll
-        for (int j = 0; j < T; ++j) acc[i][j] = D4{0.0, 0.0, 0.0, 0.0};
+            for (int j = 0; j < T; ++j) x[i][j] = D4{0.0, 0.0, 0.0, 0.0};
+    };
+    auto collect = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < T; ++i)
+#pragma unroll
+            for (int j = 0; j < T; ++j) sum[i][j] += acc[i][j];
+    };
+    clear(acc);
+    if (SHORT) clear(sum);
     auto multiply = [&](int u, D2 (&a)[T], D2 (&b)[T]) __attribute__((always_inline)) {
         const unsigned char *s = area + (u & 1) * SLOT + rd;
 #pragma unroll
@@ -127,6 +141,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && !KB ? 3 : 1) void gemm_f64_kern
             load(u, t0 + U + u);
             multiply(u, a, b);
         }
+        if (SHORT && ((t0 - g0) & (8 - U)) == 8 - U) {  // every eight groups
+            collect();
+            clear(acc);
+        }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
@@ -140,13 +158,14 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && !KB ? 3 : 1) void gemm_f64_kern
         stage(0);
         multiply(0, av[0], bv[0]);
     }
+    if (SHORT) collect();
     double *part = reinterpret_cast<double *>(area);
 #pragma unroll
     for (int i = 0; i < T; ++i)
 #pragma unroll
         for (int j = 0; j < T; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) part[((i * T + j) * 4 + r) * 64 + lane] = acc[i][j][r];
+            for (int r = 0; r < 4; ++r) part[((i * T + j) * 4 + r) * 64 + lane] = SHORT ? sum[i][j][r] : acc[i][j][r];
     __syncthreads();
     double *C = p.c + batch * p.stride_c;
     for (int e = wave; e < T * T * 4; e += NW) {  // accumulator element r of a lane: row 4 r + lane / 16, column lane % 16
@@ -164,13 +183,13 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && !KB ? 3 : 1) void gemm_f64_kern
     }
 }
 
-template <int NW, int U, bool KA, bool KB> int32_t launch(const fth::SmallGemm64 &g, hipStream_t st) {
+template <int NW, int U, bool SHORT, bool KA, bool KB> int32_t launch(const fth::SmallGemm64 &g, hipStream_t st) {
     const int tiles_m = (int)fth::ceil_div(g.m, 32), tiles_n = (int)fth::ceil_div(g.n, 32);
     // Four workgroups fit on a compute unit in this form; with a long K and more than one round of them, three share L2 better
     // (us with four / three: 1500^3 181 / 167, 4001 x 4001 x 999 797 / 748; in one round 1021 x 1024 x 1000 48.8 / 52.1; with a short K
     // 8000 x 500 x 250 60.9 / 65.4, 1768 x 1572 x 620 85 / 86), for which each takes 48 of the 160 KB of LDS.
     const unsigned reserve = NW == 4 && KA && !KB && g.k >= 800 && (int64_t)tiles_m * tiles_n * g.batch > 1024 ? 16384 : 0;
-    gemm_f64_kernel<NW, U, KA, KB><<<dim3((unsigned)(tiles_m * tiles_n), (unsigned)g.batch), dim3(64 * NW), reserve, st>>>(g, tiles_m, tiles_n);
+    gemm_f64_kernel<NW, U, SHORT, KA, KB><<<dim3((unsigned)(tiles_m * tiles_n), (unsigned)g.batch), dim3(64 * NW), reserve, st>>>(g, tiles_m, tiles_n);
     FTH_CHECK_LAUNCH("gemm_f64");
     return FTH_OK;
 }
@@ -178,8 +197,11 @@ template <int NW, int U, bool KA, bool KB> int32_t launch(const fth::SmallGemm64
 template <bool KA, bool KB> int32_t choose(const fth::SmallGemm64 &g, hipStream_t st) {
     // Few tiles: eight wavefronts share K, four groups ahead (512^3 8.9 us, four wavefronts 10.5); otherwise four, with fewer registers
     // and so more workgroups on a compute unit (1500^3 166 us, eight wavefronts 190).
-    if (fth::ceil_div(g.m, 32) * fth::ceil_div(g.n, 32) * g.batch <= 256) return launch<8, 4, KA, KB>(g, st);
-    return launch<4, 2, KA, KB>(g, st);
+    const int64_t tiles = fth::ceil_div(g.m, 32) * fth::ceil_div(g.n, 32) * g.batch;
+    if (tiles <= 256) return launch<8, 4, true, KA, KB>(g, st);
+    // The large-tile kernels cut K of about as many tiles; from 512 on they walk it in one chain, with more error than four (1021 x 1024 x
+    // 1000 7.3e-16 / 5.4e-16), and the registers of the sum would cost a workgroup of the four on a compute unit.
+    return tiles <= 512 ? launch<4, 2, true, KA, KB>(g, st) : launch<4, 2, false, KA, KB>(g, st);
 }
 
 }  // namespace
