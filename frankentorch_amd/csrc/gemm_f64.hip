@@ -216,9 +216,13 @@ bool small_gemm_f64(const SmallGemm64 &g, hipStream_t st, int32_t *rc) {
     // 64 x 64 tiles fill the chip (512^3 20.5 / 9.7, 768 x 1024 x 1024 39.3 / 35.5, but 896^3 37.9 / 41.1, 1024^3 45 / 48, 2048^3 261 / 332),
     // later with a short K (1024 x 1024 x 128 20.9 / 12.4; 2048 x 1024 x 128 16.4 / 19.1). All others at any size: 1000 x 1024 x 1021 with A stored
     // [k, m] 73.8 / 52.7, 1021 x 1024 x 1000 65 / 52, 3001 x 3000 x 301 180 / 153, 4001 x 4001 x 999 834 / 819, 300 x 300 x 9 26 / 4.3.
-    if (g.k > (tiles <= 256 ? 2048 : 2560)) return false;
+    // Two corners are slower: a very few tiles with a long K that goes straight to LDS there (64 x 64 x 2000 20.5 / 21.3 to 23.9 by form, 64 x
+    // 64 x 1408 16.9 / 16.0 to 18.2, 17 x 290 x 2000 22.5 / 21.4), and with both K contiguous a long K on few tiles more than one for
+    // every compute unit (300 x 900 x 2500 50.2 / 60.1, 1700 38.8 / 41.3, 1300 33.0 / 32.3; 450 x 1000 x 2500 72 / 64).
+    if (g.k > (tiles <= 256 ? 2048 : 2560) || (g.trans_b && g.k > 1600 && tiles > 256 && tiles <= 320)) return false;
     auto even = [](int64_t ld, int64_t stride, const double *x) { return ld % 2 == 0 && stride % 2 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0; };
     const bool direct = g.k % 16 == 0 && even(g.lda, g.stride_a, g.a) && even(g.ldb, g.stride_b, g.b) && (!g.trans_a || g.m % 2 == 0) && (g.trans_b || g.n % 2 == 0);
+    if (direct && tiles <= 8 && g.k > 1536) return false;
     if (direct && g.k > 64 && tiles > 256 && !(g.k <= 1024 && tiles64 <= 192) && !(g.k <= 256 && tiles64 <= 256)) return false;
     const bool ka = !g.trans_a, kb = g.trans_b;
     if (!ka && kb) return false;  // (the entry point refuses this form)

@@ -35,10 +35,10 @@ def _run(hip, m, n, k, form, batch=1, epilogue=0, alpha=1.0, pad=0):
 
 
 # one tile and less, K shorter than a group and than a group a wavefront, every remainder of K modulo 8 in each form, odd pitches
-# (rows that are not 16-byte aligned), column tiles that are no multiple of eight, eight wavefronts and four, the longest K of each
+# (rows that are not 16-byte aligned), column tiles that are no multiple of eight, eight wavefronts and four, the longest K of each, past which other kernels run
 @pytest.mark.parametrize("form", ["nt", "nn", "tn"])
 @pytest.mark.parametrize("m,n,k", [(1, 1, 2), (3, 5, 7), (32, 32, 8), (33, 31, 9), (64, 70, 64), (40, 300, 131), (100, 33, 1021), (17, 290, 2047), (600, 650, 13),
-                                   (1021, 1000, 30), (515, 777, 252), (700, 801, 2557), (1030, 1060, 831)])
+                                   (1021, 1000, 30), (515, 777, 252), (700, 801, 2557), (1030, 1060, 831), (64, 64, 1536), (64, 64, 2000), (300, 900, 1600), (300, 900, 1602)])
 def test_against_extended_precision(hip, form, m, n, k):
     got, ref = _run(hip, m, n, k, form)
     err = np.linalg.norm((got - ref).astype(np.float64)) / np.linalg.norm(ref.astype(np.float64))
