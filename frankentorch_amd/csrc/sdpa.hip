@@ -1001,7 +1001,8 @@ template <int D> int32_t launch_small_sdpa(SdpaArgs &a, hipStream_t st) {
 }
 
 // Blocks of 128 queries (4 wavefronts) are used whenever they still give every other CU a
-// workgroup; shorter problems fall back to blocks of 64 queries. Workgroups are issued heaviest
+// workgroup; shorter problems fall back to blocks of 64 queries, as do up to 64 queries of head size 64, of which the larger block would
+// leave half idle (us, 4 wavefronts / 2: 1024 heads x 64 x 64 29.8 / 20.8, causal 32.6 / 20.2, 260 x 20 x 20 13.4 / 8.6). Workgroups are issued heaviest
 // first, which balances causal problems. Unmasked problems of head size 64 and 128 run on the bf16 matrix units
 // (sdpa_split.hip) but for scales beyond its range and the short ones that are faster here.
 template <int D> int32_t launch_mfma(SdpaArgs &a, hipStream_t st) {
@@ -1011,7 +1012,7 @@ template <int D> int32_t launch_mfma(SdpaArgs &a, hipStream_t st) {
         const char *e = std::getenv("FT_HIP_SDPA_CFG");  // tuning knob: bit 0 = 4 wavefronts; -1 = auto
         return e ? std::atoi(e) : -1;
     }();
-    const bool wide = D >= 128 || (forced >= 0 ? (forced & 1) != 0 : 2 * wg128 >= (int64_t)cus);  // D = 128 staging does not fit 2-wavefront blocks
+    const bool wide = D >= 128 || (forced >= 0 ? (forced & 1) != 0 : 2 * wg128 >= (int64_t)cus && (D != 64 || a.mask || a.d.seq_q > 64));  // D = 128 staging does not fit 2-wavefront blocks
     if (a.mask) return wide ? launch_mfma_cfg<D, 4, true>(a, st) : launch_mfma_cfg<D, 2, true>(a, st);
     return wide ? launch_mfma_cfg<D, 4, false>(a, st) : launch_mfma_cfg<D, 2, false>(a, st);
 }

@@ -527,9 +527,15 @@ bool sdpa_split_pays(const fth_sdpa_desc &d, float scale) {
     // of 200 x 200 34.4 / 31.2, 64 heads of 100 x 2048 and above).
     const int64_t keys = d.causal && d.seq_q < d.seq_k ? d.seq_q : d.seq_k;
     if (d.d_k == 128 && (keys < 160 || (d.seq_q <= 128 && d.num_bh > 128))) return false;
+    // Head size 64: one stage of keys leaves nothing to hide a block's start and end behind, and the fp32 kernel is the faster one where blocks that
+    // are half empty at the least take a second round here (260 heads x 64 x 64 13.4 / 16.6, 512 x 48 x 64 14.3 / 17.2, 1024 x 64 x 64 causal
+    // 20.2 / 35.4, 260 x 100 x 64 14.9 / 18.1; in one, 192 x 48 x 48 9.9 / 9.2). Longer ones stay for their smaller error (1.2e-7, there 2.4e-7),
+    // on either side in time: 96 x 300 x 40 15.8 / 12.6, 128 x 600 x 64 24.9 / 28.7, 32 x 300 x 64 9.0 / 10.3. With more keys: 260 x 64 x 100 22.3 /
+    // 21.6, 768 x 127 x 127 causal 39.1 / 38.6.
+    const int64_t cus = compute_units() > 0 ? compute_units() : 256;
+    if (d.d_k == 64 && keys <= 64 && d.seq_q <= 128 && d.num_bh > cus) return false;
     // Head size 128, not causal: a second round of 256-query blocks where all blocks of the fp32 kernel, 128 queries and two on a
     // compute unit, run at once (96 heads x 640 tokens: 172 us, 165 there).
-    const int64_t cus = compute_units() > 0 ? compute_units() : 256;
     if (d.d_k == 128 && !d.causal && d.num_bh * ceil_div(d.seq_q, (int64_t)256) > cus && d.num_bh * ceil_div(d.seq_q, (int64_t)128) <= 2 * cus) return false;
     return true;
 }

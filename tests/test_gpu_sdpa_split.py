@@ -2,9 +2,14 @@
 
 Bound on the error: that of the fp32 matrix-unit kernels on the same operands, at most 2.0e-8 sqrt(keys) + 1.2e-7 (relative
 2-norm, normal operands, measured from 64 to 2048 keys; 1.6e-8 sqrt(keys) + 0.5e-7 here)."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
+from conftest import ROOT
 from frankentorch_amd.device import DeviceBuffer
 
 pytestmark = pytest.mark.gpu
@@ -44,7 +49,7 @@ def _rel(got, ref):
 # head size 128: 32-key stages, ragged ends, short last block, fewer keys than queries
 @pytest.mark.parametrize("heads,group,sq,sk,d,causal", [
     (300, 1, 256, 64, 64, False), (300, 4, 250, 65, 64, False), (300, 1, 255, 191, 64, False), (260, 1, 511, 129, 64, True), (96, 4, 300, 300, 64, True),
-    (40, 1, 250, 32, 64, False), (70, 1, 129, 33, 64, False), (70, 7, 131, 97, 64, True), (12, 1, 777, 777, 64, True), (16, 4, 700, 1500, 64, False), (9, 1, 1100, 1, 64, False),
+    (40, 1, 250, 32, 64, False), (70, 1, 129, 33, 64, False), (70, 7, 131, 97, 64, True), (12, 1, 777, 777, 64, True), (16, 4, 700, 1500, 64, False), (9, 1, 1100, 1, 64, False), (96, 1, 127, 127, 64, True),
     (3, 1, 257, 257, 128, True), (2, 2, 300, 2049, 128, False), (5, 1, 33, 161, 128, False), (40, 4, 520, 191, 128, True), (4, 1, 200, 320, 128, True)])
 def test_against_64_bit(hip, heads, group, sq, sk, d, causal):
     q, k, v = _inputs(heads, group, sq, sk, d)
@@ -112,3 +117,31 @@ def test_scales_beyond_the_range_stay_on_fp32_units(hip, d, heads):
     q *= np.float32(2.0 ** -60)
     out = _run(hip, q, k, v, True, scale=2.0 ** 57)
     assert _rel(out[0], _ref(q[0], k[0], v[0], True, 2.0 ** 57)) <= 1e-6
+
+
+CHILD = """
+import sys
+sys.path[:0] = [%(root)r, %(root)r + "/tests"]
+import numpy as np
+from frankentorch_amd import device as hip
+import test_gpu_sdpa_split as t
+np.savez(sys.argv[1], **{str(i): t._run(hip, *t._inputs(h, 1, sq, sk, 64), causal) for i, (h, sq, sk, causal, _) in enumerate(t.SHORT)})
+"""
+# heads, queries, keys, causal, on bf16 units
+SHORT = [(300, 64, 64, False, False), (260, 33, 33, True, False), (1024, 20, 128, True, False), (32, 300, 40, False, True), (260, 100, 64, True, False),
+         (70, 250, 32, False, True), (96, 300, 40, False, True), (128, 600, 64, False, True), (300, 64, 65, False, True), (96, 65, 65, False, True)]
+
+
+def test_few_keys_stay_on_fp32_units(hip, tmp_path):
+    """Up to 64 keys of head size 64 and up to 128 queries run on bf16 units where all blocks run at once; the others give the bits that they give
+    with that kernel switched off (a child process: the switch is read once). Error: theirs, at most
+    2.5e-8 sqrt(keys) + 1.4e-7 (3.05e-7 measured for 64 keys, 1.6e-7 for 16)."""
+    path = str(tmp_path / "fp32.npz")
+    subprocess.run([sys.executable, "-c", CHILD % {"root": ROOT}, path], check=True, timeout=110, env=dict(os.environ, FT_HIP_SDPA_SPLIT="0"))
+    fp32 = np.load(path)
+    for i, (heads, sq, sk, causal, split) in enumerate(SHORT):
+        q, k, v = _inputs(heads, 1, sq, sk, 64)
+        out = _run(hip, q, k, v, causal)
+        assert np.array_equal(out, fp32[str(i)]) != split, SHORT[i]
+        for h in (0, heads - 1):
+            assert _rel(out[h], _ref(q[h], k[h], v[h], causal)) <= 2.5e-8 * np.sqrt(sk) + 1.4e-7
