@@ -37,6 +37,31 @@ __device__ __forceinline__ float gelu_erf(float x) {
     return x < 0.0f ? h * e : h * (2.0f - e);
 }
 
+__device__ __forceinline__ double gelu_erf(double x) { return (0.5 * x) * (1.0 + erf(x * 0.70710678118654752440)); }
+
+// tanh-form GELU of the products' epilogues as x * sigmoid(2u), u = sqrt(2/pi) (x + 0.044715 x^3): 0.5 (1 + tanh u) = 1 / (1 + e^-2u).
+// One hardware exp2 and one division; e^-2u overflowing to inf gives x / inf = -0 where the tanh form gives -0 too.
+__device__ __forceinline__ float gelu_tanh(float x) {
+    const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
+    return x / (1.0f + __builtin_amdgcn_exp2f(u * -2.8853900817779268f));  // -2 log2(e)
+}
+__device__ __forceinline__ double gelu_tanh(double x) {
+    return 0.5 * x * (1.0 + tanh(0.79788456080286535588 * (x + 0.044715 * x * x * x)));
+}
+
+// x of lanes 0..31 and x of lanes 32..63, each broadcast to both halves (one v_permlane32_swap, no LDS round trip).
+__device__ __forceinline__ void both_halves(float x, float &lo, float &hi) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    lo = __uint_as_float(r[0]);
+    hi = __uint_as_float(r[1]);
+}
+
+// Rows of 64 bytes in LDS, chunk c (16 bytes) of row r in slot c ^ swz(r): the 128-bit reads of 16 rows at one chunk touch every bank once.
+__device__ __forceinline__ int swz(int row) {
+    const int t = row >> 2;
+    return (((t ^ (t >> 1)) & 1) << 1) | ((t >> 1) & 1);
+}
+
 // 2^t in double precision for the softmax weights of the fp64 attention kernel: t is a score minus a reference
 // maximum, so it is bounded above (a few units) and may be -inf. n = round(t), f = t - n in [-1/2, 1/2],
 // 2^f by its Taylor series to degree 12 (remainder 1.7e-16 at |f| = 1/2), scaled by 2^n with ldexp, which

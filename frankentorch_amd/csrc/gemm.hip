@@ -95,12 +95,7 @@ template <> struct Mfma<float> {
     __device__ __forceinline__ static V zero() { return make_float4(0.f, 0.f, 0.f, 0.f); }
     __device__ __forceinline__ static V make(const float *e) { return make_float4(e[0], e[1], e[2], e[3]); }
     __device__ __forceinline__ static float gelu(float x) { return fth::gelu_erf(x); }
-    // tanh-form GELU as x * sigmoid(2u), u = sqrt(2/pi) (x + 0.044715 x^3): 0.5 (1 + tanh u) = 1 / (1 + e^-2u). One
-    // hardware exp2 and one division; e^-2u overflowing to inf gives x / inf = -0 where the tanh form gives -0 too.
-    __device__ __forceinline__ static float gelu_tanh(float x) {
-        const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
-        return x / (1.0f + __builtin_amdgcn_exp2f(u * -2.8853900817779268f));  // -2 log2(e)
-    }
+    __device__ __forceinline__ static float gelu_tanh(float x) { return fth::gelu_tanh(x); }
 };
 template <> struct Mfma<double> {
     static constexpr int MT = 16;
@@ -117,10 +112,8 @@ template <> struct Mfma<double> {
     __device__ __forceinline__ static double elem(const V &v, int j) { return j == 0 ? v.x : v.y; }
     __device__ __forceinline__ static V zero() { return make_double2(0.0, 0.0); }
     __device__ __forceinline__ static V make(const double *e) { return make_double2(e[0], e[1]); }
-    __device__ __forceinline__ static double gelu(double x) { return (0.5 * x) * (1.0 + erf(x * 0.70710678118654752440)); }
-    __device__ __forceinline__ static double gelu_tanh(double x) {
-        return 0.5 * x * (1.0 + tanh(0.79788456080286535588 * (x + 0.044715 * x * x * x)));
-    }
+    __device__ __forceinline__ static double gelu(double x) { return fth::gelu_erf(x); }
+    __device__ __forceinline__ static double gelu_tanh(double x) { return fth::gelu_tanh(x); }
 };
 
 // fp32 on v_mfma_f32_16x16x4_f32: accumulator element r of `lane` is row 4 (lane / 16) + r, column lane % 16. The same

@@ -16,6 +16,7 @@
 // 2500 6.3e-16 / 8.2e-16 / 3.0e-16; us without and with it 17.7 / 17.7 (A stored [k, m] 18.4 / 19.4), 300 x 300 x 1500 21.0 / 22.4, 512^3 10.5 / 10.8.
 // Bound by the matrix units and the vector instructions that share their issue cycles: 1500^3 41 of the 78.6 TFLOP/s.
 
+#include "devmath.hpp"
 #include "gemm_f64.hpp"
 
 namespace {
@@ -25,15 +26,6 @@ typedef D2 D2_any __attribute__((aligned(8)));  // 128-bit access at any double
 using D4 = __attribute__((ext_vector_type(4))) double;
 
 constexpr int kXcds = 8;
-
-__device__ __forceinline__ double gelu_erf64(double x) { return (0.5 * x) * (1.0 + erf(x * 0.70710678118654752440)); }
-__device__ __forceinline__ double gelu_tanh64(double x) { return 0.5 * x * (1.0 + tanh(0.79788456080286535588 * (x + 0.044715 * x * x * x))); }
-
-// Slot of chunk c (16 bytes) of row r is c ^ swz(r): the 128-bit reads of 16 rows at one chunk touch every bank once.
-__device__ __forceinline__ int swz(int row) {
-    const int t = row >> 2;
-    return (((t ^ (t >> 1)) & 1) << 1) | ((t >> 1) & 1);
-}
 
 // KA, KB: K is the contiguous direction of A, of B.
 // Three wavefronts a SIMD are asked for where that keeps the accumulators out of the second half of the register file: without it 64
@@ -85,7 +77,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && !KB ? 3 : 1) void gemm_f64_kern
         for (int i = 0; i < T; ++i) v[i] = D2{k < p.k ? src[i][k * ks] : 0.0, k + 1 < p.k ? src[i][(k + 1) * ks] : 0.0};
     };
     unsigned char *area = smem[wave];
-    const int wr = qrow * 64 + ((qc ^ swz(qrow)) << 4), rd = l16 * 64 + ((g ^ swz(l16)) << 4);
+    const int wr = qrow * 64 + ((qc ^ fth::swz(qrow)) << 4), rd = l16 * 64 + ((g ^ fth::swz(l16)) << 4);
     auto stage = [&](int u) __attribute__((always_inline)) {
         unsigned char *s = area + (u & 1) * SLOT + wr;
 #pragma unroll
@@ -176,8 +168,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && !KB ? 3 : 1) void gemm_f64_kern
         for (int w = 1; w < NW; ++w) v += reinterpret_cast<const double *>(smem[w])[e * 64 + lane];
         if (p.alpha != 1.0) v = p.alpha * v;
         if (p.epilogue & FTH_EPI_BIAS) v = v + p.bias[col];
-        if (p.epilogue & FTH_EPI_GELU) v = gelu_erf64(v);
-        if (p.epilogue & FTH_EPI_GELU_TANH) v = gelu_tanh64(v);
+        if (p.epilogue & FTH_EPI_GELU) v = fth::gelu_erf(v);
+        if (p.epilogue & FTH_EPI_GELU_TANH) v = fth::gelu_tanh(v);
         if (p.epilogue & FTH_EPI_RESIDUAL) v = v + p.residual[batch * p.stride_c + row * p.ldc + col];
         C[row * p.ldc + col] = v;
     }

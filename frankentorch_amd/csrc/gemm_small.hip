@@ -30,17 +30,6 @@ constexpr int kXcds = 8;
 
 using Acc4 = __attribute__((ext_vector_type(4))) float;
 
-__device__ __forceinline__ float gelu_tanh(float x) {
-    const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
-    return x / (1.0f + __builtin_amdgcn_exp2f(u * -2.8853900817779268f));
-}
-
-// Slot of chunk c (16 bytes) of row r is c ^ swz(r): the 128-bit reads of 16 rows at one chunk touch every bank once.
-__device__ __forceinline__ int swz(int row) {
-    const int t = row >> 2;
-    return (((t ^ (t >> 1)) & 1) << 1) | ((t >> 1) & 1);
-}
-
 template <int NW, int MT, int NT, int U, int S, bool TRANS_B>
 __global__ __launch_bounds__(64 * NW) void gemm_quad_kernel(const fth::SmallGemm p, const int tiles_m, const int tiles_n) {
     constexpr int TILE = 1024, SLOT = (MT + (TRANS_B ? NT : 0)) * TILE;  // 16 rows x 64 bytes; what a group of 16 k takes
@@ -91,7 +80,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_quad_kernel(const fth::SmallGemm
         for (int i = 0; i < MT; ++i) av[u][i] = *reinterpret_cast<const Acc4 *>(ap[i] + 16 * t);
     };
     unsigned char *area = smem[wave];
-    const int wr = qrow * 64 + ((qc ^ swz(qrow)) << 4), rd = lrow * 64 + ((g ^ swz(lrow)) << 4);
+    const int wr = qrow * 64 + ((qc ^ fth::swz(qrow)) << 4), rd = lrow * 64 + ((g ^ fth::swz(lrow)) << 4);
     Acc4 sum[MT][NT], acc[S][MT][NT];
     auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -179,7 +168,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_quad_kernel(const fth::SmallGemm
             if (p.alpha != 1.f) v = p.alpha * v;
             if (p.epilogue & FTH_EPI_BIAS) v = v + p.bias[col];
             if (p.epilogue & FTH_EPI_GELU) v = fth::gelu_erf(v);
-            if (p.epilogue & FTH_EPI_GELU_TANH) v = gelu_tanh(v);
+            if (p.epilogue & FTH_EPI_GELU_TANH) v = fth::gelu_tanh(v);
             if (p.epilogue & FTH_EPI_RESIDUAL) v = v + p.residual[batch * p.stride_c + row * p.ldc + col];
             C[row * p.ldc + col] = v;
         }

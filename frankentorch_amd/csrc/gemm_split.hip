@@ -57,13 +57,9 @@ __device__ __forceinline__ float representable(float x) {
     return u >= kTooLarge || u - 1u < kTooSmall - 1u ? __builtin_nanf("") : x;  // (zero wraps round)
 }
 
-// Planes of an operand: [K-tile][plane][16-row block][16 rows][4 chunks of 8 k], a 16-byte chunk at slot chunk ^ swz(row) of
+// Planes of an operand: [K-tile][plane][16-row block][16 rows][4 chunks of 8 k], a 16-byte chunk at slot chunk ^ fth::swz(row) of
 // its row. The LDS holds the same image, and a wavefront's 128-bit operand read (16 rows at the same chunk, in the lane
 // groups the LDS serves together) touches every bank once: 0 conflict cycles by counter; chunk ^ (row / 4) has 2 a read.
-__device__ __forceinline__ int swz(int row) {
-    const int t = row >> 2;
-    return (((t ^ (t >> 1)) & 1) << 1) | ((t >> 1) & 1);
-}
 
 __device__ __forceinline__ void store_chunk(const float (&v)[8], unsigned char *planes, int64_t kt, int blocks, int64_t row, int chunk) {
     float r[8];
@@ -73,7 +69,7 @@ __device__ __forceinline__ void store_chunk(const float (&v)[8], unsigned char *
     fth::split8(r, w);
 #pragma unroll
     for (int s = 0; s < kPlanes; ++s)
-        *reinterpret_cast<u32x4 *>(planes + (kt * kPlanes + s) * blocks * kBlock + row * 64 + ((chunk ^ swz((int)(row & 15))) << 4)) = w[s];
+        *reinterpret_cast<u32x4 *>(planes + (kt * kPlanes + s) * blocks * kBlock + row * 64 + ((chunk ^ fth::swz((int)(row & 15))) << 4)) = w[s];
 }
 
 // One operand to split: [rows][k] (by_k) with row pitch ld, or [k][rows] with row pitch ld.
@@ -166,10 +162,6 @@ __device__ __forceinline__ void load_to_lds_16(const unsigned char *base, unsign
 }
 
 __device__ __forceinline__ float nan_max(float a, float b) { return __builtin_elementwise_maximum(a, b); }
-__device__ __forceinline__ float gelu_tanh(float x) {
-    const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
-    return x / (1.0f + __builtin_amdgcn_exp2f(u * -2.8853900817779268f));
-}
 
 // Four k of one operand row for the fp32 MFMAs: the first `left` of them from p on, ks apart, the others zero.
 __device__ __forceinline__ f32x4 four_k(const float *p, int64_t ks, int left) {
@@ -260,7 +252,7 @@ __global__ __launch_bounds__(WM *WN *kWave, 2) void plane_gemm_kernel(const Plan
     };
 
     struct Frag { bf16x8 a[TM], b[TN]; };
-    const int a_rd = (wm0 + l16) * 64 + ((lq ^ swz(l16)) << 4), b_rd = A_CH * kBlock + (wn0 + l16) * 64 + ((lq ^ swz(l16)) << 4);
+    const int a_rd = (wm0 + l16) * 64 + ((lq ^ fth::swz(l16)) << 4), b_rd = A_CH * kBlock + (wn0 + l16) * 64 + ((lq ^ fth::swz(l16)) << 4);
     auto fetch = [&](Frag &f, int buf, int s) __attribute__((always_inline)) {
         const unsigned char *s0 = smem + buf * BUF;
 #pragma unroll
@@ -398,7 +390,7 @@ __global__ __launch_bounds__(WM *WN *kWave, 2) void plane_gemm_kernel(const Plan
 #pragma unroll
                     for (int j = 0; j < TN; ++j)
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) acc[i][j][e] = gelu_tanh(acc[i][j][e]);
+                        for (int e = 0; e < 4; ++e) acc[i][j][e] = fth::gelu_tanh(acc[i][j][e]);
             }
         }
         const float *res = !parts && (p.g.epilogue & FTH_EPI_RESIDUAL) ? p.g.residual : nullptr;
@@ -494,7 +486,7 @@ __global__ __launch_bounds__(256) void plane_reduce_kernel(const PlaneArgs p) {
     if (p.g.alpha != 1.f) v *= p.g.alpha;
     if (p.g.epilogue & FTH_EPI_BIAS) v += p.g.bias[col];
     if (p.g.epilogue & FTH_EPI_GELU) v = fth::gelu_erf(v);
-    if (p.g.epilogue & FTH_EPI_GELU_TANH) v = gelu_tanh(v);
+    if (p.g.epilogue & FTH_EPI_GELU_TANH) v = fth::gelu_tanh(v);
     if (p.g.epilogue & FTH_EPI_RESIDUAL) v += p.g.residual[row * p.g.ldc + col];
     p.g.c[row * p.g.ldc + col] = v;
 }

@@ -24,6 +24,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "devmath.hpp"
 
 namespace {
 
@@ -542,9 +543,7 @@ __global__ __launch_bounds__(512) void i8_skinny_quad_kernel(const I8Args p) {
 #pragma unroll
         for (int t = 0; t < MT; ++t) xv[u][t] = *reinterpret_cast<const V4i *>(x[t] + at);
     };
-    // chunk c of row r in slot c ^ f(r): the 128-bit reads of 16 rows at one chunk touch every bank once
-    auto f = [](int r) { const int t = r >> 2; return (((t ^ (t >> 1)) & 1) << 1) | ((t >> 1) & 1); };
-    const int wr = qrow * 64 + ((qc ^ f(qrow)) << 4), rd = l16 * 64 + ((lq ^ f(l16)) << 4);
+    const int wr = qrow * 64 + ((qc ^ fth::swz(qrow)) << 4), rd = l16 * 64 + ((lq ^ fth::swz(l16)) << 4);
     unsigned char *area = smem[wave];
     auto stage = [&](int u) __attribute__((always_inline)) {
         unsigned char *s = area + (u & 1) * SLOT + wr;

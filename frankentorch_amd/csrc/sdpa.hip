@@ -83,13 +83,6 @@ __device__ __forceinline__ void load_to_lds_16(const float *base, unsigned lane_
                  : "memory", "m0");
 }
 
-// x of lanes 0..31 and x of lanes 32..63, each broadcast to both halves (one v_permlane32_swap, no LDS round trip).
-__device__ __forceinline__ void both_halves(float x, float &lo, float &hi) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    lo = __uint_as_float(r[0]);
-    hi = __uint_as_float(r[1]);
-}
-
 template <int N> struct VecN;
 template <> struct VecN<1> { using type = float; };
 template <> struct VecN<2> { using type = float2; };
@@ -387,7 +380,7 @@ __global__ __launch_bounds__(64 * NW, 2) void sdpa_mfma_kernel(const SdpaArgs p)
                     // a per-lane partial sum until the end.
                     if (__any(mt * c2 > m_run + kLazy)) {
                         float mlo, mhi;
-                        both_halves(mt, mlo, mhi);
+                        fth::both_halves(mt, mlo, mhi);
                         m_new = fmaxf(m_run, fmaxf(mlo, mhi) * c2);
                         alpha = __builtin_amdgcn_exp2f(m_run - m_new);
 #pragma unroll
@@ -445,7 +438,7 @@ __global__ __launch_bounds__(64 * NW, 2) void sdpa_mfma_kernel(const SdpaArgs p)
 #pragma unroll
                         for (int r = 0; r < 16; ++r) mt = fmaxf(mt, s[j][r]);
                     float mlo, mhi;
-                    both_halves(mt, mlo, mhi);
+                    fth::both_halves(mt, mlo, mhi);
                     mt = fmaxf(mlo, mhi);
                     m_new = fmaxf(m_run, mt);
                     // A mask can hide every key seen so far (m_new still -inf): the weights are then 0 and the state
@@ -485,7 +478,7 @@ __global__ __launch_bounds__(64 * NW, 2) void sdpa_mfma_kernel(const SdpaArgs p)
         }
         {  // the two halves of the wavefront hold partial row sums of the same queries
             float llo, lhi;
-            both_halves(l_run, llo, lhi);
+            fth::both_halves(l_run, llo, lhi);
             l_run = llo + lhi;
         }
 
@@ -925,7 +918,7 @@ __global__ __launch_bounds__(256) void sdpa_small_kernel(const SdpaArgs p) {
             mt = fmaxf(mt, s[r]);
         }
         float mlo, mhi;
-        both_halves(mt, mlo, mhi);
+        fth::both_halves(mt, mlo, mhi);
         mt = fmaxf(mlo, mhi);
         const float m_new = fmaxf(m_run, mt * c2);
         // a wavefront's tiles can all lie past a query's causal limit (m_new still -inf): keep its state empty
@@ -952,7 +945,7 @@ __global__ __launch_bounds__(256) void sdpa_small_kernel(const SdpaArgs p) {
             for (int ee = 0; ee < NDT; ++ee) o[ee] = __builtin_amdgcn_mfma_f32_32x32x2f32(vecn_get(vv[r], ee), e, o[ee], 0, 0, 0);
         }
         float plo, phi;
-        both_halves(psum, plo, phi);
+        fth::both_halves(psum, plo, phi);
         l_run = l_run * alpha + (plo + phi);
         m_run = m_new;
     }

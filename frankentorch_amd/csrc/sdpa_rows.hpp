@@ -4,17 +4,11 @@
 
 #include <hip/hip_runtime.h>
 
+#include "devmath.hpp"
 #include "ft_kernel_hip.h"
 #include "split_bf16.hpp"
 
 namespace fth {
-
-// x of lanes 0..31 and x of lanes 32..63, each broadcast to both halves (one v_permlane32_swap, no LDS round trip).
-__device__ __forceinline__ void both_halves(float x, float &lo, float &hi) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    lo = __uint_as_float(r[0]);
-    hi = __uint_as_float(r[1]);
-}
 
 // Online softmax of queries q0 .. q0 + 31 over keys 0 .. 32 num_kt - 1, with the scheme of sdpa_small_kernel (sdpa.hip). Lane l holds query q0 + l % 32; o[e][r] is its output element e + D / 32 (8 (r / 4) + 4 (l / 32) + r % 4), not yet
 // divided by l_run. Few registers instead of requests ahead of their use: the caller holds many, and this is rare.
