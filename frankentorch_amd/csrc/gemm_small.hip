@@ -186,7 +186,8 @@ template <int NW, int MT, int NT, int U, int S, bool TRANS_B> int32_t launch(con
 // a workgroup, then two column tiles as well, once there are workgroups enough: rows of A come from L2 less often. Six slots where they come out even (K 768 and 3072 over eight wavefronts).
 // us, eight wavefronts / four / four with two row tiles: 37 x 768 x 3072 9.2 / 13.6 / -, 37 x 2304 x 768 6.4 / 6.3 / 8.1, 200 x 1536 x 512
 // 8.2 / 7.0 / 7.8, 9 x 3072 x 768 5.1 / 5.7 / -, 64 x 50257 x 768 - / 87 / 79; with 2 x 2 tiles 65, 37 x 50257 x 768 58.6, with 3 x 2 55.6
-// (2 x 1: 62.3), 400 x 2304 x 768 20.2 (21.8); 64 x 10000 x 768 16.4 (16.1). 64 x 32000 x 1024
+// (2 x 1: 62.3; 33 to 48 rows with 2 x 2 / 3 x 2, weights mostly from HBM: 33 x 33009 x 272 20.7 / 18.4, 41 x 32000 x 1024 54 / 46, 36 x 100000 x 256
+// 49 / 38, 33 x 32768 x 2048 99 / 82, 48 x 128256 x 1024 206 / 185, 41 x 25000 x 4096 180 / 175), 400 x 2304 x 768 20.2 (21.8); 64 x 10000 x 768 16.4 (16.1). 64 x 32000 x 1024
 // eight wavefronts 75, four with 2 x 2 tiles 52.
 template <bool TRANS_B> int32_t choose(const fth::SmallGemm &g, hipStream_t st) {
     const int64_t tiles = fth::ceil_div(g.m, 16) * fth::ceil_div(g.n, 16) * g.batch, per = fth::ceil_div(g.k / 16, 8);

@@ -495,8 +495,9 @@ __global__ __launch_bounds__(256) void plane_reduce_kernel(const PlaneArgs p) {
 
 // One workgroup of 128 x 256, 128 x 192 or 128 x 128 a compute unit, or two of 64 x 128. Rates are TFLOP/s of fp32 products with every
 // compute unit busy, measured on 4096^3, 8192 x 768 x 3072, 4662 x 768 x 768 and 2331 x 768 x 768; the small tile's with one and with
-// two workgroups on a compute unit, the others' in one round and in more. The square tile is for products of which it makes one
-// round and the small one two (in full rounds it is behind the wide one: 4096^3 614 us, 581): 1031 x 3072
+// two workgroups on a compute unit, the others' in one round and in more. The square tile gains most where it makes one round and the
+// small one two; in full rounds it is behind the wide one (4096^3 614 us, 581), and of several rounds it is taken where its last one
+// comes out fuller (us without / with it: 20011 x 1000 x 520 151 / 148, 1224 x 15221 x 1768 391 / 381, 8239 x 2886 x 600 180 / 173): 1031 x 3072
 // x 768 42.9 -> 39.2 us, planes included, 3000 x 1024 x 1024 52.0 -> 47.4, 4662 x 768 x 768 44.5 -> 42.3, 6000 x 512 x 512 35.3 -> 33.7.
 struct Tile { int bm, bn; double rate[2]; };
 constexpr Tile kTiles[] = {{128, 256, {250., 250.}}, {128, 192, {238., 238.}}, {64, 128, {145., 200.}}, {128, 128, {255., 225.}}};

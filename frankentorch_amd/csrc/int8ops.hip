@@ -507,9 +507,11 @@ __global__ __launch_bounds__(512) void i8_skinny_kernel(const I8Args p) {
 // through the wavefront's own LDS (no barrier: its LDS instructions execute in order). In the MFMA layout itself neighbouring
 // lanes read different rows, and a compute unit then takes in 16 bytes a cycle instead of 64, which is what binds once the
 // activations that each workgroup reads again are as much as its weights. U steps are in flight.
-// Whole call with the quantiser, weights rotating through 300 MB, i8_skinny_kernel -> here: 13 x 4096 x 11008 16.9 -> 15.9 us, 32 x
-// 4096 x 11008 23.3 -> 19.5, 64 x 4096 x 4096 17.3 -> 15.3; on the other side 13 x 4096 x 4096 10.15 / 10.5, 1 x 4096 x 11008 13.4 / 13.9, and
-// short K, where the staging is not covered: 64 x 768 x 11008 11.2 / 14.0.
+// Whole call with the quantiser, i8_skinny_kernel -> here, us with weights that the last-level cache holds, then with weights from HBM (2.5 GB of
+// them in turn): 32 x 4096 x 11008 20.7 -> 17.1, 25.2 -> 22.0; 64 x 4096 x 11008 28.8 -> 25.5, 33.4 -> 29.3; 64 x 4096 x 4096 15.2 -> 12.4, 17.0 ->
+// 15.6; 20 x 4096 x 4096 10.2 -> 8.3, 11.1 -> 10.7; 40 x 8192 x 1024 21.0 -> 14.1, 23.3 -> 18.6. Of 9 to 16 rows only held weights gain: 13 x
+// 4096 x 11008 15.7 -> 13.7, 17.5 -> 17.8; 9 rows 14.7 -> 12.9, 16.3 -> 16.7; 16 x 2048 x 8192 8.2 -> 7.1 to 8.0, 10.0 -> 9.7. On the other side:
+// 13 x 4096 x 4096 10.15 / 10.5, 1 x 4096 x 11008 13.4 / 13.9, and short K, where the staging is not covered: 64 x 768 x 11008 11.2 / 14.0.
 template <int MT, int NT>
 __global__ __launch_bounds__(512) void i8_skinny_quad_kernel(const I8Args p) {
     constexpr int NW = 8, U = 4, TILE = 1024, SLOT = (MT + NT) * TILE;  // a tile: 16 rows x 64 bytes
