@@ -11,13 +11,11 @@
 // row and turns the kilobyte into the operand layout through LDS of its own: a write, a read, no barrier (a wavefront's LDS
 // instructions execute in order). U such loads of each operand are in flight, and a slot is requested again as soon as it is
 // used, so weights that come from HBM pay its latency once.
-// The MFMAs of one pass over the U loads (chains of 16 or 24; of 8 with two slots, or with S = 2 sets of accumulators, which four
-// wavefronts of one tile take) are added to a sum with ordinary additions before the next pass, so that a long K does not grow the
-// error with its root: a chain of L MFMAs loses 5e-8 sqrt(L / 2). Relative 2-norm error against 64 bits, one chain a wavefront -> here, at
-// the same times within 2%: 37 x 2304 x 768 2.5e-7 -> 1.2e-7, 200 x 3072 x 768 2.5e-7 -> 1.5e-7, 64 x 512 x 16384 8.1e-7 -> 1.9e-7, 64 x 5000
-// x 992 2.9e-7 -> 1.2e-7 (the large-tile kernels with K split over workgroups: 1.9e-7, 2.2e-7, 2.9e-7, 2.1e-7).
-// us, operands straight into the MFMA layout -> here (weights from HBM): 37 x 2304 x 768 8.0 -> 6.9, 37 x 3072 x 768 9.9 -> 7.5,
-// 37 x 768 x 3072 14.8 -> 9.2, 128 x 768 x 768 7.5 -> 5.6, 37 x 50257 x 768 98 -> 56 (large-tile kernel before).
+// The MFMAs of one pass over the U loads (chains of 16 or 24; of 8 with two slots) are added to a sum with ordinary additions before the
+// next pass, so that a long K does not grow the error with its root: a chain of L MFMAs loses 5e-8 sqrt(L / 2). Relative 2-norm
+// error against 64 bits, kernels before (K cut over more wavefronts or workgroups) / one chain a wavefront / here: 37 x 2304 x 768 1.9e-7 / 2.5e-7 /
+// 1.5e-7, 200 x 1536 x 512 1.55e-7 / 2.1e-7 / 1.5e-7, 64 x 5000 x 992 2.1e-7 / 2.9e-7 / 1.6e-7, 64 x 512 x 16384 2.9e-7 / 8.1e-7 / 1.9e-7; us without and
+// with the sums 5.27 / 5.42, 7.34 / 7.30, 11.6 / 11.6, 30.2 / 30.5, 400 x 2304 x 768 21.4 / 22.1.
 
 #include <cstdlib>
 
@@ -30,7 +28,7 @@ constexpr int kXcds = 8;
 
 using Acc4 = __attribute__((ext_vector_type(4))) float;
 
-template <int NW, int MT, int NT, int U, int S, bool TRANS_B>
+template <int NW, int MT, int NT, int U, bool TRANS_B>
 __global__ __launch_bounds__(64 * NW) void gemm_quad_kernel(const fth::SmallGemm p, const int tiles_m, const int tiles_n) {
     constexpr int TILE = 1024, SLOT = (MT + (TRANS_B ? NT : 0)) * TILE;  // 16 rows x 64 bytes; what a group of 16 k takes
     constexpr int PITCH = 17;
@@ -81,25 +79,20 @@ __global__ __launch_bounds__(64 * NW) void gemm_quad_kernel(const fth::SmallGemm
     };
     unsigned char *area = smem[wave];
     const int wr = qrow * 64 + ((qc ^ fth::swz(qrow)) << 4), rd = lrow * 64 + ((g ^ fth::swz(lrow)) << 4);
-    Acc4 sum[MT][NT], acc[S][MT][NT];
-    auto clear = [&]() __attribute__((always_inline)) {
+    Acc4 sum[MT][NT], acc[MT][NT];
+    auto clear = [](Acc4 (&x)[MT][NT]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int x = 0; x < S; ++x)
+        for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int j = 0; j < NT; ++j) acc[x][i][j] = Acc4{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < NT; ++j) x[i][j] = Acc4{0.f, 0.f, 0.f, 0.f};
     };
     auto collect = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int j = 0; j < NT; ++j) sum[i][j] += S == 2 ? acc[0][i][j] + acc[S - 1][i][j] : acc[0][i][j];
+            for (int j = 0; j < NT; ++j) sum[i][j] += acc[i][j];
     };
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j) sum[i][j] = Acc4{0.f, 0.f, 0.f, 0.f};
+    clear(sum);
     auto stage = [&](int u) __attribute__((always_inline)) {
         unsigned char *s = area + (u & 1) * SLOT + wr;
 #pragma unroll
@@ -120,14 +113,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_quad_kernel(const fth::SmallGemm
 #pragma unroll
             for (int e = 0; e < 4; ++e)
 #pragma unroll
-                for (int j = 0; j < NT; ++j) acc[e % S][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[j][e], acc[e % S][i][j], 0, 0, 0);
+                for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[j][e], acc[i][j], 0, 0, 0);
         }
     };
 #pragma unroll
     for (int u = 0; u < U; ++u) load(u, g0 + u);
     int t0 = g0;
     for (; t0 + U < g1; t0 += U) {
-        clear();
+        clear(acc);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             stage(u);
@@ -139,7 +132,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_quad_kernel(const fth::SmallGemm
         }
         collect();
     }
-    clear();
+    clear(acc);
 #pragma unroll
     for (int u = 0; u < U; ++u)
         if (t0 + u < g1) {
@@ -175,9 +168,9 @@ __global__ __launch_bounds__(64 * NW) void gemm_quad_kernel(const fth::SmallGemm
     }
 }
 
-template <int NW, int MT, int NT, int U, int S, bool TRANS_B> int32_t launch(const fth::SmallGemm &g, hipStream_t st) {
+template <int NW, int MT, int NT, int U, bool TRANS_B> int32_t launch(const fth::SmallGemm &g, hipStream_t st) {
     const int tiles_m = (int)fth::ceil_div(g.m, 16 * MT), tiles_n = (int)fth::ceil_div(g.n, 16 * NT);
-    gemm_quad_kernel<NW, MT, NT, U, S, TRANS_B><<<dim3((unsigned)(tiles_m * tiles_n), (unsigned)g.batch), dim3(64 * NW), 0, st>>>(g, tiles_m, tiles_n);
+    gemm_quad_kernel<NW, MT, NT, U, TRANS_B><<<dim3((unsigned)(tiles_m * tiles_n), (unsigned)g.batch), dim3(64 * NW), 0, st>>>(g, tiles_m, tiles_n);
     FTH_CHECK_LAUNCH("gemm_small");
     return FTH_OK;
 }
@@ -191,13 +184,13 @@ template <int NW, int MT, int NT, int U, int S, bool TRANS_B> int32_t launch(con
 // eight wavefronts 75, four with 2 x 2 tiles 52.
 template <bool TRANS_B> int32_t choose(const fth::SmallGemm &g, hipStream_t st) {
     const int64_t tiles = fth::ceil_div(g.m, 16) * fth::ceil_div(g.n, 16) * g.batch, per = fth::ceil_div(g.k / 16, 8);
-    if (tiles <= 288 || (g.k >= 1024 && tiles < 1536)) return per % 6 == 0 ? launch<8, 1, 1, 6, 1, TRANS_B>(g, st) : launch<8, 1, 1, 4, 1, TRANS_B>(g, st);
-    if (tiles < 1536 || g.m <= 16) return launch<4, 1, 1, 4, 2, TRANS_B>(g, st);
+    if (tiles <= 288 || (g.k >= 1024 && tiles < 1536)) return per % 6 == 0 ? launch<8, 1, 1, 6, TRANS_B>(g, st) : launch<8, 1, 1, 4, TRANS_B>(g, st);
+    if (tiles < 1536 || g.m <= 16) return launch<4, 1, 1, 4, TRANS_B>(g, st);
     if constexpr (TRANS_B) {
-        if (tiles >= 6000 && g.m > 32 && g.m <= 48) return launch<4, 3, 2, 2, 1, true>(g, st);
-        if (tiles >= 3072) return launch<4, 2, 2, 2, 1, true>(g, st);
+        if (tiles >= 6000 && g.m > 32 && g.m <= 48) return launch<4, 3, 2, 2, true>(g, st);
+        if (tiles >= 3072) return launch<4, 2, 2, 2, true>(g, st);
     }
-    return launch<4, 2, 1, 4, 1, TRANS_B>(g, st);
+    return launch<4, 2, 1, 4, TRANS_B>(g, st);
 }
 
 }  // namespace
