@@ -10,7 +10,7 @@
 // for a pass of its own, and it needs no scratch memory. Unlike fp32 MFMAs, bf16 ones leave the vector unit its issue cycles: up to
 // seven vector instructions of any kind used here hide behind one MFMA of 32 cycles (the dot-product instructions do not).
 //
-// Bound by the matrix units and the power they draw: causal, 4 x 32 heads of 2048 tokens, head size 128, 1050 -> 675 us; not causal
+// Bound by the matrix units and the power they draw: causal, 4 x 32 heads of 2048 tokens, head size 128, 1050 -> 680 us; not causal
 // 1936 -> 1235 us, 223 TFLOP/s of attention, 1.34 PFLOP/s of bf16 products. 96 heads of 1024 tokens, head size 64, 119 -> 82 us.
 // Relative 2-norm error against 64 bits, fp32 MFMA kernel / here: causal 4.5e-7 / 3.0e-7, not causal 8.9e-7 / 7.1e-7 (2048 tokens);
 // values of one sign 6.7e-7 / 4.4e-7, half of them zero 4.8e-7 / 4.5e-7, scores of standard deviation 8 1.8e-6 / 6.8e-7.
