@@ -20,7 +20,7 @@
 // weights under 2^-110 where nothing else makes up the output. What a weight loses is below 2^-134 (it is 2^-126 or zero at the
 // least, and the largest of a row at least one), so an output is off by at most seq_k 2^-134 max |V|: nothing that counts where it is
 // 2^-96 max |V| or more. A smaller one that is not zero needs keys of large weight whose values are zero or next to it. (The largest
-// |V| is kept beside the smallest for this: 0.3 us a block, 14.0 -> 14.3 us for 64 heads of 130 tokens, 694 -> 696 for the causal problem above.)
+// |V| is kept beside the smallest for this: 0.3 us a block, 14.0 -> 14.3 us for 64 heads of 130 tokens, 681 -> 685 for the causal problem above, timed in turn.)
 // A wavefront that finds a NaN, an infinity or such an output in its results, or is told of such operands, computes its 32 queries
 // again with fp32 MFMAs (sdpa_rows.hpp). Tiny values in Q and K need nothing: with the partners below 2^53 and a scale of at most
 // 2^20 what is lost of a score is below 2^-50.
